@@ -435,3 +435,32 @@ def test_argmax_matvec(P, qa, gpu):
     dW2 = dev(gpu, W2.view(np.int16))
     got2 = qa.lib().qwen_hip_argmax_matvec_bf16(ptr(dx), ptr(dW2), K, N, None)
     assert got2 == 3
+
+
+# the 8-wave blocks of 128 queries (unsplit, 256 blocks or more), over one to
+# several 32-key tiles: 256 kv heads make the grid, so the sizes can be those
+# of the walk's edges (one, two and three tiles; a last tile of one key; a
+# last query tile of one row; keys capped before the diagonal; an offset)
+@pytest.mark.parametrize("sq,sk,q_off", [(65, 20, 0), (65, 32, 0), (66, 33, 0), (100, 70, 0), (129, 129, 0),
+                                         (128, 300, 172), (129, 97, 40)])
+def test_causal_attention_wide_blocks(P, qa, gpu, sq, sk, q_off):
+    nh, nkv, hd = 512, 256, 128
+    chunk, nsplit = C.c_int(), C.c_int()
+    qa.lib().qk_attn_prefill_plan(sq, sk, q_off, nh, nkv, C.byref(chunk), C.byref(nsplit))
+    assert nsplit.value == 1
+    g = gpu.Generator(device="cuda").manual_seed(12)
+    Q = gpu.randn((sq, nh * hd), generator=g, device="cuda", dtype=gpu.float32)
+    K = gpu.randn((sk, nkv * hd), generator=g, device="cuda", dtype=gpu.float32)
+    V = gpu.randn((sk, nkv * hd), generator=g, device="cuda", dtype=gpu.float32)
+    out = gpu.full((sq, nh * hd), float("nan"), device="cuda", dtype=gpu.float32)
+    qa.check(qa.lib().qwen_hip_causal_attention(ptr(out), ptr(Q), ptr(K), ptr(V), sq, sk, nh, nkv, hd,
+                                                1.0 / np.sqrt(128.0), q_off, None), "attention")
+    gpu.cuda.synchronize()
+    q = Q.double().view(sq, nh, hd).transpose(0, 1).contiguous()
+    k = K.double().view(sk, nkv, hd).repeat_interleave(2, 1).permute(1, 2, 0).contiguous()
+    v = V.double().view(sk, nkv, hd).repeat_interleave(2, 1).transpose(0, 1).contiguous()
+    sc = gpu.bmm(q, k) / np.sqrt(128.0)
+    mask = gpu.arange(sk, device="cuda")[None, :] > q_off + gpu.arange(sq, device="cuda")[:, None]
+    ref = gpu.bmm(gpu.softmax(sc.masked_fill(mask, float("-inf")), -1), v).transpose(0, 1).reshape(sq, nh * hd)
+    # the bar of the other attention tests: the bf16 pairs leave 2^-16 per product
+    assert bool(((out.double() - ref).abs() <= 3e-5 + 1e-4 * ref.abs()).all())
