@@ -47,12 +47,15 @@ struct qwen_hip_encoder {
     hipStream_t stream;
     float *c1w, *c1b, *c2b, *c3b, *lnpw, *lnpb, *p1b, *p2b, *pe;
     enc_mat c2w, c3w, cow, p1w, p2w;
+    uint16_t *cowr;   /* cow.b16 with its columns in (row, channel) order */
+    uint16_t *zero;   /* 2 * ENC_CH zeros: the pixels outside an image */
     int stem_loaded;
     enc_layer L[QWEN_HIP_ENC_MAX_LAYERS];
     /* activations, sized for cap_chunks chunks */
-    int cap_chunks;
+    int cap_chunks, cap_cols;
     float *mel, *cols, *c1, *c2, *c3, *rows, *x, *xn, *qkv, *att, *mid, *out;
-    float *gws;   /* split-K partials of the GEMMs (QK_ENC_GEMM_WS_ELEMS floats) */
+    float *gws;   /* split-K partials of the GEMMs (gws_elems floats) */
+    long gws_elems;
 };
 
 static int dmalloc(void **p, size_t n) {
@@ -99,7 +102,7 @@ static void act_free(qwen_hip_encoder *e) {
                   (void **)&e->rows, (void **)&e->x, (void **)&e->xn, (void **)&e->qkv, (void **)&e->att,
                   (void **)&e->mid, (void **)&e->out, (void **)&e->gws};
     for (size_t i = 0; i < sizeof(b) / sizeof(b[0]); i++) dfree(b[i]);
-    e->cap_chunks = 0;
+    e->cap_chunks = e->cap_cols = 0;
 }
 
 void qwen_hip_encoder_destroy(qwen_hip_encoder *e) {
@@ -111,7 +114,8 @@ void qwen_hip_encoder_destroy(qwen_hip_encoder *e) {
                   (void **)&e->c2b,     (void **)&e->c3w.f32, (void **)&e->c3w.b16, (void **)&e->c3b,
                   (void **)&e->cow.f32, (void **)&e->cow.b16, (void **)&e->lnpw,    (void **)&e->lnpb,
                   (void **)&e->p1w.f32, (void **)&e->p1w.b16, (void **)&e->p1b,     (void **)&e->p2w.f32,
-                  (void **)&e->p2w.b16, (void **)&e->p2b,     (void **)&e->pe};
+                  (void **)&e->p2w.b16, (void **)&e->p2b,     (void **)&e->pe,
+                  (void **)&e->cowr,    (void **)&e->zero};
     for (size_t i = 0; i < sizeof(w) / sizeof(w[0]); i++) dfree(w[i]);
     for (int l = 0; l < QWEN_HIP_ENC_MAX_LAYERS; l++) {
         enc_layer *y = &e->L[l];
@@ -169,6 +173,10 @@ qwen_hip_encoder *qwen_hip_encoder_create(const qwen_hip_enc_config *cfg, int de
         return NULL;
     }
     free(pe);
+    if (dmalloc((void **)&e->zero, 2 * ENC_CH * 2) || hipMemset(e->zero, 0, 2 * ENC_CH * 2) != hipSuccess) {
+        qwen_hip_encoder_destroy(e);
+        return NULL;
+    }
     return e;
 }
 
@@ -277,6 +285,11 @@ int qwen_hip_encoder_load_stem(qwen_hip_encoder *e, const qwen_hip_enc_stem_weig
     QK_TRY(up(&e->c2b, w->conv2_b, ENC_CH));
     QK_TRY(up(&e->c3b, w->conv3_b, ENC_CH));
     QK_TRY(up_mat(&e->cow, ko, 0, w->conv_out_w, ko, w->conv_out_w && bf16_exact(w->conv_out_w, ko)));
+    if (e->cow.b16) {
+        if (!e->cowr) QK_TRY(dmalloc((void **)&e->cowr, ko * 2));
+        QK_TRY(qk_enc_reorder_launch(e->cow.b16, e->cowr, (int)d, ENC_CH, 16, e->stream));
+        QK_HIP(hipStreamSynchronize(e->stream));
+    }
     QK_TRY(up(&e->lnpw, w->ln_post_w, d));
     QK_TRY(up(&e->lnpb, w->ln_post_b, d));
     QK_TRY(up_mat(&e->p1w, d * d, 0, w->proj1_w, d * d, w->proj1_w && bf16_exact(w->proj1_w, d * d)));
@@ -369,14 +382,10 @@ static int reserve(qwen_hip_encoder *e, int chunks, int tokens) {
     const size_t cw = c->chunk_size;
     const size_t w1 = conv_out(cw), w2 = conv_out(w1), w3 = conv_out(w2);
     const size_t n1 = (size_t)chunks * 64 * w1, n2 = (size_t)chunks * 32 * w2, n3 = (size_t)chunks * 16 * w3;
-    size_t cols = n1 * ENC_K1;
-    if (n2 * ENC_K2 > cols) cols = n2 * ENC_K2;
-    if (n3 * ENC_K2 > cols) cols = n3 * ENC_K2;
     const size_t T = (size_t)chunks * w3;   /* >= tokens */
     (void)tokens;
     const size_t d = c->d_model;
     int rc = dmalloc((void **)&e->mel, (size_t)ENC_MEL * chunks * cw * 4);
-    if (!rc) rc = dmalloc((void **)&e->cols, cols * 4);
     if (!rc) rc = dmalloc((void **)&e->c1, (size_t)ENC_CH * n1 * 4);
     if (!rc) rc = dmalloc((void **)&e->c2, (size_t)ENC_CH * n2 * 4);
     if (!rc) rc = dmalloc((void **)&e->c3, (size_t)ENC_CH * n3 * 4);
@@ -387,10 +396,38 @@ static int reserve(qwen_hip_encoder *e, int chunks, int tokens) {
     if (!rc) rc = dmalloc((void **)&e->att, T * d * 4);
     if (!rc) rc = dmalloc((void **)&e->mid, T * (size_t)(c->ffn_dim > (int)d ? c->ffn_dim : (int)d) * 4);
     if (!rc) rc = dmalloc((void **)&e->out, T * (size_t)c->output_dim * 4);
-    if (!rc) rc = dmalloc((void **)&e->gws, (size_t)QK_ENC_GEMM_WS_ELEMS * 4);
+    e->gws_elems = (long)(T * d) > QK_ENC_GEMM_WS_ELEMS ? (long)(T * d) : QK_ENC_GEMM_WS_ELEMS;
+    if (!rc) rc = dmalloc((void **)&e->gws, (size_t)e->gws_elems * 4);
     if (rc) { act_free(e); return rc; }
     e->cap_chunks = chunks;
     return 0;
+}
+
+/* the im2col patches of the general path */
+static int reserve_cols(qwen_hip_encoder *e, int chunks) {
+    if (chunks <= e->cap_cols) return 0;
+    QK_HIP(hipStreamSynchronize(e->stream));
+    dfree((void **)&e->cols);
+    e->cap_cols = 0;
+    const size_t w1 = conv_out(e->cfg.chunk_size), w2 = conv_out(w1), w3 = conv_out(w2);
+    const size_t n[3] = {chunks * 64 * w1 * ENC_K1, chunks * 32 * w2 * ENC_K2, chunks * 16 * w3 * ENC_K2};
+    size_t cols = n[0];
+    for (int i = 1; i < 3; i++) cols = n[i] > cols ? n[i] : cols;
+    QK_TRY(dmalloc((void **)&e->cols, cols * 4));
+    e->cap_cols = chunks;
+    return 0;
+}
+
+/* Every matrix bf16-valued and of widths the ring products take (d <= 1024,
+ * k walks of whole 32-deep tiles, rows of whole float4s): the path of
+ * run_ring; otherwise the general one. */
+static int ring_ok(const qwen_hip_encoder *e) {
+    const qwen_hip_enc_config *c = &e->cfg;
+    if (c->d_model > 1024 || c->ffn_dim % 32 || c->output_dim % 4) return 0;
+    int ok = e->c2w.b16 && e->c3w.b16 && e->cow.b16 && e->cowr && e->p1w.b16 && e->p2w.b16;
+    for (int l = 0; l < c->layers; l++)
+        ok = ok && e->L[l].wqkv.b16 && e->L[l].wo.b16 && e->L[l].fc1w.b16 && e->L[l].fc2w.b16;
+    return ok;
 }
 
 /* C = A . W^T with the activations A [M][K] and a weight matrix W [N][K] */
@@ -398,7 +435,7 @@ static int gemm(qwen_hip_encoder *e, const float *A, int lda, const enc_mat *W, 
                 int N, int K, const float *bias_m, const float *bias_n, int gelu, int add) {
     qk_enc_gemm_args g = {.A = A, .B = W->f32, .C = C, .M = M, .N = N, .K = K, .lda = lda, .ldb = ldb, .ldc = ldc,
                           .bias_m = bias_m, .bias_n = bias_n, .gelu = gelu, .add = add,
-                          .ws = e->gws, .ws_elems = QK_ENC_GEMM_WS_ELEMS, .B16 = W->b16};
+                          .ws = e->gws, .ws_elems = e->gws_elems, .B16 = W->b16};
     return qk_enc_gemm_launch(&g, e->stream);
 }
 
@@ -407,7 +444,7 @@ static int gemm_add_ln(qwen_hip_encoder *e, const float *A, int lda, const enc_m
                        int T, const float *lnw, const float *lnb) {
     const int d = e->cfg.d_model;
     qk_enc_gemm_args g = {.A = A, .B = W->f32, .C = e->x, .M = T, .N = d, .K = K, .lda = lda, .ldb = K, .ldc = d,
-                          .bias_n = bias, .add = 1, .ws = e->gws, .ws_elems = QK_ENC_GEMM_WS_ELEMS, .B16 = W->b16,
+                          .bias_n = bias, .add = 1, .ws = e->gws, .ws_elems = e->gws_elems, .B16 = W->b16,
                           .ln_w = lnw, .ln_b = lnb, .ln_out = e->xn, .ln_eps = 1e-5f};
     return qk_enc_gemm_launch(&g, e->stream);
 }
@@ -435,13 +472,14 @@ static int stem_layer(qwen_hip_encoder *e, const float *in, int c_in, int chunks
     return qk_enc_gemm_launch(&g, e->stream);
 }
 
-static int run(qwen_hip_encoder *e, int mel_frames, int *tokens_out) {
+static int run_general(qwen_hip_encoder *e, int mel_frames, int *tokens_out) {
     const qwen_hip_enc_config *c = &e->cfg;
     const int cw = c->chunk_size, d = c->d_model, H = c->heads;
     const int chunks = (mel_frames + cw - 1) / cw;
     const int last = mel_frames - (chunks - 1) * cw;
     const int w1 = conv_out(cw), w2 = conv_out(w1), w3 = conv_out(w2);
     const int T = qwen_hip_encoder_tokens(c, mel_frames);
+    QK_TRY(reserve_cols(e, chunks));
     /* conv stem (qwen_asr_encoder.c:237-279); the mel is [128][mel_frames] */
     QK_TRY(stem_layer(e, e->mel, 1, chunks, ENC_MEL, cw, ENC_K1, mel_frames, e->c1w, NULL, e->c1b, e->c1,
                       conv_out(last)));
@@ -454,7 +492,7 @@ static int run(qwen_hip_encoder *e, int mel_frames, int *tokens_out) {
     {
         qk_enc_gemm_args g = {.A = e->rows, .B = e->cow.f32, .C = e->x, .M = T, .N = d, .K = ENC_CH * 16,
                               .lda = ENC_CH * 16, .ldb = ENC_CH * 16, .ldc = d, .pe = e->pe, .pe_rows = w3,
-                              .ws = e->gws, .ws_elems = QK_ENC_GEMM_WS_ELEMS, .B16 = e->cow.b16};
+                              .ws = e->gws, .ws_elems = e->gws_elems, .B16 = e->cow.b16};
         QK_TRY(qk_enc_gemm_launch(&g, e->stream));
     }
     const int win = w3 * (c->n_window_infer / cw);
@@ -465,7 +503,7 @@ static int run(qwen_hip_encoder *e, int mel_frames, int *tokens_out) {
     for (int l = 0; l < c->layers; l++) {
         const enc_layer *y = &e->L[l];
         QK_TRY(gemm(e, e->xn, d, &y->wqkv, d, e->qkv, 3 * d, T, 3 * d, d, NULL, y->bqkv, 0, 0));
-        QK_TRY(qk_enc_attention_launch(e->qkv, e->att, T, H, 64, win, scale, e->stream));
+        QK_TRY(qk_enc_attention_launch(e->qkv, e->att, NULL, T, H, 64, win, scale, e->stream));
         QK_TRY(gemm_add_ln(e, e->att, d, &y->wo, d, y->bo, T, y->ln2w, y->ln2b));
         QK_TRY(gemm(e, e->xn, d, &y->fc1w, d, e->mid, c->ffn_dim, T, c->ffn_dim, d, NULL, y->fc1b, 1, 0));
         const int last = l + 1 == c->layers;
@@ -475,6 +513,58 @@ static int run(qwen_hip_encoder *e, int mel_frames, int *tokens_out) {
     /* proj1 + GELU, proj2 on the ln_post rows (:358-371) */
     QK_TRY(gemm(e, e->xn, d, &e->p1w, d, e->mid, d, T, d, d, NULL, e->p1b, 1, 0));
     QK_TRY(gemm(e, e->mid, d, &e->p2w, d, e->out, c->output_dim, T, c->output_dim, d, NULL, e->p2b, 0, 0));
+    *tokens_out = T;
+    return 0;
+}
+
+/* The same on activations kept as bf16 halves (qk_enc_ring_launch): every
+ * product's rows are written as halves by their producer, the stem's patches
+ * are gathered from its pixels, and each residual projection's reduce also
+ * applies the next LayerNorm. */
+static int run_ring(qwen_hip_encoder *e, const float *mel, int mel_frames, int *tokens_out) {
+    const qwen_hip_enc_config *c = &e->cfg;
+    const int cw = c->chunk_size, d = c->d_model, H = c->heads;
+    const int chunks = (mel_frames + cw - 1) / cw;
+    const int last = mel_frames - (chunks - 1) * cw;
+    const int w1 = conv_out(cw), w2 = conv_out(w1), w3 = conv_out(w2);
+    const int T = qwen_hip_encoder_tokens(c, mel_frames);
+    uint16_t *const c1 = (uint16_t *)e->c1, *const c2 = (uint16_t *)e->c2, *const c3 = (uint16_t *)e->c3;
+    uint16_t *const xn = (uint16_t *)e->xn, *const att = (uint16_t *)e->att, *const mid = (uint16_t *)e->mid;
+    hipStream_t s = e->stream;
+#define RING(...)                                                                  \
+    do {                                                                           \
+        qk_enc_ring_args g_ = {__VA_ARGS__};                                       \
+        QK_TRY(qk_enc_ring_launch(&g_, e->gws, e->gws_elems, s));                  \
+    } while (0)
+    QK_TRY(qk_enc_conv1_halves_launch(mel, ENC_K1, e->c1w, e->c1b, c1, chunks, ENC_MEL, cw, 64, w1, mel_frames,
+                                      conv_out(last), s));
+    RING(.A = c1, .W = e->c2w.b16, .zero = e->zero, .M = chunks * 32 * w2, .N = ENC_CH, .K = ENC_K2, .taps = 9,
+         .in_h = 64, .in_w = w1, .col_h = 32, .col_w = w2, .chunks = chunks, .valid = conv_out(conv_out(last)),
+         .bias = e->c2b, .gelu = 1, .out = c2);
+    RING(.A = c2, .W = e->c3w.b16, .zero = e->zero, .M = chunks * 16 * w3, .N = ENC_CH, .K = ENC_K2, .taps = 9,
+         .in_h = 32, .in_w = w2, .col_h = 16, .col_w = w3, .chunks = chunks,
+         .valid = conv_out(conv_out(conv_out(last))), .bias = e->c3b, .gelu = 1, .out = c3);
+    /* conv_out + the chunk's positions, first LayerNorm */
+    RING(.A = c3, .W = e->cowr, .zero = e->zero, .M = T, .N = d, .K = ENC_CH * 16, .taps = 16, .in_h = 16, .in_w = w3,
+         .pe = e->pe, .pe_rows = w3, .C = e->x, .out = xn, .ln_w = e->L[0].ln1w, .ln_b = e->L[0].ln1b,
+         .ln_eps = 1e-5f);
+    const int win = w3 * (c->n_window_infer / cw);
+    const float scale = 1.0f / sqrtf((float)c->head_dim);
+    for (int l = 0; l < c->layers; l++) {
+        const enc_layer *y = &e->L[l];
+        const int end = l + 1 == c->layers;
+        RING(.A = xn, .W = y->wqkv.b16, .M = T, .N = 3 * d, .K = d, .bias = y->bqkv, .C = e->qkv);
+        QK_TRY(qk_enc_attention_launch(e->qkv, NULL, att, T, H, 64, win, scale, s));
+        RING(.A = att, .W = y->wo.b16, .M = T, .N = d, .K = d, .bias = y->bo, .add = 1, .C = e->x, .out = xn,
+             .ln_w = y->ln2w, .ln_b = y->ln2b, .ln_eps = 1e-5f);
+        RING(.A = xn, .W = y->fc1w.b16, .M = T, .N = c->ffn_dim, .K = d, .bias = y->fc1b, .gelu = 1, .out = mid);
+        RING(.A = mid, .W = y->fc2w.b16, .M = T, .N = d, .K = c->ffn_dim, .bias = y->fc2b, .add = 1, .C = e->x,
+             .out = xn, .ln_w = end ? e->lnpw : e->L[l + 1].ln1w, .ln_b = end ? e->lnpb : e->L[l + 1].ln1b,
+             .ln_eps = 1e-5f);
+    }
+    RING(.A = xn, .W = e->p1w.b16, .M = T, .N = d, .K = d, .bias = e->p1b, .gelu = 1, .out = mid);
+    RING(.A = mid, .W = e->p2w.b16, .M = T, .N = c->output_dim, .K = d, .bias = e->p2b, .C = e->out);
+#undef RING
     *tokens_out = T;
     return 0;
 }
@@ -495,7 +585,7 @@ int qwen_hip_encoder_forward(qwen_hip_encoder *e, const float *mel, int mel_fram
     if (!mel || !out) { qk_set_err("encoder: NULL mel or output"); return QWEN_HIP_EINVAL; }
     QK_HIP(hipMemcpyAsync(e->mel, mel, (size_t)ENC_MEL * mel_frames * 4, hipMemcpyHostToDevice, e->stream));
     int T = 0;
-    QK_TRY(run(e, mel_frames, &T));
+    QK_TRY(ring_ok(e) ? run_ring(e, e->mel, mel_frames, &T) : run_general(e, mel_frames, &T));
     QK_HIP(hipMemcpyAsync(out, e->out, (size_t)T * e->cfg.output_dim * 4, hipMemcpyDeviceToHost, e->stream));
     QK_HIP(hipStreamSynchronize(e->stream));
     return T;
@@ -505,9 +595,13 @@ int qwen_hip_encoder_forward_device(qwen_hip_encoder *e, const float *d_mel, int
     int rc = ready(e, mel_frames);
     if (rc) return rc;
     if (!d_mel || !d_out) { qk_set_err("encoder: NULL mel or output"); return QWEN_HIP_EINVAL; }
-    QK_HIP(hipMemcpyAsync(e->mel, d_mel, (size_t)ENC_MEL * mel_frames * 4, hipMemcpyDeviceToDevice, e->stream));
     int T = 0;
-    QK_TRY(run(e, mel_frames, &T));
+    if (ring_ok(e)) {
+        QK_TRY(run_ring(e, d_mel, mel_frames, &T));
+    } else {
+        QK_HIP(hipMemcpyAsync(e->mel, d_mel, (size_t)ENC_MEL * mel_frames * 4, hipMemcpyDeviceToDevice, e->stream));
+        QK_TRY(run_general(e, mel_frames, &T));
+    }
     QK_HIP(hipStreamSynchronize(e->stream));
     *d_out = e->out;
     return T;

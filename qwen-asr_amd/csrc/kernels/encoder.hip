@@ -3,11 +3,15 @@
 // transformer layers with windowed bidirectional attention -> ln_post,
 // proj1 + GELU, proj2).
 //
-// Every matrix product runs on the fp32 matrix cores (v_mfma_f32_16x16x4_f32):
-// the reference computes the encoder in fp32 on weights widened from bf16
-// (load_bf16_as_f32, qwen_asr_encoder.c:43-65), so products stay exact fp32
-// and only the summation order differs.
+// The reference computes the encoder in fp32 on weights widened from bf16
+// (load_bf16_as_f32, qwen_asr_encoder.c:43-65).  bf16-valued weights are kept in
+// bf16 (exact) and the fp32 activations are carried as hi + lo bf16 on the bf16
+// matrix cores; other weights, and attention, run on the fp32 matrix cores.
 //
+//   enc_ring     products on bf16 weights with activations kept as halves; the
+//                stem convolutions and conv_out gather their rows from the
+//                stem's pixels (enc_conv1_halves writes the first ones)
+// The general forms (any weight values and widths):
 //   enc_im2col   Conv2D(3x3, stride 2, pad 1) patches of all chunks at once:
 //                row n = (chunk, oh, ow), column k = (ki, kj, ic) tap-major
 //                (the reference's im2col, qwen_asr_kernels.c:566-590, with
@@ -27,6 +31,7 @@
 #include "common.h"
 #include "qk_kernels.h"
 #include "qwen_asr_hip.h"
+#include "ring.h"
 
 #include <math.h>
 
@@ -34,11 +39,15 @@ __device__ __forceinline__ f32x4 enc_mfma(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// GELU, tanh form (qwen_gelu, qwen_asr_kernels.c:886-893)
+// GELU, tanh form (qwen_gelu, qwen_asr_kernels.c:886-893): 0.5 v (1 + tanh u) =
+// v / (1 + e^(-2u)), with no cancellation for negative u.  The hardware exponential
+// and reciprocal: the error of e^(-2u) (|2u| ulp) is weighted by e / (1 + e)^2, at
+// most 0.4 ulp of v, as tanhf's.  (With tanhf or expf the serial chains of a GEMM
+// tile's 32 values per lane took as long as its k walk.)
 __device__ __forceinline__ float enc_gelu(float v) {
     const float x3 = v * v * v;
     const float inner = 0.7978845608028654f * (v + 0.044715f * x3);
-    return 0.5f * v * (1.0f + tanhf(inner));
+    return v * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * inner));
 }
 
 // ---------------------------------------------------------------------------
@@ -545,6 +554,342 @@ extern "C" int qk_enc_stem_rows_launch(const float *c3, float *rows, int chunks,
 }
 
 // ---------------------------------------------------------------------------
+// The bf16-weight encoder: every activation that feeds a product is kept as
+// rows of two bf16 halves, [K hi | K lo] (hi = bf16(x), lo = bf16(x - hi): the
+// bytes of an fp32 row), written by its producer, so the products stream both
+// operands through the LDS ring of ring.h with no conversion in the k loop.
+// Weights of other than bf16 values, or widths that are no multiple of 128,
+// run on enc_gemm_hl / enc_gemm above.
+//
+// What bounds it: at 100 to 400 rows these products are a few microseconds
+// each, mostly ramp, latency of the k walk and drain; a k tile staged through
+// registers (one in flight) took ~2x a ring step.  @RINGM@
+// ---------------------------------------------------------------------------
+typedef float ec_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 ec_bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t enc_pack(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((ec_f32x2){a, b}, ec_bf16x2));
+}
+
+__device__ __forceinline__ void enc_split2(float a, float b, uint32_t &hi, uint32_t &lo) {
+    hi = enc_pack(a, b);
+    lo = enc_pack(a - bf16_lo(hi), b - bf16_hi(hi));
+}
+
+// four values at columns n .. n + 3 of a row of n_cols
+__device__ __forceinline__ void enc_store_halves(uint16_t *row, int n_cols, int n, float4 v) {
+    uint2 h, l;
+    enc_split2(v.x, v.y, h.x, l.x);
+    enc_split2(v.z, v.w, h.y, l.y);
+    *reinterpret_cast<uint2 *>(row + n) = h;
+    *reinterpret_cast<uint2 *>(row + n_cols + n) = l;
+}
+
+// stem: row m = (chunk, oh, ow) is padding of the last chunk
+__device__ __forceinline__ bool enc_ring_pad(const qk_enc_ring_args &a, int m) {
+    if (a.valid <= 0) return false;
+    const int ow = m % a.col_w, c = m / (a.col_w * a.col_h);
+    return c == a.chunks - 1 && ow >= a.valid;
+}
+
+// Results of a product: split-K partials, fp32 + bias, or halves of the GELU.
+enum { ENC_PART, ENC_F32, ENC_GELU };
+
+// One tile of the product; GATHER: rows of A are gathered from stem pixels.  The
+// epilogue is chosen at compile time: with tests between the 32 values of a lane
+// their chains ran one after the other, 9.3 us of a 390 x 3584 x 896 GELU
+// product's 20 against @EPI@.
+template <int BM, int NST, bool GATHER, int EPI>
+__global__ __launch_bounds__(ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring_args a) {
+    using RS = RingShape<BM, 128>;
+    constexpr int NW = RS::NW, WGN = RS::WGN, WTN = RS::WTN, TN = RS::TN, AB = RS::AB, LPW = RS::LPW;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[NST * RS::STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * 128;
+    const int kb = blockIdx.z * a.kc, ke = min(a.K, kb + a.kc), nk = (ke - kb) / QK_GBK;
+    const int rr = lane >> 2, cl = (lane & 3) ^ ((rr >> 1) & 3);
+    f32x4 acc[2][TN];
+    if constexpr (GATHER) {
+        // the wave's A groups: hi and lo of rows m0 + 16 wave + rr; W rows past N re-read row N - 1
+        static_assert(BM / 16 == NW, "one hi and one lo group per wave");
+        const int m = min(m0 + 16 * wave + rr, a.M - 1);
+        int pix;
+        unsigned mask = 0;
+        if (a.taps == 9) {             // 3 x 3, stride 2, padding 1
+            const int ow = m % a.col_w, t = m / a.col_w, oh = t % a.col_h, c = t / a.col_h;
+            const int ih = 2 * oh - 1, iw = 2 * ow - 1;
+            pix = (c * a.in_h + ih) * a.in_w + iw;
+#pragma unroll
+            for (int tap = 0; tap < 9; tap++) {
+                const int y = ih + tap / 3, x = iw + tap % 3;
+                if (y >= 0 && y < a.in_h && x >= 0 && x < a.in_w) mask |= 1u << tap;
+            }
+        } else {                       // a token's column of in_h pixels, in_w apart
+            const int c = m / a.in_w;
+            pix = c * a.in_h * a.in_w + m % a.in_w;
+            mask = 0xffffffffu;
+        }
+        const uint16_t *w[LPW - 2];
+#pragma unroll
+        for (int j = 0; j < LPW - 2; j++)
+            w[j] = a.W + (size_t)min(n0 + 16 * (wave + NW * j) + rr, a.N - 1) * a.K + kb + 8 * cl;
+        ring_walk<BM, 128, NST>(nk, lds, acc, [&](int kt, unsigned char *st) {
+            // a 32-wide k tile lies in one tap
+            const int k = kb + kt * QK_GBK, tap = k / QK_ENC_CH, ic = k - tap * QK_ENC_CH;
+            const int off = a.taps == 9 ? (tap / 3) * a.in_w + tap % 3 : tap * a.in_w;
+            const uint16_t *p = (mask >> tap) & 1 ? a.A + (long)(pix + off) * (2 * QK_ENC_CH) : a.zero;
+            p += ic + 8 * cl;
+            lds_load16(p, st + 1024 * wave);
+            lds_load16(p + QK_ENC_CH, st + AB + 1024 * wave);
+#pragma unroll
+            for (int j = 0; j < LPW - 2; j++) lds_load16(w[j] + kt * QK_GBK, st + 2 * AB + 1024 * (wave + NW * j));
+        });
+    } else {
+        const uint16_t *src[LPW];
+        int dst[LPW];
+#pragma unroll
+        for (int j = 0; j < LPW; j++) {
+            const int g = wave + NW * j, ga = g < BM / 16 ? g : g - BM / 16;
+            src[j] = (g < BM / 8 ? a.A + (size_t)min(m0 + 16 * ga + rr, a.M - 1) * (2 * a.K) + (g < BM / 16 ? 0 : a.K)
+                                 : a.W + (size_t)min(n0 + 16 * (g - BM / 8) + rr, a.N - 1) * a.K) + kb + 8 * cl;
+            dst[j] = 1024 * g;         // A_hi, A_lo and W groups follow one another
+        }
+        ring_walk<BM, 128, NST>(nk, lds, acc, [&](int kt, unsigned char *st) {
+#pragma unroll
+            for (int j = 0; j < LPW; j++) lds_load16(src[j] + kt * QK_GBK, st + dst[j]);
+        });
+    }
+
+    const int wm = wave / WGN, wn = wave % WGN, mr = m0 + wm * 32 + 4 * (lane >> 4);
+    const bool odd = lane & 1;
+    float bias[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const int n = n0 + wn * WTN + j * 16 + (lane & 15);
+        bias[j] = EPI != ENC_PART && a.bias ? a.bias[min(n, a.N - 1)] : 0.0f;
+    }
+    bool pad[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) pad[i][r] = GATHER && EPI == ENC_GELU && enc_ring_pad(a, mr + 16 * i + r);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float v = acc[i][j][r];
+                if (EPI != ENC_PART) v += bias[j];
+                if (EPI == ENC_GELU) v = pad[i][r] ? 0.0f : enc_gelu(v);
+                acc[i][j][r] = v;
+            }
+    if constexpr (EPI == ENC_PART || EPI == ENC_F32) {
+        float *y = EPI == ENC_PART ? a.ws + (size_t)blockIdx.z * a.M * a.N : a.C;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    const int m = mr + 16 * i + r, n = n0 + wn * WTN + j * 16 + (lane & 15);
+                    if (m < a.M && n < a.N) y[(size_t)m * a.N + n] = acc[i][j][r];
+                }
+    } else {
+        // columns n and n ^ 1 lie in neighbouring lanes (N is even): the even one
+        // stores both hi halves, the odd one both lo halves
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) {
+                    const int m = mr + 16 * i + r, n = n0 + wn * WTN + j * 16 + (lane & 15);
+                    const float v = acc[i][j][r], pv = dpp_read<0xB1>(v);
+                    uint32_t h, l;
+                    enc_split2(odd ? pv : v, odd ? v : pv, h, l);
+                    if (m < a.M && n < a.N)
+                        *reinterpret_cast<uint32_t *>(a.out + (size_t)m * 2 * a.N + (odd ? a.N + n - 1 : n)) = odd ? l : h;
+                }
+    }
+}
+
+// Split-K partials summed in slice order, then the epilogue: 4 columns a thread.
+__global__ __launch_bounds__(256) void enc_ring_reduce(qk_enc_ring_args a) {
+    const long MN = (long)a.M * a.N, n4 = MN / 4;
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n4; e += (long)gridDim.x * 256) {
+        const float4 s = sum_splits4<QK_ENC_RING_SPLIT>(a.ws + 4 * e, a.split, MN);
+        const int m = (int)(4 * e / a.N), n = (int)(4 * e % a.N);
+        const float4 b = a.bias ? *reinterpret_cast<const float4 *>(a.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 v = make_float4(s.x + b.x, s.y + b.y, s.z + b.z, s.w + b.w);
+        if (a.gelu) v = make_float4(enc_gelu(v.x), enc_gelu(v.y), enc_gelu(v.z), enc_gelu(v.w));
+        if (enc_ring_pad(a, m)) v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (a.C) *reinterpret_cast<float4 *>(a.C + 4 * e) = v;
+        else enc_store_halves(a.out + (size_t)m * 2 * a.N, a.N, n, v);
+    }
+}
+
+// x = (x +) sum of the partials + bias (+ the positions' table), then its
+// LayerNorm as halves: one block per row, N <= 1024, 4 columns a thread.
+__global__ __launch_bounds__(256) void enc_ring_reduce_ln(qk_enc_ring_args a) {
+    __shared__ float red[2][4];
+    const int m = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n = 4 * threadIdx.x;
+    const bool on = n < a.N;
+    const int nc = on ? n : 0;
+    float *xr = a.C + (size_t)m * a.N + nc;
+    const float4 w = *reinterpret_cast<const float4 *>(a.ln_w + nc), b = *reinterpret_cast<const float4 *>(a.ln_b + nc);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f), o = v, p = v;
+    if (a.bias) v = *reinterpret_cast<const float4 *>(a.bias + nc);
+    if (a.pe) p = *reinterpret_cast<const float4 *>(a.pe + (size_t)(m % a.pe_rows) * a.N + nc);
+    if (a.add) o = *reinterpret_cast<const float4 *>(xr);
+    const float4 s = sum_splits4<QK_ENC_RING_SPLIT>(a.ws + (size_t)m * a.N + nc, a.split, (long)a.M * a.N);
+    v.x = ((s.x + v.x) + p.x) + o.x;
+    v.y = ((s.y + v.y) + p.y) + o.y;
+    v.z = ((s.z + v.z) + p.z) + o.z;
+    v.w = ((s.w + v.w) + p.w) + o.w;
+    if (on) *reinterpret_cast<float4 *>(xr) = v;
+    else v = make_float4(0.f, 0.f, 0.f, 0.f);
+    float t = wave_sum((v.x + v.y) + (v.z + v.w));
+    if (lane == 0) red[0][wave] = t;
+    __syncthreads();
+    const float mean = (red[0][0] + red[0][1] + red[0][2] + red[0][3]) / (float)a.N;
+    const float dx = v.x - mean, dy = v.y - mean, dz = v.z - mean, dw = v.w - mean;
+    t = wave_sum(on ? fmaf(dw, dw, fmaf(dz, dz, fmaf(dy, dy, dx * dx))) : 0.0f);
+    if (lane == 0) red[1][wave] = t;
+    __syncthreads();
+    const float var = (red[1][0] + red[1][1] + red[1][2] + red[1][3]) / (float)a.N;
+    const float inv = 1.0f / sqrtf(var + a.ln_eps);
+    if (on)
+        enc_store_halves(a.out + (size_t)m * 2 * a.N, a.N, n,
+                         make_float4(dx * inv * w.x + b.x, dy * inv * w.y + b.y, dz * inv * w.z + b.z,
+                                     dw * inv * w.w + b.w));
+}
+
+// Tile height and split of an M x N x K product.  64-row tiles (32 up to 32
+// rows; 128 where those alone give every CU a block).  K is split until the
+// launch has about QK_ENC_RING_TARGET blocks, k walks of 4 k tiles at least; a
+// product whose epilogue needs no reduce pass (`fused`) is only split where
+// its tiles would leave most CUs idle.
+extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, long ws_elems, int *bm, int *kc,
+                                 int *split) {
+    const long nt = (N + 127) / 128;
+    *bm = M <= 32 && !gather ? 32 : (long)((M + 127) / 128) * nt >= 256 ? 128 : 64;
+    const long tiles = (M + *bm - 1) / *bm * nt;
+    const int kt = K / QK_GBK;
+    long ns = (QK_ENC_RING_TARGET + tiles - 1) / tiles;
+    if (fused && tiles >= QK_ENC_RING_FUSED) ns = 1;
+    if (ns > QK_ENC_RING_SPLIT) ns = QK_ENC_RING_SPLIT;
+    if (ns > kt / 4) ns = kt / 4;
+    while (ns > 1 && ns * M * N > ws_elems) ns--;
+    if (ns < 1) ns = 1;
+    const int per = (int)((kt + ns - 1) / ns);
+    *kc = per * QK_GBK;
+    *split = (kt + per - 1) / per;
+}
+
+extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_elems, hipStream_t s) {
+    if (!a || !a->A || !a->W || a->M <= 0 || a->N <= 0 || (a->N & 3) || a->K <= 0 || a->K % QK_GBK) return QWEN_HIP_EINVAL;
+    const bool ln = a->ln_w != nullptr, gather = a->taps > 0;
+    if (ln ? (!a->ln_b || !a->C || !a->out || !ws || a->N > 1024 || (long)a->M * a->N > ws_elems || (a->pe && a->pe_rows <= 0))
+           : (!a->C == !a->out || a->pe || a->add || (a->gelu ? !a->out : !a->C) || (gather && a->C)))
+        return QWEN_HIP_EINVAL;
+    if (gather && (a->K != a->taps * QK_ENC_CH || (a->taps != 9 && a->taps != a->in_h) || a->taps > 32 || !a->zero ||
+                   a->in_h <= 0 || a->in_w <= 0 || (a->taps == 9 && (a->col_h <= 0 || a->col_w <= 0))))
+        return QWEN_HIP_EINVAL;
+    if (a->valid > 0 && (a->col_h <= 0 || a->col_w <= 0)) return QWEN_HIP_EINVAL;
+    qk_enc_ring_args g = *a;
+    int bm;
+    qk_enc_ring_plan(a->M, a->N, a->K, !ln, gather, ws ? ws_elems : 0, &bm, &g.kc, &g.split);
+    g.ws = ln || g.split > 1 ? ws : nullptr;
+    const dim3 grid((a->N + 127) / 128, (a->M + bm - 1) / bm, g.split), block(64 * ring_waves(bm, 128));
+    const int epi = g.ws ? ENC_PART : a->C ? ENC_F32 : ENC_GELU;
+#define QK_ENC_RING(BM_, NST_, G_, E_)                                     \
+    if (bm == BM_ && gather == G_ && epi == E_) enc_ring<BM_, NST_, G_, E_><<<grid, block, 0, s>>>(g);
+#define QK_ENC_RING_BM(BM_, NST_, G_) \
+    QK_ENC_RING(BM_, NST_, G_, ENC_PART) QK_ENC_RING(BM_, NST_, G_, ENC_GELU)
+    QK_ENC_RING_BM(128, 3, true) QK_ENC_RING_BM(64, 4, true)
+    QK_ENC_RING_BM(128, 3, false) QK_ENC_RING_BM(64, 4, false) QK_ENC_RING_BM(32, 4, false)
+    QK_ENC_RING(128, 3, false, ENC_F32) QK_ENC_RING(64, 4, false, ENC_F32) QK_ENC_RING(32, 4, false, ENC_F32)
+#undef QK_ENC_RING_BM
+#undef QK_ENC_RING
+    if (ln) {
+        enc_ring_reduce_ln<<<a->M, 256, 0, s>>>(g);
+    } else if (g.split > 1) {
+        long blocks = ((long)a->M * a->N / 4 + 255) / 256;
+        enc_ring_reduce<<<(int)(blocks < 4096 ? blocks : 4096), 256, 0, s>>>(g);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
+}
+
+// conv1 (one input channel) from the mel [128][frames], as halves [pos][480 hi |
+// 480 lo]: a thread holds 4 channels' weights and walks positions, 9 mel values
+// (the same for the 120 threads of a position) and 36 multiply-adds each.
+// Bound by the 4 bytes written per output.
+__global__ __launch_bounds__(256) void enc_conv1_halves(const float *mel, int kpad, const float *w, const float *b,
+                                                        uint16_t *out, int rows, int h_in, int w_in, int h_out,
+                                                        int w_out, int mel_frames, int chunks, int valid) {
+    constexpr int q4 = QK_ENC_CH / 4;
+    // the grid stride is a multiple of q4: a thread keeps one channel quad
+    const long i0 = blockIdx.x * 256L + threadIdx.x, stride = (long)gridDim.x * 256;
+    const int c0 = 4 * (int)(i0 % q4), dpos = (int)(stride / q4);
+    float wr[4][9], br[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        br[j] = b[c0 + j];
+#pragma unroll
+        for (int t = 0; t < 9; t++) wr[j][t] = w[(c0 + j) * kpad + t];
+    }
+    for (int pos = (int)(i0 / q4); pos < rows; pos += dpos) {
+        const int ow = pos % w_out, t1 = pos / w_out, oh = t1 % h_out, c = t1 / h_out;
+        float v[4] = {br[0], br[1], br[2], br[3]};
+#pragma unroll
+        for (int t = 0; t < 9; t++) {
+            const int ih = 2 * oh - 1 + t / 3, iw = 2 * ow - 1 + t % 3, f = c * w_in + iw;
+            const bool in = ih >= 0 && ih < h_in && iw >= 0 && iw < w_in && f < mel_frames;
+            const float x = in ? mel[(long)ih * mel_frames + f] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = fmaf(x, wr[j][t], v[j]);
+        }
+        const bool pad = c == chunks - 1 && ow >= valid;
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = pad ? 0.0f : enc_gelu(v[j]);
+        enc_store_halves(out + (size_t)pos * 2 * QK_ENC_CH, QK_ENC_CH, c0, make_float4(v[0], v[1], v[2], v[3]));
+    }
+}
+
+extern "C" int qk_enc_conv1_halves_launch(const float *mel, int kpad, const float *w, const float *b, uint16_t *out,
+                                          int chunks, int h_in, int w_in, int h_out, int w_out, int mel_frames,
+                                          int valid, hipStream_t s) {
+    const long rows = (long)chunks * h_out * w_out;
+    if (!mel || !w || !b || !out || kpad < 9 || rows <= 0 || rows > 0x7fffffffL || mel_frames <= 0) return QWEN_HIP_EINVAL;
+    constexpr int unit = 15;           // blocks: a multiple of 15, so the grid stride is one of 120 (256 * 15 = 32 * 120)
+    long blocks = (rows * (QK_ENC_CH / 4) + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    blocks = (blocks + unit - 1) / unit * unit;
+    enc_conv1_halves<<<(int)blocks, 256, 0, s>>>(mel, kpad, w, b, out, (int)rows, h_in, w_in, h_out, w_out, mel_frames,
+                                                 chunks, valid);
+    return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
+}
+
+// out[n][f ch + c] = in[n][c h + f]: conv_out's columns (channel, row) in the
+// order of a token's pixels (row, channel)
+__global__ __launch_bounds__(256) void enc_reorder(const uint16_t *in, uint16_t *out, int ch, int h, long n) {
+    const long e = blockIdx.x * 256L + threadIdx.x;
+    if (e >= n) return;
+    const int K = ch * h, k = (int)(e % K), f = k / ch, c = k % ch;
+    out[e] = in[e - k + c * h + f];
+}
+
+extern "C" int qk_enc_reorder_launch(const uint16_t *in, uint16_t *out, int rows, int ch, int h, hipStream_t s) {
+    const long n = (long)rows * ch * h;
+    if (!in || !out || n <= 0) return QWEN_HIP_EINVAL;
+    enc_reorder<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(in, out, ch, h, n);
+    return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
+}
+
+// ---------------------------------------------------------------------------
 // LayerNorm, one block per row (qwen_layer_norm: mean, then mean of squared
 // deviations, then (x - mean) * inv_std * w + b).
 // ---------------------------------------------------------------------------
@@ -582,51 +927,69 @@ extern "C" int qk_enc_layernorm_launch(const float *x, const float *w, const flo
 }
 
 // ---------------------------------------------------------------------------
-// Windowed bidirectional attention, head_dim 64, on the fp32 matrix cores.
-// Block = one wave: 16 queries of one window, one head.  S^T = K Q^T and
-// O^T += V^T P^T on v_mfma_f32_16x16x4_f32: lane l holds query l & 15, keys
-// (first product) and dims (second) 4 (l >> 4) + r of each 16-row tile, so
-// the scores come out in the register layout the second product takes as
-// its B operand.  Online softmax over blocks of 64 keys of the window
-// [ws, we); K and V are read straight from qkv [T][3 H 64] (q | k | v).
+// Windowed bidirectional attention, head_dim 64, on the fp32 matrix cores
+// (v_mfma_f32_16x16x4_f32).  Block: 16 queries of one window and one head, 4
+// waves; wave w takes the keys 32 w + 128 i .. + 32 of the window, two tiles of
+// 16.  S^T = K Q^T: lane l holds query l & 15 and keys 4 (l >> 4) + r of a tile,
+// the layout the second product takes as its B operand; O^T += V^T P^T with row
+// l & 15 of tile dt standing for dim 4 (l & 15) + dt, so a lane's V values of a
+// key are one float4 and its results (dims 16 (l >> 4) + 4 r + dt) are 16
+// consecutive dims.  Online softmax per wave; the waves' (m, l, o) meet in LDS.
+// Bound by latency (104 keys a window: one round of 16 independent 16-byte
+// loads per lane, then 64 MFMAs): a window walked by one wave in blocks of 64
+// keys with 4-byte V loads took @ATT@.
+// The result goes out as fp32 or, for the bf16 products, as halves.
 // ---------------------------------------------------------------------------
 #define EA_Q 16
-#define EA_KB 64
+#define EA_KW 32                  // keys per wave and round
+#define EA_LD 68                  // floats per query of a wave's o (16-byte rows, spread over the banks)
 
-__global__ __launch_bounds__(64) void enc_attention(const float *qkv, float *out, int T, int H, int win, float scale) {
+__global__ __launch_bounds__(256) void enc_attention(const float *qkv, float *out, uint16_t *out16, int T, int H, int win,
+                                                     float scale) {
     constexpr int hd = 64;
-    const int lane = threadIdx.x, h = blockIdx.y;
+    __shared__ float sm[4][EA_Q], sl[4][EA_Q];
+    __shared__ __attribute__((aligned(16))) float so[4][EA_Q][EA_LD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = blockIdx.y;
     const int lq = lane & 15, lg = lane >> 4;
     const int tpw = (win + EA_Q - 1) / EA_Q;
     const int ws = (blockIdx.x / tpw) * win, we = min(T, ws + win);
     const int q0 = ws + (blockIdx.x % tpw) * EA_Q;
     if (q0 >= we) return;                              // whole block: a short last window
     const long stride = 3L * H * hd;
-    const int qi = q0 + lq;
-    const float *qrow = qkv + (long)min(qi, T - 1) * stride + h * hd;
+    const float *qrow = qkv + (long)min(q0 + lq, T - 1) * stride + h * hd;
     const float *kbase = qkv + (long)H * hd + h * hd, *vbase = qkv + 2L * H * hd + h * hd;
 
     float4 q[4];                                       // Q^T operand: dims 16 kb + 4 lg + c
 #pragma unroll
     for (int kb = 0; kb < 4; kb++) q[kb] = *reinterpret_cast<const float4 *>(qrow + 16 * kb + 4 * lg);
-    f32x4 o[4];                                        // O^T[16 dt + 4 lg + r][query lq]
+    f32x4 o[4];                                        // O^T: dims 16 lg + 4 r + dt of query lq
 #pragma unroll
     for (int dt = 0; dt < 4; dt++) o[dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float m = -1e30f, l = 0.0f;                        // the reference's max_score start
 
-    for (int k0 = ws; k0 < we; k0 += EA_KB) {
-        float p[4][4];                                 // key k0 + 16 t + 4 lg + r
+    for (int k0 = ws + EA_KW * wave; k0 < we; k0 += 4 * EA_KW) {
+        float4 kk[2][4], vv[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const float *krow = kbase + (long)min(k0 + 16 * t + lq, T - 1) * stride + 4 * lg;
+#pragma unroll
+            for (int kb = 0; kb < 4; kb++) kk[t][kb] = *reinterpret_cast<const float4 *>(krow + 16 * kb);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                vv[t][c] = *reinterpret_cast<const float4 *>(vbase + (long)min(k0 + 16 * t + 4 * lg + c, T - 1) * stride +
+                                                             4 * lq);
+        float p[2][4];                                 // key k0 + 16 t + 4 lg + r
         float mx = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const float *krow = kbase + (long)min(k0 + 16 * t + lq, T - 1) * stride;
+        for (int t = 0; t < 2; t++) {
             f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kb = 0; kb < 4; kb++) {
-                const float4 kk = *reinterpret_cast<const float4 *>(krow + 16 * kb + 4 * lg);
+            for (int kb = 0; kb < 4; kb++)
 #pragma unroll
-                for (int c = 0; c < 4; c++) acc = enc_mfma((&kk.x)[c], (&q[kb].x)[c], acc);
-            }
+                for (int c = 0; c < 4; c++) acc = enc_mfma((&kk[t][kb].x)[c], (&q[kb].x)[c], acc);
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 p[t][r] = k0 + 16 * t + 4 * lg + r < we ? acc[r] * scale : -INFINITY;
@@ -638,7 +1001,7 @@ __global__ __launch_bounds__(64) void enc_attention(const float *qkv, float *out
         const float corr = __expf(m - mn);
         float sum = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+        for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 p[t][r] = __expf(p[t][r] - mn);
@@ -649,32 +1012,50 @@ __global__ __launch_bounds__(64) void enc_attention(const float *qkv, float *out
 #pragma unroll
         for (int dt = 0; dt < 4; dt++) o[dt] *= corr;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            if (k0 + 16 * t >= we) break;              // uniform: the tile holds no key of the window
+        for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const float *vrow = vbase + (long)min(k0 + 16 * t + 4 * lg + c, T - 1) * stride;
+            for (int c = 0; c < 4; c++)
 #pragma unroll
-                for (int dt = 0; dt < 4; dt++) o[dt] = enc_mfma(vrow[16 * dt + lq], p[t][c], o[dt]);
-            }
-        }
+                for (int dt = 0; dt < 4; dt++) o[dt] = enc_mfma((&vv[t][c].x)[dt], p[t][c], o[dt]);
     }
     l = xor_sum16_32(l);
-    if (qi >= we) return;
-    const float inv = 1.0f / l;
-    float *orow = out + (long)qi * H * hd + h * hd + 4 * lg;
+    if (lg == 0) {
+        sm[wave][lq] = m;
+        sl[wave][lq] = l;
+    }
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
-        *reinterpret_cast<float4 *>(orow + 16 * dt) =
-            make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
+    for (int r = 0; r < 4; r++)
+        *reinterpret_cast<float4 *>(&so[wave][lq][16 * lg + 4 * r]) = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
+    __syncthreads();
+    // thread: query tid / 16, dims 4 (tid % 16) .. + 3; wave 0 always holds keys, so M is finite
+    const int qq = threadIdx.x >> 4, d = 4 * (threadIdx.x & 15);
+    const float M = fmaxf(fmaxf(sm[0][qq], sm[1][qq]), fmaxf(sm[2][qq], sm[3][qq]));
+    float L = 0.0f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const float e = __expf(sm[w][qq] - M);
+        const float4 v = *reinterpret_cast<const float4 *>(&so[w][qq][d]);
+        L = fmaf(sl[w][qq], e, L);
+        acc.x = fmaf(v.x, e, acc.x);
+        acc.y = fmaf(v.y, e, acc.y);
+        acc.z = fmaf(v.z, e, acc.z);
+        acc.w = fmaf(v.w, e, acc.w);
+    }
+    const int qi = q0 + qq;
+    if (qi >= we) return;
+    const float inv = 1.0f / L;
+    const float4 v = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    if (out16) enc_store_halves(out16 + (size_t)qi * 2 * H * hd, H * hd, h * hd + d, v);
+    else *reinterpret_cast<float4 *>(out + (long)qi * H * hd + h * hd + d) = v;
 }
 
-extern "C" int qk_enc_attention_launch(const float *qkv, float *out, int T, int H, int hd, int win, float scale,
-                                       hipStream_t s) {
-    if (!qkv || !out || T <= 0 || H <= 0 || hd != 64 || win <= 0) return QWEN_HIP_EINVAL;
+extern "C" int qk_enc_attention_launch(const float *qkv, float *out, uint16_t *out16, int T, int H, int hd, int win,
+                                       float scale, hipStream_t s) {
+    if (!qkv || !out == !out16 || T <= 0 || H <= 0 || hd != 64 || win <= 0) return QWEN_HIP_EINVAL;
     const long nwin = (T + win - 1) / win, tpw = (win + EA_Q - 1) / EA_Q;
     if (nwin * tpw > 0x7fffffffL) return QWEN_HIP_EINVAL;
     dim3 grid((unsigned)(nwin * tpw), H);
-    enc_attention<<<grid, 64, 0, s>>>(qkv, out, T, H, win, scale);
+    enc_attention<<<grid, 256, 0, s>>>(qkv, out, out16, T, H, win, scale);
     return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
 }

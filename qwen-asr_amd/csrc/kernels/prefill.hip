@@ -11,6 +11,7 @@
 #include "common.h"
 #include "qk_kernels.h"
 #include "qwen_asr_hip.h"
+#include "ring.h"
 
 #include <math.h>
 
@@ -430,7 +431,6 @@ __global__ __launch_bounds__(256) void gemm_hilo(const uint16_t *__restrict__ ah
 // p ^ ((r / 4) % 4), also 16 distinct groups, it read 0.12 conflict cycles
 // per active LDS cycle).
 // ---------------------------------------------------------------------------
-#define QK_GBK 32
 
 template <int EPI, int BM>
 __global__ __launch_bounds__(512, 1) void gemm_hilo_wide(const uint16_t *__restrict__ ahi,
@@ -559,117 +559,6 @@ static void gemm_wide_dispatch(const uint16_t *a_hi, const uint16_t *a_lo, const
 // per CU.  The 16-row load groups of a stage (A_hi, A_lo, W) are dealt
 // round-robin to the waves: LPW 1 KB load instructions per wave and stage.
 // ---------------------------------------------------------------------------
-__host__ __device__ constexpr int ring_waves(int bm, int bn) { return bm / 32 * (bn / 64) < 4 ? 4 : bm / 32 * (bn / 64); }
-__device__ constexpr int vmcnt_imm(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
-
-// wait until at most later * LPW of this wave's loads are outstanding
-// (later <= MAXL: the stages issued after the one about to be read)
-template <int LPW, int MAXL>
-__device__ __forceinline__ void ring_wait(int later) {
-    if constexpr (MAXL > 0) {
-        if (later >= MAXL) {
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(MAXL * LPW));
-            return;
-        }
-        ring_wait<LPW, MAXL - 1>(later);
-    } else {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    }
-}
-
-// 16 bytes per lane from global memory straight into LDS (lane l at byte 16 l
-// of the 1 KB at l0).  Called through this helper: with the builtin written in
-// the kernel on pointers held in an array, hipcc's host pass drops the
-// kernel's launch stub.
-__device__ __forceinline__ void lds_load16(const uint16_t *g, unsigned char *l0) {
-    __builtin_amdgcn_global_load_lds(g, l0, 16, 0, 0);
-}
-
-template <int BM, int BN>
-struct RingShape {
-    static constexpr int NW = ring_waves(BM, BN), WGM = BM / 32, WGN = NW / WGM, WTN = BN / WGN, TM = 2,
-                         TN = WTN / 16;
-    static constexpr int AB = BM * 64, STAGE = 2 * AB + BN * 64;   // bytes: one A half, one stage
-    static constexpr int GROUPS = (2 * BM + BN) / 16, LPW = GROUPS / NW;
-    static_assert(WGM * WGN == NW && WTN % 16 == 0 && GROUPS % NW == 0, "wave grid / load split");
-};
-
-// The k walk of block (blockIdx.x, blockIdx.y, blockIdx.z) into acc: wave
-// (wm, wn) = (wave / WGN, wave % WGN) holds rows m0 + 32 wm + 16 i + 4 (l >> 4)
-// + r, columns n0 + WTN wn + 16 j + (l & 15) (lane l, acc[i][j][r]).  lds:
-// NST stages of the kernel's shared memory.
-template <int BM, int BN, int NST>
-__device__ __forceinline__ void ring_tile(const uint16_t *__restrict__ ahi, const uint16_t *__restrict__ alo,
-                                          const uint16_t *__restrict__ W, int M, int K, int kc, unsigned char *lds,
-                                          f32x4 (&acc)[2][RingShape<BM, BN>::TN]) {
-    using RS = RingShape<BM, BN>;
-    constexpr int NW = RS::NW, WGN = RS::WGN, WTN = RS::WTN, TM = RS::TM, TN = RS::TN;
-    constexpr int AB = RS::AB, STAGE = RS::STAGE, LPW = RS::LPW;
-    static_assert((NST - 2) * LPW <= 63 && NST * STAGE <= 160 * 1024, "vmcnt / LDS range");
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int kb = blockIdx.z * kc, ke = min(K, kb + kc);
-    const int nk = (ke - kb) / QK_GBK;
-
-    // this lane's load slots: row rr of each of the wave's 16-row groups,
-    // k chunk cl (swizzled); rows past M re-read row M - 1 (results dropped)
-    const int rr = lane >> 2, cl = (lane & 3) ^ ((rr >> 1) & 3);
-    const uint16_t *src[LPW];
-    int dst[LPW];
-#pragma unroll
-    for (int j = 0; j < LPW; j++) {
-        const int g = wave + NW * j;
-        if (g < BM / 16) {
-            src[j] = ahi + (size_t)min(m0 + 16 * g + rr, M - 1) * K + kb + 8 * cl;
-            dst[j] = 1024 * g;
-        } else if (g < BM / 8) {
-            src[j] = alo + (size_t)min(m0 + 16 * (g - BM / 16) + rr, M - 1) * K + kb + 8 * cl;
-            dst[j] = AB + 1024 * (g - BM / 16);
-        } else {
-            src[j] = W + (size_t)(n0 + 16 * (g - BM / 8) + rr) * K + kb + 8 * cl;
-            dst[j] = 2 * AB + 1024 * (g - BM / 8);
-        }
-    }
-    auto issue = [&](int kt) {
-        unsigned char *st = lds + (kt % NST) * STAGE;
-#pragma unroll
-        for (int j = 0; j < LPW; j++) lds_load16(src[j] + kt * QK_GBK, st + dst[j]);
-    };
-
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-    const int fr = lane & 15;
-    const int fo = fr * 64 + 16 * ((lane >> 4) ^ ((fr >> 1) & 3));
-    for (int t = 0; t < NST - 1 && t < nk; t++) issue(t);
-    for (int kt = 0; kt < nk; kt++) {
-        ring_wait<LPW, NST - 2>(min(nk - 1 - kt, NST - 2));
-        // every wave's share of stage kt is in LDS and stage kt - 1 is free (a
-        // plain s_barrier: __syncthreads() would also drain the later stages)
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (kt + NST - 1 < nk) issue(kt + NST - 1);
-        const unsigned char *st = lds + (kt % NST) * STAGE;
-        bf16x8 bfr[TN];
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-            bfr[j] = *reinterpret_cast<const bf16x8 *>(st + 2 * AB + (wn * WTN + j * 16) * 64 + fo);
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int ro = (wm * 32 + i * 16) * 64 + fo;
-            const bf16x8 ah = *reinterpret_cast<const bf16x8 *>(st + ro);
-            const bf16x8 al = *reinterpret_cast<const bf16x8 *>(st + AB + ro);
-#pragma unroll
-            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bfr[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bfr[j], acc[i][j], 0, 0, 0);
-        }
-    }
-}
-
 template <int EPI, int BM, int BN, int NST>
 __global__ __launch_bounds__(ring_waves(BM, BN) * 64) void gemm_hilo_ring(const uint16_t *__restrict__ ahi,
                                                                            const uint16_t *__restrict__ alo,

@@ -409,7 +409,49 @@ int qk_enc_stem_rows_launch(const float *c3, float *rows, int chunks, int w, int
                             hipStream_t s);
 int qk_enc_layernorm_launch(const float *x, const float *w, const float *b, float *out, int rows, int D, float eps,
                             hipStream_t s);
-int qk_enc_attention_launch(const float *qkv, float *out, int T, int H, int hd, int win, float scale, hipStream_t s);
+/* the result as fp32 [T][64 H] (out) or as halves (out16, see below) */
+int qk_enc_attention_launch(const float *qkv, float *out, uint16_t *out16, int T, int H, int hd, int win, float scale,
+                            hipStream_t s);
+
+/* Products on bf16 weights with the activations kept as "halves": rows of 2 K
+ * bf16, [K hi | K lo] (hi = bf16(x), lo = bf16(x - hi)).
+ * A: rows of halves [M][2 K], or (taps > 0) stem pixels [..][2 * 480] halves from
+ * which the rows are gathered, K = taps * 480 tap-major: taps 9 is a 3x3, stride
+ * 2, pad 1 window over [chunk][in_h][in_w] pixels for row m = (chunk, oh, ow) of
+ * col_h x col_w, with `zero` (2 * 480 zeros) outside; taps == in_h is pixel
+ * column m % in_w of chunk m / in_w, top to bottom.
+ * Result, one of: C fp32 [M][N] (+ bias); out halves [M][2 N] of the GELU (bias
+ * added before; valid > 0: row m's positions ow >= valid of the last chunk are 0); with
+ * ln_w, x = C (+= when add) product + bias + pe[m % pe_rows] and out = halves of
+ * LayerNorm(x) (N <= 1024).  ws: split-K partials (always used with ln_w, then at
+ * least M N floats).  kc, split and ws of the struct are set by the launcher. */
+#define QK_ENC_CH 480             /* channels of the stem, QWEN_CONV_HIDDEN (qwen_asr.h:39) */
+#define QK_ENC_RING_TARGET 256    /* blocks a split launch aims for */
+#define QK_ENC_RING_FUSED 96      /* tiles from which a product without a reduce pass is not split */
+#define QK_ENC_RING_SPLIT 8       /* at most */
+typedef struct {
+    const uint16_t *A, *W, *zero;
+    int M, N, K;
+    int taps, in_h, in_w, col_h, col_w, chunks, valid;
+    const float *bias, *pe;
+    int pe_rows, gelu, add;
+    float *C;
+    uint16_t *out;
+    const float *ln_w, *ln_b;
+    float ln_eps;
+    float *ws;
+    int kc, split;
+} qk_enc_ring_args;
+int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_elems, hipStream_t s);
+/* tile rows, k per split and splits of such a product (fused: no reduce pass needed) */
+void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, long ws_elems, int *bm, int *kc, int *split);
+/* conv1 from the mel [h_in][mel_frames] (chunks of w_in frames) and weights
+ * w[480][kpad] (9 taps) as halves [chunk][h_out][w_out][2 * 480], + bias, GELU,
+ * the last chunk's positions ow >= valid 0 */
+int qk_enc_conv1_halves_launch(const float *mel, int kpad, const float *w, const float *b, uint16_t *out, int chunks,
+                               int h_in, int w_in, int h_out, int w_out, int mel_frames, int valid, hipStream_t s);
+/* out[n][f * ch + c] = in[n][c * h + f] */
+int qk_enc_reorder_launch(const uint16_t *in, uint16_t *out, int rows, int ch, int h, hipStream_t s);
 
 /* ---- elementwise (op-level ABI) --------------------------------------- */
 int qk_add_launch(float *a, const float *b, long n, hipStream_t s);
