@@ -47,8 +47,8 @@ struct qwen_hip_encoder {
     hipStream_t stream;
     float *c1w, *c1b, *c2b, *c3b, *lnpw, *lnpb, *p1b, *p2b, *pe;
     enc_mat c2w, c3w, cow, p1w, p2w;
-    uint16_t *cowr;   /* cow.b16 with its columns in (row, channel) order */
-    uint16_t *zero;   /* 2 * ENC_CH zeros: the pixels outside an image */
+    uint16_t *c2t, *c3t, *cowt;   /* the bf16 stem matrices as the gathering products read them */
+    uint16_t *zero;               /* 64 zeros: the pixels outside an image */
     int stem_loaded;
     enc_layer L[QWEN_HIP_ENC_MAX_LAYERS];
     /* activations, sized for cap_chunks chunks */
@@ -115,7 +115,7 @@ void qwen_hip_encoder_destroy(qwen_hip_encoder *e) {
                   (void **)&e->cow.f32, (void **)&e->cow.b16, (void **)&e->lnpw,    (void **)&e->lnpb,
                   (void **)&e->p1w.f32, (void **)&e->p1w.b16, (void **)&e->p1b,     (void **)&e->p2w.f32,
                   (void **)&e->p2w.b16, (void **)&e->p2b,     (void **)&e->pe,
-                  (void **)&e->cowr,    (void **)&e->zero};
+                  (void **)&e->c2t,     (void **)&e->c3t,     (void **)&e->cowt,    (void **)&e->zero};
     for (size_t i = 0; i < sizeof(w) / sizeof(w[0]); i++) dfree(w[i]);
     for (int l = 0; l < QWEN_HIP_ENC_MAX_LAYERS; l++) {
         enc_layer *y = &e->L[l];
@@ -173,7 +173,7 @@ qwen_hip_encoder *qwen_hip_encoder_create(const qwen_hip_enc_config *cfg, int de
         return NULL;
     }
     free(pe);
-    if (dmalloc((void **)&e->zero, 2 * ENC_CH * 2) || hipMemset(e->zero, 0, 2 * ENC_CH * 2) != hipSuccess) {
+    if (dmalloc((void **)&e->zero, 128) || hipMemset(e->zero, 0, 128) != hipSuccess) {
         qwen_hip_encoder_destroy(e);
         return NULL;
     }
@@ -220,6 +220,13 @@ static int up(float **dst, const float *src, size_t n) {
     if (!*dst) QK_TRY(dmalloc((void **)dst, n * sizeof(float)));
     QK_HIP(hipMemcpy(*dst, src, n * sizeof(float), hipMemcpyHostToDevice));
     return 0;
+}
+
+/* the gathering products' copy of a bf16 matrix [rows][ch * h] */
+static int tiled(qwen_hip_encoder *e, const enc_mat *m, uint16_t **t, int rows, int ch, int h) {
+    if (!m->b16) return 0;
+    if (!*t) QK_TRY(dmalloc((void **)t, (size_t)rows * ch * h * 2));
+    return qk_enc_tile_weights_launch(m->b16, *t, rows, ch, h, e->stream);
 }
 
 int qwen_hip_encoder_load_layer(qwen_hip_encoder *e, int l, const qwen_hip_enc_layer_weights *w) {
@@ -285,11 +292,10 @@ int qwen_hip_encoder_load_stem(qwen_hip_encoder *e, const qwen_hip_enc_stem_weig
     QK_TRY(up(&e->c2b, w->conv2_b, ENC_CH));
     QK_TRY(up(&e->c3b, w->conv3_b, ENC_CH));
     QK_TRY(up_mat(&e->cow, ko, 0, w->conv_out_w, ko, w->conv_out_w && bf16_exact(w->conv_out_w, ko)));
-    if (e->cow.b16) {
-        if (!e->cowr) QK_TRY(dmalloc((void **)&e->cowr, ko * 2));
-        QK_TRY(qk_enc_reorder_launch(e->cow.b16, e->cowr, (int)d, ENC_CH, 16, e->stream));
-        QK_HIP(hipStreamSynchronize(e->stream));
-    }
+    QK_TRY(tiled(e, &e->c2w, &e->c2t, ENC_CH, ENC_K2, 1));
+    QK_TRY(tiled(e, &e->c3w, &e->c3t, ENC_CH, ENC_K2, 1));
+    QK_TRY(tiled(e, &e->cow, &e->cowt, (int)d, ENC_CH, 16));
+    QK_HIP(hipStreamSynchronize(e->stream));
     QK_TRY(up(&e->lnpw, w->ln_post_w, d));
     QK_TRY(up(&e->lnpb, w->ln_post_b, d));
     QK_TRY(up_mat(&e->p1w, d * d, 0, w->proj1_w, d * d, w->proj1_w && bf16_exact(w->proj1_w, d * d)));
@@ -424,7 +430,7 @@ static int reserve_cols(qwen_hip_encoder *e, int chunks) {
 static int ring_ok(const qwen_hip_encoder *e) {
     const qwen_hip_enc_config *c = &e->cfg;
     if (c->d_model > 1024 || c->ffn_dim % 32 || c->output_dim % 4) return 0;
-    int ok = e->c2w.b16 && e->c3w.b16 && e->cow.b16 && e->cowr && e->p1w.b16 && e->p2w.b16;
+    int ok = e->c2w.b16 && e->c3w.b16 && e->cow.b16 && e->p1w.b16 && e->p2w.b16;
     for (int l = 0; l < c->layers; l++)
         ok = ok && e->L[l].wqkv.b16 && e->L[l].wo.b16 && e->L[l].fc1w.b16 && e->L[l].fc2w.b16;
     return ok;
@@ -538,14 +544,14 @@ static int run_ring(qwen_hip_encoder *e, const float *mel, int mel_frames, int *
     } while (0)
     QK_TRY(qk_enc_conv1_halves_launch(mel, ENC_K1, e->c1w, e->c1b, c1, chunks, ENC_MEL, cw, 64, w1, mel_frames,
                                       conv_out(last), s));
-    RING(.A = c1, .W = e->c2w.b16, .zero = e->zero, .M = chunks * 32 * w2, .N = ENC_CH, .K = ENC_K2, .taps = 9,
+    RING(.A = c1, .W = e->c2t, .zero = e->zero, .M = chunks * 32 * w2, .N = ENC_CH, .K = ENC_K2, .taps = 9,
          .in_h = 64, .in_w = w1, .col_h = 32, .col_w = w2, .chunks = chunks, .valid = conv_out(conv_out(last)),
          .bias = e->c2b, .gelu = 1, .out = c2);
-    RING(.A = c2, .W = e->c3w.b16, .zero = e->zero, .M = chunks * 16 * w3, .N = ENC_CH, .K = ENC_K2, .taps = 9,
+    RING(.A = c2, .W = e->c3t, .zero = e->zero, .M = chunks * 16 * w3, .N = ENC_CH, .K = ENC_K2, .taps = 9,
          .in_h = 32, .in_w = w2, .col_h = 16, .col_w = w3, .chunks = chunks,
          .valid = conv_out(conv_out(conv_out(last))), .bias = e->c3b, .gelu = 1, .out = c3);
     /* conv_out + the chunk's positions, first LayerNorm */
-    RING(.A = c3, .W = e->cowr, .zero = e->zero, .M = T, .N = d, .K = ENC_CH * 16, .taps = 16, .in_h = 16, .in_w = w3,
+    RING(.A = c3, .W = e->cowt, .zero = e->zero, .M = T, .N = d, .K = ENC_CH * 16, .taps = 16, .in_h = 16, .in_w = w3,
          .pe = e->pe, .pe_rows = w3, .C = e->x, .out = xn, .ln_w = e->L[0].ln1w, .ln_b = e->L[0].ln1b,
          .ln_eps = 1e-5f);
     const int win = w3 * (c->n_window_infer / cw);

@@ -557,7 +557,11 @@ extern "C" int qk_enc_stem_rows_launch(const float *c3, float *rows, int chunks,
 // The bf16-weight encoder: every activation that feeds a product is kept as
 // rows of two bf16 halves, [K hi | K lo] (hi = bf16(x), lo = bf16(x - hi): the
 // bytes of an fp32 row), written by its producer, so the products stream both
-// operands through the LDS ring of ring.h with no conversion in the k loop.
+// operands through the LDS ring of ring.h with no conversion in the k loop.  Stem
+// pixels hold their 480 channels as 15 times [32 hi | 32 lo], and the weights of
+// the products that gather them lie as [K / 32][N][32]: a 32-deep k tile then
+// reads whole 128-byte lines (with half lines the load path bounded these
+// products: @CONV@).
 // Weights of other than bf16 values, or widths that are no multiple of 128,
 // run on enc_gemm_hl / enc_gemm above.
 //
@@ -577,13 +581,15 @@ __device__ __forceinline__ void enc_split2(float a, float b, uint32_t &hi, uint3
     lo = enc_pack(a - bf16_lo(hi), b - bf16_hi(hi));
 }
 
-// four values at columns n .. n + 3 of a row of n_cols
+// four values at columns n .. n + 3 of a row of n_cols, or (PIXEL) of a stem pixel
+template <bool PIXEL>
 __device__ __forceinline__ void enc_store_halves(uint16_t *row, int n_cols, int n, float4 v) {
     uint2 h, l;
     enc_split2(v.x, v.y, h.x, l.x);
     enc_split2(v.z, v.w, h.y, l.y);
-    *reinterpret_cast<uint2 *>(row + n) = h;
-    *reinterpret_cast<uint2 *>(row + n_cols + n) = l;
+    row += PIXEL ? n + (n & ~31) : n;
+    *reinterpret_cast<uint2 *>(row) = h;
+    *reinterpret_cast<uint2 *>(row + (PIXEL ? 32 : n_cols)) = l;
 }
 
 // stem: row m = (chunk, oh, ow) is padding of the last chunk
@@ -600,50 +606,73 @@ enum { ENC_PART, ENC_F32, ENC_GELU };
 // epilogue is chosen at compile time: with tests between the 32 values of a lane
 // their chains ran one after the other, 9.3 us of a 390 x 3584 x 896 GELU
 // product's 20 against @EPI@.
-template <int BM, int NST, bool GATHER, int EPI>
-__global__ __launch_bounds__(ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring_args a) {
+template <int BM, int NST, bool GATHER, int EPI, int KG>
+__global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring_args a) {
     using RS = RingShape<BM, 128>;
     constexpr int NW = RS::NW, WGN = RS::WGN, WTN = RS::WTN, TN = RS::TN, AB = RS::AB, LPW = RS::LPW;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[NST * RS::STAGE];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int NI = KG == 2 ? 1 : 2;                // 16-row tiles this wave finishes
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[KG * NST * RS::STAGE];   // two groups: RingShape2's stages
+    const int lane = threadIdx.x & 63, bwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = bwave / NW, wave = bwave % NW;      // k group, wave of the group
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * 128;
     const int kb = blockIdx.z * a.kc, ke = min(a.K, kb + a.kc), nk = (ke - kb) / QK_GBK;
     const int rr = lane >> 2, cl = (lane & 3) ^ ((rr >> 1) & 3);
-    f32x4 acc[2][TN];
+    f32x4 acc[NI][TN];
     if constexpr (GATHER) {
-        // the wave's A groups: hi and lo of rows m0 + 16 wave + rr; W rows past N re-read row N - 1
-        static_assert(BM / 16 == NW, "one hi and one lo group per wave");
-        const int m = min(m0 + 16 * wave + rr, a.M - 1);
-        int pix;
-        unsigned mask = 0;
-        if (a.taps == 9) {             // 3 x 3, stride 2, padding 1
-            const int ow = m % a.col_w, t = m / a.col_w, oh = t % a.col_h, c = t / a.col_h;
-            const int ih = 2 * oh - 1, iw = 2 * ow - 1;
-            pix = (c * a.in_h + ih) * a.in_w + iw;
+        // the wave's A groups: rows m0 + 8 (2 wave + h) + lane / 8, h = 0, 1
+        static_assert(BM / 16 == NW && KG == 1, "two 8-row groups per wave");
+        const int r8 = lane >> 3, c8 = (lane & 7) ^ r8;
+        int pix[2];
+        unsigned mask[2] = {0, 0};
 #pragma unroll
-            for (int tap = 0; tap < 9; tap++) {
-                const int y = ih + tap / 3, x = iw + tap % 3;
-                if (y >= 0 && y < a.in_h && x >= 0 && x < a.in_w) mask |= 1u << tap;
+        for (int h = 0; h < 2; h++) {
+            const int m = min(m0 + 8 * (2 * wave + h) + r8, a.M - 1);
+            if (a.taps == 9) {         // 3 x 3, stride 2, padding 1
+                const int ow = m % a.col_w, t = m / a.col_w, oh = t % a.col_h, c = t / a.col_h;
+                const int ih = 2 * oh - 1, iw = 2 * ow - 1;
+                pix[h] = (c * a.in_h + ih) * a.in_w + iw;
+#pragma unroll
+                for (int tap = 0; tap < 9; tap++) {
+                    const int y = ih + tap / 3, x = iw + tap % 3;
+                    if (y >= 0 && y < a.in_h && x >= 0 && x < a.in_w) mask[h] |= 1u << tap;
+                }
+            } else {                   // a token's column of in_h pixels, in_w apart
+                pix[h] = m / a.in_w * a.in_h * a.in_w + m % a.in_w;
+                mask[h] = 0xffffffffu;
             }
-        } else {                       // a token's column of in_h pixels, in_w apart
-            const int c = m / a.in_w;
-            pix = c * a.in_h * a.in_w + m % a.in_w;
-            mask = 0xffffffffu;
         }
+        // W rows (16 per group): those past N re-read row N - 1
         const uint16_t *w[LPW - 2];
 #pragma unroll
         for (int j = 0; j < LPW - 2; j++)
-            w[j] = a.W + (size_t)min(n0 + 16 * (wave + NW * j) + rr, a.N - 1) * a.K + kb + 8 * cl;
-        ring_walk<BM, 128, NST>(nk, lds, acc, [&](int kt, unsigned char *st) {
+            w[j] = a.W + (size_t)(kb / QK_GBK) * a.N * QK_GBK + (size_t)min(n0 + 16 * (wave + NW * j) + rr, a.N - 1) * QK_GBK +
+                   8 * cl;
+        const size_t wstep = (size_t)a.N * QK_GBK;
+        ring_walk<BM, 128, NST, true>(nk, lds, acc, [&](int kt, unsigned char *st) {
             // a 32-wide k tile lies in one tap
             const int k = kb + kt * QK_GBK, tap = k / QK_ENC_CH, ic = k - tap * QK_ENC_CH;
             const int off = a.taps == 9 ? (tap / 3) * a.in_w + tap % 3 : tap * a.in_w;
-            const uint16_t *p = (mask >> tap) & 1 ? a.A + (long)(pix + off) * (2 * QK_ENC_CH) : a.zero;
-            p += ic + 8 * cl;
-            lds_load16(p, st + 1024 * wave);
-            lds_load16(p + QK_ENC_CH, st + AB + 1024 * wave);
 #pragma unroll
-            for (int j = 0; j < LPW - 2; j++) lds_load16(w[j] + kt * QK_GBK, st + 2 * AB + 1024 * (wave + NW * j));
+            for (int h = 0; h < 2; h++) {
+                const uint16_t *p = (mask[h] >> tap) & 1 ? a.A + (long)(pix[h] + off) * (2 * QK_ENC_CH) + 2 * ic : a.zero;
+                lds_load16(p + 8 * c8, st + 1024 * (2 * wave + h));
+            }
+#pragma unroll
+            for (int j = 0; j < LPW - 2; j++) lds_load16(w[j] + kt * wstep, st + 2 * AB + 1024 * (wave + NW * j));
+        });
+    } else if constexpr (KG == 2) {
+        using R2 = RingShape2<BM, 128>;
+        const int r8 = lane >> 3, c8 = (lane & 7) ^ r8;
+        const uint16_t *src[R2::LPW2];
+#pragma unroll
+        for (int j = 0; j < R2::LPW2; j++) {
+            const int g = bwave + 2 * NW * j, ga = g < BM / 8 ? g : g - BM / 8;
+            src[j] = (g < BM / 4 ? a.A + (size_t)min(m0 + 8 * ga + r8, a.M - 1) * (2 * a.K) + (g < BM / 8 ? 0 : a.K)
+                                 : a.W + (size_t)min(n0 + 8 * (g - BM / 4) + r8, a.N - 1) * a.K) + kb + 8 * c8;
+        }
+        ring_walk2<BM, 128, NST>(nk / 2, lds, acc[0], [&](int p, unsigned char *st) {
+#pragma unroll
+            for (int j = 0; j < R2::LPW2; j++) lds_load16(src[j] + 64 * p, st + 1024 * (bwave + 2 * NW * j));
         });
     } else {
         const uint16_t *src[LPW];
@@ -661,7 +690,7 @@ __global__ __launch_bounds__(ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring
         });
     }
 
-    const int wm = wave / WGN, wn = wave % WGN, mr = m0 + wm * 32 + 4 * (lane >> 4);
+    const int wm = wave / WGN, wn = wave % WGN, mr = m0 + wm * 32 + 16 * kg + 4 * (lane >> 4);
     const bool odd = lane & 1;
     float bias[TN];
 #pragma unroll
@@ -669,13 +698,13 @@ __global__ __launch_bounds__(ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring
         const int n = n0 + wn * WTN + j * 16 + (lane & 15);
         bias[j] = EPI != ENC_PART && a.bias ? a.bias[min(n, a.N - 1)] : 0.0f;
     }
-    bool pad[2][4];
+    bool pad[NI][4];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < NI; i++)
 #pragma unroll
         for (int r = 0; r < 4; r++) pad[i][r] = GATHER && EPI == ENC_GELU && enc_ring_pad(a, mr + 16 * i + r);
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < NI; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
@@ -688,7 +717,7 @@ __global__ __launch_bounds__(ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring
     if constexpr (EPI == ENC_PART || EPI == ENC_F32) {
         float *y = EPI == ENC_PART ? a.ws + (size_t)blockIdx.z * a.M * a.N : a.C;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < NI; i++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
@@ -700,7 +729,7 @@ __global__ __launch_bounds__(ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring
         // columns n and n ^ 1 lie in neighbouring lanes (N is even): the even one
         // stores both hi halves, the odd one both lo halves
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < NI; i++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
@@ -710,7 +739,8 @@ __global__ __launch_bounds__(ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring
                     uint32_t h, l;
                     enc_split2(odd ? pv : v, odd ? v : pv, h, l);
                     if (m < a.M && n < a.N)
-                        *reinterpret_cast<uint32_t *>(a.out + (size_t)m * 2 * a.N + (odd ? a.N + n - 1 : n)) = odd ? l : h;
+                        *reinterpret_cast<uint32_t *>(a.out + (size_t)m * 2 * a.N + (GATHER ? n + (n & ~31) : n) +
+                                                      (odd ? (GATHER ? 32 : a.N) - 1 : 0)) = odd ? l : h;
                 }
     }
 }
@@ -726,7 +756,8 @@ __global__ __launch_bounds__(256) void enc_ring_reduce(qk_enc_ring_args a) {
         if (a.gelu) v = make_float4(enc_gelu(v.x), enc_gelu(v.y), enc_gelu(v.z), enc_gelu(v.w));
         if (enc_ring_pad(a, m)) v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (a.C) *reinterpret_cast<float4 *>(a.C + 4 * e) = v;
-        else enc_store_halves(a.out + (size_t)m * 2 * a.N, a.N, n, v);
+        else if (a.taps) enc_store_halves<true>(a.out + (size_t)m * 2 * a.N, a.N, n, v);
+        else enc_store_halves<false>(a.out + (size_t)m * 2 * a.N, a.N, n, v);
     }
 }
 
@@ -762,7 +793,7 @@ __global__ __launch_bounds__(256) void enc_ring_reduce_ln(qk_enc_ring_args a) {
     const float var = (red[1][0] + red[1][1] + red[1][2] + red[1][3]) / (float)a.N;
     const float inv = 1.0f / sqrtf(var + a.ln_eps);
     if (on)
-        enc_store_halves(a.out + (size_t)m * 2 * a.N, a.N, n,
+        enc_store_halves<false>(a.out + (size_t)m * 2 * a.N, a.N, n,
                          make_float4(dx * inv * w.x + b.x, dy * inv * w.y + b.y, dz * inv * w.z + b.z,
                                      dw * inv * w.w + b.w));
 }
@@ -778,13 +809,14 @@ extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, lon
     *bm = M <= 32 && !gather ? 32 : (long)((M + 127) / 128) * nt >= 256 ? 128 : 64;
     const long tiles = (M + *bm - 1) / *bm * nt;
     const int kt = K / QK_GBK;
-    long ns = (QK_ENC_RING_TARGET + tiles - 1) / tiles;
+    long ns = QK_ENC_RING_TARGET / tiles;
     if (fused && tiles >= QK_ENC_RING_FUSED) ns = 1;
     if (ns > QK_ENC_RING_SPLIT) ns = QK_ENC_RING_SPLIT;
     if (ns > kt / 4) ns = kt / 4;
     while (ns > 1 && ns * M * N > ws_elems) ns--;
     if (ns < 1) ns = 1;
-    const int per = (int)((kt + ns - 1) / ns);
+    int per = (int)((kt + ns - 1) / ns);
+    if (K % 64 == 0) per += per & 1;      // whole 64-deep stages
     *kc = per * QK_GBK;
     *split = (kt + per - 1) / per;
 }
@@ -803,15 +835,20 @@ extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_
     int bm;
     qk_enc_ring_plan(a->M, a->N, a->K, !ln, gather, ws ? ws_elems : 0, &bm, &g.kc, &g.split);
     g.ws = ln || g.split > 1 ? ws : nullptr;
-    const dim3 grid((a->N + 127) / 128, (a->M + bm - 1) / bm, g.split), block(64 * ring_waves(bm, 128));
+    const dim3 grid((a->N + 127) / 128, (a->M + bm - 1) / bm, g.split);
+    // launches of at most one block per CU: 64-deep stages, two k groups per block
+    const int kgs = bm < 128 && !gather && a->K % 64 == 0 && g.kc % 64 == 0 && (long)grid.x * grid.y * grid.z <= 256 ? 2 : 1;
     const int epi = g.ws ? ENC_PART : a->C ? ENC_F32 : ENC_GELU;
-#define QK_ENC_RING(BM_, NST_, G_, E_)                                     \
-    if (bm == BM_ && gather == G_ && epi == E_) enc_ring<BM_, NST_, G_, E_><<<grid, block, 0, s>>>(g);
-#define QK_ENC_RING_BM(BM_, NST_, G_) \
-    QK_ENC_RING(BM_, NST_, G_, ENC_PART) QK_ENC_RING(BM_, NST_, G_, ENC_GELU)
-    QK_ENC_RING_BM(128, 3, true) QK_ENC_RING_BM(64, 4, true)
-    QK_ENC_RING_BM(128, 3, false) QK_ENC_RING_BM(64, 4, false) QK_ENC_RING_BM(32, 4, false)
-    QK_ENC_RING(128, 3, false, ENC_F32) QK_ENC_RING(64, 4, false, ENC_F32) QK_ENC_RING(32, 4, false, ENC_F32)
+#define QK_ENC_RING(BM_, NST_, G_, E_, KG_)                               \
+    if (bm == BM_ && gather == G_ && epi == E_ && kgs == KG_)             \
+        enc_ring<BM_, NST_, G_, E_, KG_><<<grid, KG_ * 64 * ring_waves(BM_, 128), 0, s>>>(g);
+#define QK_ENC_RING_BM(BM_, NST_, G_, KG_) \
+    QK_ENC_RING(BM_, NST_, G_, ENC_PART, KG_) QK_ENC_RING(BM_, NST_, G_, ENC_GELU, KG_)
+    QK_ENC_RING_BM(128, 3, true, 1) QK_ENC_RING_BM(64, 4, true, 1)
+    QK_ENC_RING_BM(128, 3, false, 1) QK_ENC_RING_BM(64, 4, false, 1) QK_ENC_RING_BM(64, 4, false, 2)
+    QK_ENC_RING_BM(32, 4, false, 1) QK_ENC_RING_BM(32, 4, false, 2)
+    QK_ENC_RING(128, 3, false, ENC_F32, 1) QK_ENC_RING(64, 4, false, ENC_F32, 1)
+    QK_ENC_RING(64, 4, false, ENC_F32, 2) QK_ENC_RING(32, 4, false, ENC_F32, 1) QK_ENC_RING(32, 4, false, ENC_F32, 2)
 #undef QK_ENC_RING_BM
 #undef QK_ENC_RING
     if (ln) {
@@ -823,8 +860,7 @@ extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_
     return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
 }
 
-// conv1 (one input channel) from the mel [128][frames], as halves [pos][480 hi |
-// 480 lo]: a thread holds 4 channels' weights and walks positions, 9 mel values
+// conv1 (one input channel) from the mel [128][frames], as pixels of halves: a thread holds 4 channels' weights and walks positions, 9 mel values
 // (the same for the 120 threads of a position) and 36 multiply-adds each.
 // Bound by the 4 bytes written per output.
 __global__ __launch_bounds__(256) void enc_conv1_halves(const float *mel, int kpad, const float *w, const float *b,
@@ -855,7 +891,7 @@ __global__ __launch_bounds__(256) void enc_conv1_halves(const float *mel, int kp
         const bool pad = c == chunks - 1 && ow >= valid;
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = pad ? 0.0f : enc_gelu(v[j]);
-        enc_store_halves(out + (size_t)pos * 2 * QK_ENC_CH, QK_ENC_CH, c0, make_float4(v[0], v[1], v[2], v[3]));
+        enc_store_halves<true>(out + (size_t)pos * 2 * QK_ENC_CH, QK_ENC_CH, c0, make_float4(v[0], v[1], v[2], v[3]));
     }
 }
 
@@ -873,19 +909,19 @@ extern "C" int qk_enc_conv1_halves_launch(const float *mel, int kpad, const floa
     return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
 }
 
-// out[n][f ch + c] = in[n][c h + f]: conv_out's columns (channel, row) in the
-// order of a token's pixels (row, channel)
-__global__ __launch_bounds__(256) void enc_reorder(const uint16_t *in, uint16_t *out, int ch, int h, long n) {
+// Weights [rows][ch h] (column c h + f) as the gathering products read them: k =
+// f ch + c, [k / 32][row][k % 32].
+__global__ __launch_bounds__(256) void enc_tile_weights(const uint16_t *in, uint16_t *out, int rows, int ch, int h, long n) {
     const long e = blockIdx.x * 256L + threadIdx.x;
     if (e >= n) return;
-    const int K = ch * h, k = (int)(e % K), f = k / ch, c = k % ch;
-    out[e] = in[e - k + c * h + f];
+    const int row = (int)(e / 32 % rows), k = (int)(e / 32 / rows) * 32 + (int)(e % 32), f = k / ch, c = k % ch;
+    out[e] = in[(long)row * ch * h + c * h + f];
 }
 
-extern "C" int qk_enc_reorder_launch(const uint16_t *in, uint16_t *out, int rows, int ch, int h, hipStream_t s) {
+extern "C" int qk_enc_tile_weights_launch(const uint16_t *in, uint16_t *out, int rows, int ch, int h, hipStream_t s) {
     const long n = (long)rows * ch * h;
-    if (!in || !out || n <= 0) return QWEN_HIP_EINVAL;
-    enc_reorder<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(in, out, ch, h, n);
+    if (!in || !out || n <= 0 || (ch * h) % 32) return QWEN_HIP_EINVAL;
+    enc_tile_weights<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(in, out, rows, ch, h, n);
     return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
 }
 
@@ -1046,7 +1082,7 @@ __global__ __launch_bounds__(256) void enc_attention(const float *qkv, float *ou
     if (qi >= we) return;
     const float inv = 1.0f / L;
     const float4 v = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
-    if (out16) enc_store_halves(out16 + (size_t)qi * 2 * H * hd, H * hd, h * hd + d, v);
+    if (out16) enc_store_halves<false>(out16 + (size_t)qi * 2 * H * hd, H * hd, h * hd + d, v);
     else *reinterpret_cast<float4 *>(out + (long)qi * H * hd + h * hd + d) = v;
 }
 

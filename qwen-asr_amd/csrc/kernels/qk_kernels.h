@@ -415,10 +415,11 @@ int qk_enc_attention_launch(const float *qkv, float *out, uint16_t *out16, int T
 
 /* Products on bf16 weights with the activations kept as "halves": rows of 2 K
  * bf16, [K hi | K lo] (hi = bf16(x), lo = bf16(x - hi)).
- * A: rows of halves [M][2 K], or (taps > 0) stem pixels [..][2 * 480] halves from
- * which the rows are gathered, K = taps * 480 tap-major: taps 9 is a 3x3, stride
+ * A: rows of halves [M][2 K] and W [N][K], or (taps > 0) stem pixels, each 15 x
+ * [32 hi | 32 lo] channels, from which the rows are gathered, K = taps * 480
+ * tap-major, W [K / 32][N][32], out pixels too: taps 9 is a 3x3, stride
  * 2, pad 1 window over [chunk][in_h][in_w] pixels for row m = (chunk, oh, ow) of
- * col_h x col_w, with `zero` (2 * 480 zeros) outside; taps == in_h is pixel
+ * col_h x col_w, with `zero` (64 zeros) outside; taps == in_h is pixel
  * column m % in_w of chunk m / in_w, top to bottom.
  * Result, one of: C fp32 [M][N] (+ bias); out halves [M][2 N] of the GELU (bias
  * added before; valid > 0: row m's positions ow >= valid of the last chunk are 0); with
@@ -446,12 +447,13 @@ int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_elems, hipS
 /* tile rows, k per split and splits of such a product (fused: no reduce pass needed) */
 void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, long ws_elems, int *bm, int *kc, int *split);
 /* conv1 from the mel [h_in][mel_frames] (chunks of w_in frames) and weights
- * w[480][kpad] (9 taps) as halves [chunk][h_out][w_out][2 * 480], + bias, GELU,
+ * w[480][kpad] (9 taps) as pixels [chunk][h_out][w_out], + bias, GELU,
  * the last chunk's positions ow >= valid 0 */
 int qk_enc_conv1_halves_launch(const float *mel, int kpad, const float *w, const float *b, uint16_t *out, int chunks,
                                int h_in, int w_in, int h_out, int w_out, int mel_frames, int valid, hipStream_t s);
-/* out[n][f * ch + c] = in[n][c * h + f] */
-int qk_enc_reorder_launch(const uint16_t *in, uint16_t *out, int rows, int ch, int h, hipStream_t s);
+/* weights [rows][ch * h], column c * h + f, as a gathering product's W: k = f * ch
+ * + c, [k / 32][row][k % 32] (h 1: the columns keep their order) */
+int qk_enc_tile_weights_launch(const uint16_t *in, uint16_t *out, int rows, int ch, int h, hipStream_t s);
 
 /* ---- elementwise (op-level ABI) --------------------------------------- */
 int qk_add_launch(float *a, const float *b, long n, hipStream_t s);

@@ -47,7 +47,9 @@ struct RingShape {
 // bytes, k chunk c of row r in slot c ^ ((r / 2) % 4).  Wave (wm, wn) = (wave /
 // WGN, wave % WGN) ends up with rows 32 wm + 16 i + 4 (l >> 4) + r, columns WTN
 // wn + 16 j + (l & 15) of the tile (lane l, acc[i][j][r]).
-template <int BM, int BN, int NST, typename ISSUE>
+// PAIRED: A rows of 128 bytes, 32 hi then 32 lo values (whole cache lines), chunk c
+// of row r in slot c ^ (r % 8).
+template <int BM, int BN, int NST, bool PAIRED = false, typename ISSUE>
 __device__ __forceinline__ void ring_walk(int nk, unsigned char *lds, f32x4 (&acc)[2][RingShape<BM, BN>::TN],
                                           ISSUE issue) {
     using RS = RingShape<BM, BN>;
@@ -65,6 +67,7 @@ __device__ __forceinline__ void ring_walk(int nk, unsigned char *lds, f32x4 (&ac
 
     const int fr = lane & 15;
     const int fo = fr * 64 + 16 * ((lane >> 4) ^ ((fr >> 1) & 3));
+    const int fp = fr * 128 + 16 * ((lane >> 4) ^ (fr & 7));
     for (int t = 0; t < NST - 1 && t < nk; t++) issue(t, lds + t * STAGE);
     for (int kt = 0; kt < nk; kt++) {
         ring_wait<LPW, NST - 2>(min(nk - 1 - kt, NST - 2));
@@ -79,7 +82,67 @@ __device__ __forceinline__ void ring_walk(int nk, unsigned char *lds, f32x4 (&ac
             bfr[j] = *reinterpret_cast<const bf16x8 *>(st + 2 * AB + (wn * WTN + j * 16) * 64 + fo);
 #pragma unroll
         for (int i = 0; i < TM; i++) {
-            const int ro = (wm * 32 + i * 16) * 64 + fo;
+            const int ro = (wm * 32 + i * 16) * (PAIRED ? 128 : 64) + (PAIRED ? fp : fo);
+            const bf16x8 ah = *reinterpret_cast<const bf16x8 *>(st + ro);
+            const bf16x8 al = *reinterpret_cast<const bf16x8 *>(st + (PAIRED ? ro ^ 64 : AB + ro));
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bfr[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bfr[j], acc[i][j], 0, 0, 0);
+        }
+    }
+}
+
+// The walk for launches of about one block per CU and K a multiple of 64: stages
+// of 64 k, rows of 128 bytes, and 2 NW waves, group kg = wave / NW multiplying k
+// 32 kg .. + 32 of every stage.  With 64-byte rows a load takes half of each
+// cache line and the other half is fetched again a k tile later, which bounds
+// the loads of a CU (1200 cycles per 64 k of a 64 x 128 tile, 600 of them MFMAs,
+// whether the data is in L2 or not); whole lines halve that, and the two waves
+// of a SIMD overlap one's fragment reads with the other's MFMAs.  @WALK2@
+// issue(p, st): this wave's LPW2 1 KB loads (8 rows of 128 bytes) of stage p;
+// chunk c of row r in slot c ^ (r % 8).  The groups' sums are added at the end
+// (group 0's + group 1's), each group finishing one 16-row tile: fin[j][r] is
+// row 32 wm + 16 kg + 4 (l >> 4) + r, column WTN wn + 16 j + (l & 15).
+template <int BM, int BN>
+struct RingShape2 : RingShape<BM, BN> {
+    static constexpr int AB2 = BM * 128, STAGE2 = 2 * AB2 + BN * 128;
+    static constexpr int GROUPS2 = (2 * BM + BN) / 8, LPW2 = GROUPS2 / (2 * RingShape<BM, BN>::NW);
+    static_assert(GROUPS2 % (2 * RingShape<BM, BN>::NW) == 0, "load split");
+};
+
+template <int BM, int BN, int NST, typename ISSUE>
+__device__ __forceinline__ void ring_walk2(int np, unsigned char *lds, f32x4 (&fin)[RingShape<BM, BN>::TN],
+                                           ISSUE issue) {
+    using RS = RingShape2<BM, BN>;
+    constexpr int NW = RS::NW, WGN = RS::WGN, WTN = RS::WTN, TM = RS::TM, TN = RS::TN;
+    constexpr int AB = RS::AB2, STAGE = RS::STAGE2, LPW = RS::LPW2;
+    static_assert((NST - 2) * LPW <= 63 && NST * STAGE <= 160 * 1024, "vmcnt / LDS range");
+    static_assert(2 * NW * TN * 64 * 16 <= NST * STAGE, "exchange fits the stages");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = wave / NW, wi = wave % NW, wm = wi / WGN, wn = wi % WGN;
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    const int fr = lane & 15;
+    const int fo = fr * 128 + 16 * ((4 * kg + (lane >> 4)) ^ (fr & 7));
+    for (int t = 0; t < NST - 1 && t < np; t++) issue(t, lds + t * STAGE);
+    for (int p = 0; p < np; p++) {
+        ring_wait<LPW, NST - 2>(min(np - 1 - p, NST - 2));
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (p + NST - 1 < np) issue(p + NST - 1, lds + ((p + NST - 1) % NST) * STAGE);
+        const unsigned char *st = lds + (p % NST) * STAGE;
+        bf16x8 bfr[TN];
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+            bfr[j] = *reinterpret_cast<const bf16x8 *>(st + 2 * AB + (wn * WTN + j * 16) * 128 + fo);
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            const int ro = (wm * 32 + i * 16) * 128 + fo;
             const bf16x8 ah = *reinterpret_cast<const bf16x8 *>(st + ro);
             const bf16x8 al = *reinterpret_cast<const bf16x8 *>(st + AB + ro);
 #pragma unroll
@@ -88,6 +151,16 @@ __device__ __forceinline__ void ring_walk(int nk, unsigned char *lds, f32x4 (&ac
             for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bfr[j], acc[i][j], 0, 0, 0);
         }
     }
+    __syncthreads();                                           // the stages are free
+    f32x4 *x = reinterpret_cast<f32x4 *>(lds);
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        fin[j] = kg ? acc[1][j] : acc[0][j];
+        x[(wave * TN + j) * 64 + lane] = kg ? acc[0][j] : acc[1][j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < TN; j++) fin[j] += x[(((1 - kg) * NW + wi) * TN + j) * 64 + lane];
 }
 
 // The k walk of block (blockIdx.x, blockIdx.y, blockIdx.z) of a plain product
