@@ -561,13 +561,15 @@ extern "C" int qk_enc_stem_rows_launch(const float *c3, float *rows, int chunks,
 // pixels hold their 480 channels as 15 times [32 hi | 32 lo], and the weights of
 // the products that gather them lie as [K / 32][N][32]: a 32-deep k tile then
 // reads whole 128-byte lines (with half lines the load path bounded these
-// products: @CONV@).
+// products: conv2 of 743 frames 102 -> 75 us, conv_out of 3000 41 -> 29; on
+// enc_gemm_hl they took 172 and ~45).
 // Weights of other than bf16 values, or widths that are no multiple of 128,
 // run on enc_gemm_hl / enc_gemm above.
 //
 // What bounds it: at 100 to 400 rows these products are a few microseconds
-// each, mostly ramp, latency of the k walk and drain; a k tile staged through
-// registers (one in flight) took ~2x a ring step.  @RINGM@
+// each, mostly ramp, the k walk's load path and drain; a k tile staged through
+// registers (one in flight) took ~2x a ring step.  390 rows, 896 wide: Q|K|V 13.7 +
+// 6.6 us of reduce -> 12.8, fc1 17.7 + 7.5 -> 13.5, fc2 17.5 + 7.5 -> 14.2 + 4.4.
 // ---------------------------------------------------------------------------
 typedef float ec_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 ec_bf16x2 __attribute__((ext_vector_type(2)));
@@ -605,7 +607,7 @@ enum { ENC_PART, ENC_F32, ENC_GELU };
 // One tile of the product; GATHER: rows of A are gathered from stem pixels.  The
 // epilogue is chosen at compile time: with tests between the 32 values of a lane
 // their chains ran one after the other, 9.3 us of a 390 x 3584 x 896 GELU
-// product's 20 against @EPI@.
+// product's 20 against 1.9 of its 12 now.
 template <int BM, int NST, bool GATHER, int EPI, int KG>
 __global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring_args a) {
     using RS = RingShape<BM, 128>;
@@ -799,10 +801,12 @@ __global__ __launch_bounds__(256) void enc_ring_reduce_ln(qk_enc_ring_args a) {
 }
 
 // Tile height and split of an M x N x K product.  64-row tiles (32 up to 32
-// rows; 128 where those alone give every CU a block).  K is split until the
-// launch has about QK_ENC_RING_TARGET blocks, k walks of 4 k tiles at least; a
-// product whose epilogue needs no reduce pass (`fused`) is only split where
-// its tiles would leave most CUs idle.
+// rows; 128 where those alone give every CU a block).  K is split while the launch
+// stays within QK_ENC_RING_TARGET blocks, one per CU (fc2 at 390 rows: 294 blocks
+// in six splits 18.2 us, 245 in five 14.2), k walks of 4 k tiles at least.  A
+// product whose epilogue needs no reduce pass (`fused`) and walks up to
+// QK_ENC_RING_FUSED k tiles is not cut in two: that saves 3.5 us, the reduce takes
+// 4.5 (in five, 97 x 3072 x 1024: 7.6 + 4.5 us against 13.4 unsplit).
 extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, long ws_elems, int *bm, int *kc,
                                  int *split) {
     const long nt = (N + 127) / 128;
@@ -810,7 +814,7 @@ extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, lon
     const long tiles = (M + *bm - 1) / *bm * nt;
     const int kt = K / QK_GBK;
     long ns = QK_ENC_RING_TARGET / tiles;
-    if (fused && tiles >= QK_ENC_RING_FUSED) ns = 1;
+    if (fused && ns <= 2 && kt <= QK_ENC_RING_FUSED) ns = 1;
     if (ns > QK_ENC_RING_SPLIT) ns = QK_ENC_RING_SPLIT;
     if (ns > kt / 4) ns = kt / 4;
     while (ns > 1 && ns * M * N > ws_elems) ns--;
@@ -860,16 +864,20 @@ extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_
     return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
 }
 
-// conv1 (one input channel) from the mel [128][frames], as pixels of halves: a thread holds 4 channels' weights and walks positions, 9 mel values
-// (the same for the 120 threads of a position) and 36 multiply-adds each.
-// Bound by the 4 bytes written per output.
+// conv1 (one input channel) from the mel [128][frames], as pixels of halves: a
+// thread holds 4 channels' weights and walks units of C1_OW consecutive output
+// positions of a row: 3 x (2 C1_OW + 1) mel values (the same for the 120 threads of
+// a unit), then 36 multiply-adds, 4 GELUs and a split per position.  Bound by
+// those operations and the 4 bytes written per output (46 M outputs of 30 s: 74 us;
+// one position at a time, twice the index work, 94).
+#define C1_OW 5
 __global__ __launch_bounds__(256) void enc_conv1_halves(const float *mel, int kpad, const float *w, const float *b,
-                                                        uint16_t *out, int rows, int h_in, int w_in, int h_out,
+                                                        uint16_t *out, int units, int h_in, int w_in, int h_out,
                                                         int w_out, int mel_frames, int chunks, int valid) {
-    constexpr int q4 = QK_ENC_CH / 4;
+    constexpr int q4 = QK_ENC_CH / 4, NC = 2 * C1_OW + 1;
     // the grid stride is a multiple of q4: a thread keeps one channel quad
     const long i0 = blockIdx.x * 256L + threadIdx.x, stride = (long)gridDim.x * 256;
-    const int c0 = 4 * (int)(i0 % q4), dpos = (int)(stride / q4);
+    const int c0 = 4 * (int)(i0 % q4), du = (int)(stride / q4), upr = (w_out + C1_OW - 1) / C1_OW;
     float wr[4][9], br[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -877,28 +885,40 @@ __global__ __launch_bounds__(256) void enc_conv1_halves(const float *mel, int kp
 #pragma unroll
         for (int t = 0; t < 9; t++) wr[j][t] = w[(c0 + j) * kpad + t];
     }
-    for (int pos = (int)(i0 / q4); pos < rows; pos += dpos) {
-        const int ow = pos % w_out, t1 = pos / w_out, oh = t1 % h_out, c = t1 / h_out;
-        float v[4] = {br[0], br[1], br[2], br[3]};
+    for (int u = (int)(i0 / q4); u < units; u += du) {
+        const int ow0 = u % upr * C1_OW, t1 = u / upr, oh = t1 % h_out, c = t1 / h_out;
+        float x[3][NC];
 #pragma unroll
-        for (int t = 0; t < 9; t++) {
-            const int ih = 2 * oh - 1 + t / 3, iw = 2 * ow - 1 + t % 3, f = c * w_in + iw;
-            const bool in = ih >= 0 && ih < h_in && iw >= 0 && iw < w_in && f < mel_frames;
-            const float x = in ? mel[(long)ih * mel_frames + f] : 0.0f;
+        for (int y = 0; y < 3; y++) {
+            const int ih = 2 * oh - 1 + y;
+            const float *row = mel + (long)min(max(ih, 0), h_in - 1) * mel_frames;
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = fmaf(x, wr[j][t], v[j]);
+            for (int k = 0; k < NC; k++) {
+                const int iw = 2 * ow0 - 1 + k, f = c * w_in + iw;
+                const bool in = ih >= 0 && ih < h_in && iw >= 0 && iw < w_in && f < mel_frames;
+                x[y][k] = in ? row[f] : 0.0f;
+            }
         }
-        const bool pad = c == chunks - 1 && ow >= valid;
+        uint16_t *o = out + ((size_t)t1 * w_out + ow0) * 2 * QK_ENC_CH;
+        const int n = min(C1_OW, w_out - ow0), nv = c == chunks - 1 ? valid - ow0 : C1_OW;
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = pad ? 0.0f : enc_gelu(v[j]);
-        enc_store_halves<true>(out + (size_t)pos * 2 * QK_ENC_CH, QK_ENC_CH, c0, make_float4(v[0], v[1], v[2], v[3]));
+        for (int p = 0; p < C1_OW; p++) {
+            float v[4] = {br[0], br[1], br[2], br[3]};
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = fmaf(x[t / 3][2 * p + t % 3], wr[j][t], v[j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = p < nv ? enc_gelu(v[j]) : 0.0f;
+            if (p < n) enc_store_halves<true>(o + p * 2 * QK_ENC_CH, QK_ENC_CH, c0, make_float4(v[0], v[1], v[2], v[3]));
+        }
     }
 }
 
 extern "C" int qk_enc_conv1_halves_launch(const float *mel, int kpad, const float *w, const float *b, uint16_t *out,
                                           int chunks, int h_in, int w_in, int h_out, int w_out, int mel_frames,
                                           int valid, hipStream_t s) {
-    const long rows = (long)chunks * h_out * w_out;
+    const long rows = (long)chunks * h_out * ((w_out + C1_OW - 1) / C1_OW);
     if (!mel || !w || !b || !out || kpad < 9 || rows <= 0 || rows > 0x7fffffffL || mel_frames <= 0) return QWEN_HIP_EINVAL;
     constexpr int unit = 15;           // blocks: a multiple of 15, so the grid stride is one of 120 (256 * 15 = 32 * 120)
     long blocks = (rows * (QK_ENC_CH / 4) + 255) / 256;
@@ -973,7 +993,7 @@ extern "C" int qk_enc_layernorm_launch(const float *x, const float *w, const flo
 // consecutive dims.  Online softmax per wave; the waves' (m, l, o) meet in LDS.
 // Bound by latency (104 keys a window: one round of 16 independent 16-byte
 // loads per lane, then 64 MFMAs): a window walked by one wave in blocks of 64
-// keys with 4-byte V loads took @ATT@.
+// keys with 4-byte V loads took 12.6 us at 390 tokens x 14 heads, this 7.5.
 // The result goes out as fp32 or, for the bf16 products, as halves.
 // ---------------------------------------------------------------------------
 #define EA_Q 16

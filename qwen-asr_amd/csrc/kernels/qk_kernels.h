@@ -428,7 +428,7 @@ int qk_enc_attention_launch(const float *qkv, float *out, uint16_t *out16, int T
  * least M N floats).  kc, split and ws of the struct are set by the launcher. */
 #define QK_ENC_CH 480             /* channels of the stem, QWEN_CONV_HIDDEN (qwen_asr.h:39) */
 #define QK_ENC_RING_TARGET 256    /* blocks a split launch aims for */
-#define QK_ENC_RING_FUSED 96      /* tiles from which a product without a reduce pass is not split */
+#define QK_ENC_RING_FUSED 32      /* k tiles up to which a product without a reduce pass is not split */
 #define QK_ENC_RING_SPLIT 8       /* at most */
 typedef struct {
     const uint16_t *A, *W, *zero;

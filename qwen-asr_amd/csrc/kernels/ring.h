@@ -99,7 +99,8 @@ __device__ __forceinline__ void ring_walk(int nk, unsigned char *lds, f32x4 (&ac
 // cache line and the other half is fetched again a k tile later, which bounds
 // the loads of a CU (1200 cycles per 64 k of a 64 x 128 tile, 600 of them MFMAs,
 // whether the data is in L2 or not); whole lines halve that, and the two waves
-// of a SIMD overlap one's fragment reads with the other's MFMAs.  @WALK2@
+// of a SIMD overlap one's fragment reads with the other's MFMAs.  Measured,
+// k walk of a 390 x 3584 x 896 product, one block per CU: 9.4 us plain, 8.0.
 // issue(p, st): this wave's LPW2 1 KB loads (8 rows of 128 bytes) of stage p;
 // chunk c of row r in slot c ^ (r % 8).  The groups' sums are added at the end
 // (group 0's + group 1's), each group finishing one 16-row tile: fin[j][r] is

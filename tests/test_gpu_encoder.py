@@ -187,3 +187,132 @@ def test_encoder_fp32_weights_take_the_fp32_gemm(P, qa, gpu):
     err = np.abs(out - ref)
     assert np.all(err <= ATOL + RTOL * np.abs(ref)), float(err.max())
     e.close()
+
+
+class RingArgs(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("A", "W", "zero")] + [(n, C.c_int) for n in (
+        "M", "N", "K", "taps", "in_h", "in_w", "col_h", "col_w", "chunks", "valid")] + [
+        ("bias", C.c_void_p), ("pe", C.c_void_p), ("pe_rows", C.c_int), ("gelu", C.c_int), ("add", C.c_int),
+        ("C", C.c_void_p), ("out", C.c_void_p), ("ln_w", C.c_void_p), ("ln_b", C.c_void_p), ("ln_eps", C.c_float),
+        ("ws", C.c_void_p), ("kc", C.c_int), ("split", C.c_int)]
+
+
+def halves(gpu, x, pixel=False):
+    """fp32 [M][K] -> rows [K hi | K lo], or pixels K / 32 x [32 hi | 32 lo], and the value they carry"""
+    hi = x.bfloat16()
+    lo = (x - hi.float()).bfloat16()
+    M, K = x.shape
+    t = gpu.stack([hi.view(M, K // 32, 32), lo.view(M, K // 32, 32)], 2) if pixel else gpu.cat([hi, lo], 1)
+    return t.reshape(M, 2 * K).contiguous(), hi.double() + lo.double()
+
+
+def unhalve(gpu, t, N, pixel=False):
+    t = t.double()
+    return (t.view(-1, N // 32, 2, 32).sum(2).reshape(-1, N) if pixel else t[:, :N] + t[:, N:])
+
+
+def gelu64(gpu, v):
+    return 0.5 * v * (1 + gpu.tanh(0.7978845608028654 * (v + 0.044715 * v ** 3)))
+
+
+# 32-, 64- and 128-row tiles; one and two k groups; split and unsplit; ragged
+# rows, columns and k walks (K 96: no whole 64-deep stages)
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (32, 96, 64), (33, 192, 96), (97, 1024, 1024), (390, 896, 3584),
+                                   (65, 4096, 896), (1600, 3072, 128), (4100, 1024, 64)])
+@pytest.mark.parametrize("what", ["f32", "gelu", "ln"])
+def test_ring_products(P, qa, gpu, M, N, K, what):
+    """qk_enc_ring_launch on rows of halves against a float64 product of the
+    same halves: fp32 accumulation leaves 4 K 2^-24 sum |x w|, halves of the
+    result 2^-16 relative."""
+    lib = qa.lib()
+    lib.qk_enc_ring_launch.argtypes = [C.c_void_p, C.c_void_p, C.c_long, C.c_void_p]
+    g = gpu.Generator(device="cuda").manual_seed(M + N)
+    r = lambda *s: gpu.randn(*s, generator=g, device="cuda")
+    x, W = r(M, K), (r(N, K) * 0.05).bfloat16()
+    A, xv = halves(gpu, x)
+    bias, x0 = r(N), r(M, N)
+    ws = gpu.empty(max(8 * 64 * 64 * 1024, M * N), device="cuda")
+    f, out = x0.clone(), gpu.zeros(M, 2 * N, dtype=gpu.bfloat16, device="cuda")
+    a = RingArgs(A=A.data_ptr(), W=W.data_ptr(), M=M, N=N, K=K, bias=bias.data_ptr())
+    if what == "f32":
+        a.C = f.data_ptr()
+    elif what == "gelu":
+        a.out, a.gelu = out.data_ptr(), 1
+    else:
+        w, b = 1 + 0.1 * r(N), r(N)
+        a.C, a.out, a.add, a.ln_w, a.ln_b, a.ln_eps = f.data_ptr(), out.data_ptr(), 1, w.data_ptr(), b.data_ptr(), 1e-5
+    if what == "ln" and N > 1024:
+        assert lib.qk_enc_ring_launch(C.byref(a), ws.data_ptr(), ws.numel(), None) == -1
+        return
+    qa.check(lib.qk_enc_ring_launch(C.byref(a), ws.data_ptr(), ws.numel(), None), "ring")
+    gpu.cuda.synchronize()
+    y = xv @ W.double().t().contiguous() + bias.double()
+    bound = 4 * K * 2.0 ** -24 * (xv.abs() @ W.double().abs().t().contiguous()) + 1e-6
+    if what == "f32":
+        assert bool(((f.double() - y).abs() <= bound).all())
+    elif what == "gelu":
+        got = unhalve(gpu, out, N)
+        ref = gelu64(gpu, y)
+        assert bool(((got - ref).abs() <= 1.2 * bound + 2.0 ** -16 * ref.abs() + 2.0 ** -22 * y.abs()).all())
+    else:
+        y = y + x0.double()
+        assert bool(((f.double() - y).abs() <= bound + 2.0 ** -22 * y.abs()).all())
+        fd = f.double()
+        ref = (fd - fd.mean(1, keepdim=True)) / gpu.sqrt(fd.var(1, unbiased=False, keepdim=True) + 1e-5) * w + b
+        assert float((unhalve(gpu, out, N) - ref).abs().max()) < 2e-4      # 2^-16 of values up to ~8
+
+
+@pytest.mark.parametrize("chunks,h,w,valid", [(1, 8, 5, 3), (3, 32, 25, 1), (9, 32, 50, 25), (2, 4, 1, 1)])
+def test_ring_convolution(P, qa, gpu, chunks, h, w, valid):
+    """The gathered 3x3 / stride 2 / padding 1 convolution with GELU, weights
+    through qk_enc_tile_weights_launch, and the last chunk's padding zeroed,
+    against float64 on the same halves."""
+    lib, CH = qa.lib(), 480
+    lib.qk_enc_ring_launch.argtypes = [C.c_void_p, C.c_void_p, C.c_long, C.c_void_p]
+    lib.qk_enc_tile_weights_launch.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p]
+    g = gpu.Generator(device="cuda").manual_seed(h * w)
+    x = gpu.randn(chunks * h * w, CH, generator=g, device="cuda")
+    W = (gpu.randn(CH, 9 * CH, generator=g, device="cuda") * 0.02).bfloat16()      # [n][tap][channel]
+    Wt, zero = gpu.empty_like(W), gpu.zeros(64, dtype=gpu.bfloat16, device="cuda")
+    qa.check(lib.qk_enc_tile_weights_launch(W.data_ptr(), Wt.data_ptr(), CH, 9 * CH, 1, None), "tile")
+    A, xv = halves(gpu, x, pixel=True)
+    ho, wo = (h + 1) // 2, (w + 1) // 2
+    M = chunks * ho * wo
+    bias = gpu.randn(CH, generator=g, device="cuda")
+    out = gpu.full((M, 2 * CH), 7.0, dtype=gpu.bfloat16, device="cuda")
+    ws = gpu.empty(8 * M * CH, device="cuda")
+    a = RingArgs(A=A.data_ptr(), W=Wt.data_ptr(), zero=zero.data_ptr(), M=M, N=CH, K=9 * CH, taps=9, in_h=h, in_w=w,
+                 col_h=ho, col_w=wo, chunks=chunks, valid=valid, bias=bias.data_ptr(), gelu=1, out=out.data_ptr())
+    qa.check(lib.qk_enc_ring_launch(C.byref(a), ws.data_ptr(), ws.numel(), None), "ring")
+    gpu.cuda.synchronize()
+    im = gpu.nn.functional.pad(xv.view(chunks, h, w, CH), (0, 0, 1, 2, 1, 2))
+    cols = gpu.cat([im[:, i:i + 2 * ho - 1:2, j:j + 2 * wo - 1:2] for i in range(3) for j in range(3)], -1).reshape(M, -1)
+    y = cols @ W.double().t().contiguous() + bias.double()
+    bound = 4 * 9 * CH * 2.0 ** -24 * (cols.abs() @ W.double().abs().t().contiguous()) + 1e-6
+    ref = gelu64(gpu, y).view(chunks, ho, wo, CH)
+    ref[-1, :, valid:] = 0
+    ref = ref.view(M, CH)
+    got = unhalve(gpu, out, CH, pixel=True)
+    assert bool(((got - ref).abs() <= 1.2 * bound + 2.0 ** -16 * ref.abs() + 2.0 ** -22 * y.abs()).all())
+
+
+# windows of one and several rounds of the four waves' 128 keys; ragged last
+# windows of one key, and a window longer than the sequence
+@pytest.mark.parametrize("T,win", [(1, 104), (97, 104), (209, 104), (33, 16), (300, 150), (401, 400), (130, 1000)])
+def test_window_attention(P, qa, gpu, T, win):
+    lib, H = qa.lib(), 3
+    lib.qk_enc_attention_launch.argtypes = [C.c_void_p] * 3 + [C.c_int] * 4 + [C.c_float, C.c_void_p]
+    g = gpu.Generator(device="cuda").manual_seed(T)
+    qkv = gpu.randn(T, 3, H, 64, generator=g, device="cuda")
+    out, out16 = gpu.empty(T, H * 64, device="cuda"), gpu.empty(T, 2 * H * 64, dtype=gpu.bfloat16, device="cuda")
+    qa.check(lib.qk_enc_attention_launch(qkv.data_ptr(), out.data_ptr(), None, T, H, 64, win, 0.125, None), "attn")
+    qa.check(lib.qk_enc_attention_launch(qkv.data_ptr(), None, out16.data_ptr(), T, H, 64, win, 0.125, None), "attn")
+    gpu.cuda.synchronize()
+    ref = gpu.empty(T, H, 64, dtype=gpu.float64, device="cuda")
+    for t0 in range(0, T, win):
+        q, k, v = (qkv[t0:t0 + win, i].double().transpose(0, 1).contiguous() for i in range(3))
+        p = gpu.softmax(gpu.bmm(q, k.transpose(1, 2).contiguous()) * 0.125, -1)
+        ref[t0:t0 + win] = gpu.bmm(p, v).transpose(0, 1)
+    ref = ref.view(T, H * 64)
+    assert float((out.double() - ref).abs().max()) < 1e-5                # fp32 products and sums
+    assert bool(((unhalve(gpu, out16, H * 64) - out.double()).abs() <= 2.0 ** -16 * out.double().abs() + 1e-9).all())
