@@ -55,31 +55,17 @@
 #define PF_VLDB PF_KT                     // bf16 row stride of the V^T tiles: 64 B, swizzled chunks
 #define PF_MINIT (-1.0e30f)       // running-max start, as the reference's -1e30 (:1069)
 
-typedef float pf_f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 pf_bf16x2 __attribute__((ext_vector_type(2)));
-
-// two bf16 (round to nearest even) in one word: one v_cvt_pk_bf16_f32
-__device__ __forceinline__ uint32_t pf_pack(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((pf_f32x2){a, b}, pf_bf16x2));
-}
-
-// x = hi + lo + O(2^-17 |x|), hi and lo bf16, two values per word
-__device__ __forceinline__ void pf_split2(float a, float b, uint32_t &hi, uint32_t &lo) {
-    hi = pf_pack(a, b);
-    lo = pf_pack(a - bf16_lo(hi), b - bf16_hi(hi));
-}
-
 __device__ __forceinline__ void pf_split4(float4 v, uint2 &h, uint2 &l) {
-    pf_split2(v.x, v.y, h.x, l.x);
-    pf_split2(v.z, v.w, h.y, l.y);
+    bf16_split2(v.x, v.y, h.x, l.x);
+    bf16_split2(v.z, v.w, h.y, l.y);
 }
 
 __device__ __forceinline__ void pf_split8(const float *x, bf16x8 &hi, bf16x8 &lo) {
     uint4 h, l;
-    pf_split2(x[0], x[1], h.x, l.x);
-    pf_split2(x[2], x[3], h.y, l.y);
-    pf_split2(x[4], x[5], h.z, l.z);
-    pf_split2(x[6], x[7], h.w, l.w);
+    bf16_split2(x[0], x[1], h.x, l.x);
+    bf16_split2(x[2], x[3], h.y, l.y);
+    bf16_split2(x[4], x[5], h.z, l.z);
+    bf16_split2(x[6], x[7], h.w, l.w);
     hi = __builtin_bit_cast(bf16x8, h);
     lo = __builtin_bit_cast(bf16x8, l);
 }

@@ -21,6 +21,19 @@ __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
     return (uint16_t)(b >> 16);
 }
 
+// Two values rounded to nearest even in one word (a low): one v_cvt_pk_bf16_f32.
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t bf16_pack2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, bf16x2_t));
+}
+
+// x = hi + lo + O(2^-17 |x|), both bf16: the words of two values
+__device__ __forceinline__ void bf16_split2(float a, float b, uint32_t &hi, uint32_t &lo) {
+    hi = bf16_pack2(a, b);
+    lo = bf16_pack2(a - bf16_lo(hi), b - bf16_hi(hi));
+}
+
 // Dot of 8 bf16 weights (one 16-byte load) with 8 fp32 activations.
 __device__ __forceinline__ float dot8_bf16(uint4 w, const float *x, float acc) {
     acc = fmaf(bf16_lo(w.x), x[0], acc);

@@ -571,24 +571,12 @@ extern "C" int qk_enc_stem_rows_launch(const float *c3, float *rows, int chunks,
 // registers (one in flight) took ~2x a ring step.  390 rows, 896 wide: Q|K|V 13.7 +
 // 6.6 us of reduce -> 12.8, fc1 17.7 + 7.5 -> 13.5, fc2 17.5 + 7.5 -> 14.2 + 4.4.
 // ---------------------------------------------------------------------------
-typedef float ec_f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 ec_bf16x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t enc_pack(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((ec_f32x2){a, b}, ec_bf16x2));
-}
-
-__device__ __forceinline__ void enc_split2(float a, float b, uint32_t &hi, uint32_t &lo) {
-    hi = enc_pack(a, b);
-    lo = enc_pack(a - bf16_lo(hi), b - bf16_hi(hi));
-}
-
 // four values at columns n .. n + 3 of a row of n_cols, or (PIXEL) of a stem pixel
 template <bool PIXEL>
 __device__ __forceinline__ void enc_store_halves(uint16_t *row, int n_cols, int n, float4 v) {
     uint2 h, l;
-    enc_split2(v.x, v.y, h.x, l.x);
-    enc_split2(v.z, v.w, h.y, l.y);
+    bf16_split2(v.x, v.y, h.x, l.x);
+    bf16_split2(v.z, v.w, h.y, l.y);
     row += PIXEL ? n + (n & ~31) : n;
     *reinterpret_cast<uint2 *>(row) = h;
     *reinterpret_cast<uint2 *>(row + (PIXEL ? 32 : n_cols)) = l;
@@ -739,7 +727,7 @@ __global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_
                     const int m = mr + 16 * i + r, n = n0 + wn * WTN + j * 16 + (lane & 15);
                     const float v = acc[i][j][r], pv = dpp_read<0xB1>(v);
                     uint32_t h, l;
-                    enc_split2(odd ? pv : v, odd ? v : pv, h, l);
+                    bf16_split2(odd ? pv : v, odd ? v : pv, h, l);
                     if (m < a.M && n < a.N)
                         *reinterpret_cast<uint32_t *>(a.out + (size_t)m * 2 * a.N + (GATHER ? n + (n & ~31) : n) +
                                                       (odd ? (GATHER ? 32 : a.N) - 1 : 0)) = odd ? l : h;

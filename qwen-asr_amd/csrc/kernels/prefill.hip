@@ -145,11 +145,14 @@ __global__ __launch_bounds__(256) void rmsnorm_split_rows(float *x, const float 
     for (int j = 0; j < Q; j++) {
         const float4 ww = wv[j];
         const float e[4] = {v[j].x, v[j].y, v[j].z, v[j].w}, we[4] = {ww.x, ww.y, ww.z, ww.w};
-        uint16_t hh[4], ll[4];
+        float x4[4];
+        uint2 hh, ll;
 #pragma unroll
-        for (int k = 0; k < 4; k++) split2(w ? (e[k] * we[k]) * rinv : e[k], hh[k], ll[k]);
-        h[64 * j] = make_uint2(hh[0] | ((unsigned)hh[1] << 16), hh[2] | ((unsigned)hh[3] << 16));
-        l[64 * j] = make_uint2(ll[0] | ((unsigned)ll[1] << 16), ll[2] | ((unsigned)ll[3] << 16));
+        for (int k = 0; k < 4; k++) x4[k] = w ? (e[k] * we[k]) * rinv : e[k];
+        bf16_split2(x4[0], x4[1], hh.x, ll.x);
+        bf16_split2(x4[2], x4[3], hh.y, ll.y);
+        h[64 * j] = hh;
+        l[64 * j] = ll;
     }
 }
 
@@ -249,11 +252,14 @@ __global__ __launch_bounds__(256) void rmsnorm_split_vec(float *x, const float *
     for (int e = 0; e < V4; e++) {
         const float4 ww = wv[e];
         const float el[4] = {v[e].x, v[e].y, v[e].z, v[e].w}, we[4] = {ww.x, ww.y, ww.z, ww.w};
-        uint16_t hh[4], ll[4];
+        float x4[4];
+        uint2 hh, ll;
 #pragma unroll
-        for (int k = 0; k < 4; k++) split2(w ? (el[k] * we[k]) * rinv : el[k], hh[k], ll[k]);
-        h[256 * e] = make_uint2(hh[0] | ((unsigned)hh[1] << 16), hh[2] | ((unsigned)hh[3] << 16));
-        l[256 * e] = make_uint2(ll[0] | ((unsigned)ll[1] << 16), ll[2] | ((unsigned)ll[3] << 16));
+        for (int k = 0; k < 4; k++) x4[k] = w ? (el[k] * we[k]) * rinv : el[k];
+        bf16_split2(x4[0], x4[1], hh.x, ll.x);
+        bf16_split2(x4[2], x4[3], hh.y, ll.y);
+        h[256 * e] = hh;
+        l[256 * e] = ll;
     }
 }
 
@@ -416,6 +422,69 @@ __global__ __launch_bounds__(256) void gemm_hilo(const uint16_t *__restrict__ ah
     }
 }
 
+// silu(g) u: swiglu1 with the hardware exponential, whose error (|g| ulp of e^-g,
+// weighted by e^-g / (1 + e^-g)) stays two orders below the halves' 2^-17
+__device__ __forceinline__ float gemm_swiglu(float g, float u) {
+    return (g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))) * u;
+}
+
+// The epilogue of a tile held as acc[i][j][r]: row mr + 16 i + r, column nc + 16 j
+// (nc = ... + (lane & 15), whole 16-column tiles inside N).  ADD reads every old
+// value of a row tile before it stores one: written as y += v the compiler must
+// keep each load behind the store before it, a memory latency per value (8191 rows
+// by 1024 columns: K 2048 88 -> 72 us, K 3072 106 -> 101).  SWIGLU: the four lanes of a quad hold
+// the gates and ups of two outputs; lanes 0, 1 store the hi and the lo word of one
+// row's two outputs, lanes 2, 3 those of the next row
+// (401 x 6144 x 1024: 21.7 -> 20.0 us against 2-byte stores from every second lane
+// and scalar roundings).
+template <int EPI, int TM, int TN>
+__device__ __forceinline__ void gemm_store(const f32x4 (&acc)[TM][TN], int mr, int nc, int M, int N, float *y,
+                                           uint16_t *ohi, uint16_t *olo) {
+    if constexpr (EPI == QK_GEMM_SWIGLU) {
+        const int q = threadIdx.x & 3;
+        uint16_t *o = (q & 1) ? olo : ohi;
+        const int oc = (nc - q) / 2;                      // the quad's first output column
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    float s[2], t[2];
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {
+                        const float v = acc[i][j][r + k], p = dpp_read<0xB1>(v);
+                        s[k] = gemm_swiglu((q & 1) ? p : v, (q & 1) ? v : p);
+                        t[k] = dpp_read<0x4E>(s[k]);       // the other pair's output
+                    }
+                    uint32_t h, l;
+                    bf16_split2(q < 2 ? s[0] : t[1], q < 2 ? t[0] : s[1], h, l);
+                    const int m = mr + 16 * i + r + (q >> 1);
+                    if (m < M) *reinterpret_cast<uint32_t *>(o + (size_t)m * (N / 2) + oc + 8 * j) = (q & 1) ? l : h;
+                }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            float old[4][TN];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float *p = y + (size_t)min(mr + 16 * i + r, M - 1) * N + nc;
+#pragma unroll
+                for (int j = 0; j < TN; j++) old[r][j] = EPI == QK_GEMM_ADD ? p[16 * j] : 0.0f;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int m = mr + 16 * i + r;
+                float *p = y + (size_t)m * N + nc;
+                if (m < M) {
+#pragma unroll
+                    for (int j = 0; j < TN; j++) p[16 * j] = EPI == QK_GEMM_ADD ? old[r][j] + acc[i][j][r] : acc[i][j][r];
+                }
+            }
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Large-M GEMM (same product and epilogues as gemm_hilo): block tile BM x 256
 // with 8 waves, each 64 x (256 / WGN) (BM 128: 2 x 4 waves of 64 x 64; BM 256:
@@ -509,29 +578,8 @@ __global__ __launch_bounds__(512, 1) void gemm_hilo_wide(const uint16_t *__restr
         }
     }
 
-    float *yz = y + (EPI == QK_GEMM_STORE ? (size_t)blockIdx.z * M * N : 0);
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + wn * TN * 16 + j * 16 + (lane & 15);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * 64 + i * 16 + 4 * (lane >> 4) + r;
-                const float v = acc[i][j][r];
-                if (EPI == QK_GEMM_SWIGLU) {
-                    const float u = __shfl_xor(v, 1, QK_WAVE);   // column n+1 lives in lane l^1
-                    if ((lane & 1) == 0 && m < M) {
-                        const size_t o = (size_t)m * (N / 2) + (n >> 1);
-                        split2(swiglu1(v, u), ohi[o], olo[o]);
-                    }
-                } else if (m < M) {
-                    if (EPI == QK_GEMM_STORE) yz[(size_t)m * N + n] = v;
-                    else y[(size_t)m * N + n] += v;
-                }
-            }
-        }
-    }
+    gemm_store<EPI>(acc, m0 + wm * 64 + 4 * (lane >> 4), n0 + wn * TN * 16 + (lane & 15), M, N,
+                    y + (EPI == QK_GEMM_STORE ? (size_t)blockIdx.z * M * N : 0), ohi, olo);
 }
 
 template <int BM>
@@ -559,43 +607,28 @@ static void gemm_wide_dispatch(const uint16_t *a_hi, const uint16_t *a_lo, const
 // per CU.  The 16-row load groups of a stage (A_hi, A_lo, W) are dealt
 // round-robin to the waves: LPW 1 KB load instructions per wave and stage.
 // ---------------------------------------------------------------------------
-template <int EPI, int BM, int BN, int NST>
-__global__ __launch_bounds__(ring_waves(BM, BN) * 64) void gemm_hilo_ring(const uint16_t *__restrict__ ahi,
-                                                                           const uint16_t *__restrict__ alo,
-                                                                           const uint16_t *__restrict__ W, int M,
-                                                                           int N, int K, int kc, float *y,
-                                                                           uint16_t *ohi, uint16_t *olo) {
+// KG 2: launches of about one block per CU (ring_walk2)
+template <int EPI, int BM, int BN, int NST, int KG>
+__global__ __launch_bounds__(KG *ring_waves(BM, BN) * 64) void gemm_hilo_ring(const uint16_t *__restrict__ ahi,
+                                                                               const uint16_t *__restrict__ alo,
+                                                                               const uint16_t *__restrict__ W, int M,
+                                                                               int N, int K, int kc, float *y,
+                                                                               uint16_t *ohi, uint16_t *olo) {
     using RS = RingShape<BM, BN>;
-    constexpr int WGN = RS::WGN, WTN = RS::WTN, TM = RS::TM, TN = RS::TN;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[NST * RS::STAGE];
+    constexpr int NW = RS::NW, WGN = RS::WGN, WTN = RS::WTN, TN = RS::TN, TM = KG == 2 ? 1 : RS::TM;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[KG * NST * RS::STAGE];
     f32x4 acc[TM][TN];
-    ring_tile<BM, BN, NST>(ahi, alo, W, M, K, kc, lds, acc);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    float *yz = y + (EPI == QK_GEMM_STORE ? (size_t)blockIdx.z * M * N : 0);
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + wn * WTN + j * 16 + (lane & 15);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * 32 + i * 16 + 4 * (lane >> 4) + r;
-                const float v = acc[i][j][r];
-                if (EPI == QK_GEMM_SWIGLU) {
-                    const float u = __shfl_xor(v, 1, QK_WAVE);   // column n+1 lives in lane l^1
-                    if ((lane & 1) == 0 && m < M) {
-                        const size_t o = (size_t)m * (N / 2) + (n >> 1);
-                        split2(swiglu1(v, u), ohi[o], olo[o]);
-                    }
-                } else if (m < M) {
-                    if (EPI == QK_GEMM_STORE) yz[(size_t)m * N + n] = v;
-                    else y[(size_t)m * N + n] += v;
-                }
-            }
-        }
-    }
+    const int lane = threadIdx.x & 63, bwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = bwave / NW, wave = bwave % NW, wm = wave / WGN, wn = wave % WGN;
+    if constexpr (KG == 2) ring_tile2<BM, BN, NST>(ahi, alo, W, M, K, kc, lds, acc[0]);
+    else ring_tile<BM, BN, NST>(ahi, alo, W, M, K, kc, lds, acc);
+    gemm_store<EPI>(acc, blockIdx.y * BM + wm * 32 + 16 * kg + 4 * (lane >> 4), blockIdx.x * BN + wn * WTN + (lane & 15),
+                    M, N, y + (EPI == QK_GEMM_STORE ? (size_t)blockIdx.z * M * N : 0), ohi, olo);
+}
+
+// two k groups: at most one block per CU, whole 64-deep stages
+static int ring_groups(const dim3 &grid, int K, int kc) {
+    return K % 64 == 0 && kc % 64 == 0 && (long)grid.x * grid.y * grid.z <= 256 ? 2 : 1;
 }
 
 // Q|K|V projection with the RoPE / append epilogue (the work of rope_append
@@ -608,38 +641,41 @@ __global__ __launch_bounds__(ring_waves(BM, BN) * 64) void gemm_hilo_ring(const 
 // the cache.  The sums and products are rope_append's, so the result equals
 // GEMM (STORE, one split) + rope_append bit for bit.
 #define RP_ROW (QWEN_HIP_HEAD_DIM + 4)        // floats per row of the staged tile
-__global__ __launch_bounds__(256) void gemm_hilo_ring_rope(const uint16_t *__restrict__ ahi,
+template <int KG>
+__global__ __launch_bounds__(KG * 256) void gemm_hilo_ring_rope(const uint16_t *__restrict__ ahi,
                                                            const uint16_t *__restrict__ alo,
                                                            const uint16_t *__restrict__ W, int M, int K,
                                                            qk_rope_append_args ra) {
     using RS = RingShape<64, QWEN_HIP_HEAD_DIM>;
-    constexpr int WGN = RS::WGN, WTN = RS::WTN, TM = RS::TM, TN = RS::TN, hd = QWEN_HIP_HEAD_DIM, half = hd / 2;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[QK_GEMM_RING_NST * RS::STAGE];
+    constexpr int NW = RS::NW, WGN = RS::WGN, WTN = RS::WTN, TM = KG == 2 ? 1 : RS::TM, TN = RS::TN, hd = QWEN_HIP_HEAD_DIM,
+                  half = hd / 2, NP = 4 / KG;          // passes of four rows per wave
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[KG * QK_GEMM_RING_NST * RS::STAGE];
     static_assert(64 * RP_ROW * sizeof(float) <= sizeof(lds) && RP_ROW % 4 == 0, "staged tile");
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int lane = threadIdx.x & 63, bwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = bwave / NW, wave = bwave % NW, wm = wave / WGN, wn = wave % WGN;
     const int m0 = blockIdx.y * 64, head = blockIdx.x;
     const int nqk = ra.heads + ra.kv_heads, qd = ra.heads * hd;
     const bool is_q = head < ra.heads, is_k = !is_q && head < nqk;
-    // this wave's 16 rows of the tile: row rl0 + 4 k + g in pass k for the
+    // this wave's 4 NP rows of the tile: row rl0 + 4 k + g in pass k for the
     // 16-lane group g, whose lane c holds dims 4c .. 4c+3 and 64+4c .. 64+4c+3
-    const int rl0 = 16 * wave, g = lane >> 4, c = lane & 15;
+    const int rl0 = 4 * NP * bwave, g = lane >> 4, c = lane & 15;
     // the epilogue's operands (the rows' cos / sin, the norm weights) are
     // loaded before the k walk, so their latency passes under it
-    float4 cv[4], sv[4], wl = make_float4(0.f, 0.f, 0.f, 0.f), wh = wl;
+    float4 cv[NP], sv[NP], wl = make_float4(0.f, 0.f, 0.f, 0.f), wh = wl;
     if (is_q || is_k) {
         const float *nw = is_q ? ra.q_norm : ra.k_norm;
         wl = *reinterpret_cast<const float4 *>(nw + 4 * c);
         wh = *reinterpret_cast<const float4 *>(nw + half + 4 * c);
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
+        for (int k = 0; k < NP; k++) {
             const size_t p = (size_t)ra.start + min(m0 + rl0 + 4 * k + g, M - 1);
             cv[k] = *reinterpret_cast<const float4 *>(ra.rope_cos + p * hd + 4 * c);
             sv[k] = *reinterpret_cast<const float4 *>(ra.rope_sin + p * hd + 4 * c);
         }
     }
     f32x4 acc[TM][TN];
-    ring_tile<64, QWEN_HIP_HEAD_DIM, QK_GEMM_RING_NST>(ahi, alo, W, M, K, K, lds, acc);
+    if constexpr (KG == 2) ring_tile2<64, QWEN_HIP_HEAD_DIM, QK_GEMM_RING_NST>(ahi, alo, W, M, K, K, lds, acc[0]);
+    else ring_tile<64, QWEN_HIP_HEAD_DIM, QK_GEMM_RING_NST>(ahi, alo, W, M, K, K, lds, acc);
 
     __syncthreads();                                   // every wave is past its last k step
     float *T = reinterpret_cast<float *>(lds);         // [64][RP_ROW]
@@ -649,12 +685,12 @@ __global__ __launch_bounds__(256) void gemm_hilo_ring_rope(const uint16_t *__res
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                T[(wm * 32 + i * 16 + 4 * (lane >> 4) + r) * RP_ROW + wn * WTN + j * 16 + (lane & 15)] = acc[i][j][r];
+                T[(wm * 32 + (i + kg) * 16 + 4 * (lane >> 4) + r) * RP_ROW + wn * WTN + j * 16 + (lane & 15)] = acc[i][j][r];
     __syncthreads();
 
     // rows past M are computed on the tile's (finite) contents and not stored
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < NP; k++) {
         const int rl = rl0 + 4 * k + g, srow = m0 + rl;
         float4 lo = *reinterpret_cast<const float4 *>(T + rl * RP_ROW + 4 * c);
         float4 hi = *reinterpret_cast<const float4 *>(T + rl * RP_ROW + half + 4 * c);
@@ -689,20 +725,25 @@ extern "C" int qk_gemm_rope_launch(const uint16_t *a_hi, const uint16_t *a_lo, c
          (uintptr_t)ra->k_cache | (uintptr_t)ra->v_cache | (uintptr_t)ra->q_out) % 16)
         return QWEN_HIP_EINVAL;
     const dim3 grid(ra->heads + 2 * ra->kv_heads, (M + 63) / 64);
-    gemm_hilo_ring_rope<<<grid, 256, 0, s>>>(a_hi, a_lo, W, M, K, *ra);
+    if (ring_groups(grid, K, K) == 2) gemm_hilo_ring_rope<2><<<grid, 512, 0, s>>>(a_hi, a_lo, W, M, K, *ra);
+    else gemm_hilo_ring_rope<1><<<grid, 256, 0, s>>>(a_hi, a_lo, W, M, K, *ra);
     return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
 }
 
-template <int BM, int BN, int NST>
+template <int BM, int BN, int NST, int KG>
 static void gemm_ring_dispatch(const uint16_t *a_hi, const uint16_t *a_lo, const uint16_t *W, int M, int N, int K,
                                const qk_gemm_plan *p, int epi, float *y, uint16_t *oh, uint16_t *ol, hipStream_t s) {
-    const dim3 grid(N / BN, (M + BM - 1) / BM, p->nsplit), block(64 * ring_waves(BM, BN));
+    const dim3 grid(N / BN, (M + BM - 1) / BM, p->nsplit), block(KG * 64 * ring_waves(BM, BN));
+    if (KG == 1 && BM <= 64 && ring_groups(grid, K, p->kc) == 2) {
+        gemm_ring_dispatch<BM, BN, NST, BM <= 64 ? 2 : 1>(a_hi, a_lo, W, M, N, K, p, epi, y, oh, ol, s);
+        return;
+    }
     if (epi == QK_GEMM_STORE)
-        gemm_hilo_ring<QK_GEMM_STORE, BM, BN, NST><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
+        gemm_hilo_ring<QK_GEMM_STORE, BM, BN, NST, KG><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
     else if (epi == QK_GEMM_ADD)
-        gemm_hilo_ring<QK_GEMM_ADD, BM, BN, NST><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
+        gemm_hilo_ring<QK_GEMM_ADD, BM, BN, NST, KG><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
     else
-        gemm_hilo_ring<QK_GEMM_SWIGLU, BM, BN, NST><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
+        gemm_hilo_ring<QK_GEMM_SWIGLU, BM, BN, NST, KG><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
 }
 
 // the ring configurations built: (bm, bn, nst); 0 when the plan names another
@@ -710,7 +751,7 @@ static int gemm_ring_launch(const uint16_t *a_hi, const uint16_t *a_lo, const ui
                             const qk_gemm_plan *p, int epi, float *y, uint16_t *oh, uint16_t *ol, hipStream_t s) {
 #define QK_RING(BM_, BN_, NST_)                                                                  \
     if (p->bm == BM_ && p->bn == BN_ && p->nst == NST_) {                                        \
-        gemm_ring_dispatch<BM_, BN_, NST_>(a_hi, a_lo, W, M, N, K, p, epi, y, oh, ol, s);        \
+        gemm_ring_dispatch<BM_, BN_, NST_, 1>(a_hi, a_lo, W, M, N, K, p, epi, y, oh, ol, s);        \
         return 1;                                                                                \
     }
     QK_RING(64, 128, QK_GEMM_RING_NST) QK_RING(32, 128, QK_GEMM_RING_NST) QK_RING(128, 128, 3)

@@ -203,3 +203,28 @@ __device__ __forceinline__ void ring_tile(const uint16_t *__restrict__ ahi, cons
         for (int j = 0; j < LPW; j++) lds_load16(src[j] + kt * QK_GBK, st + dst[j]);
     });
 }
+
+// ring_tile by two k groups (ring_walk2): K and kc multiples of 64
+template <int BM, int BN, int NST>
+__device__ __forceinline__ void ring_tile2(const uint16_t *__restrict__ ahi, const uint16_t *__restrict__ alo,
+                                           const uint16_t *__restrict__ W, int M, int K, int kc, unsigned char *lds,
+                                           f32x4 (&fin)[RingShape<BM, BN>::TN]) {
+    using RS = RingShape2<BM, BN>;
+    constexpr int NW2 = 2 * RS::NW, LPW = RS::LPW2;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int kb = blockIdx.z * kc, ke = min(K, kb + kc);
+    const int r8 = lane >> 3, c8 = (lane & 7) ^ r8;
+    const uint16_t *src[LPW];
+#pragma unroll
+    for (int j = 0; j < LPW; j++) {
+        const int g = wave + NW2 * j;                     // A_hi, A_lo, W groups of 8 rows follow one another
+        src[j] = (g < BM / 8   ? ahi + (size_t)min(m0 + 8 * g + r8, M - 1) * K
+                  : g < BM / 4 ? alo + (size_t)min(m0 + 8 * (g - BM / 8) + r8, M - 1) * K
+                               : W + (size_t)(n0 + 8 * (g - BM / 4) + r8) * K) + kb + 8 * c8;
+    }
+    ring_walk2<BM, BN, NST>((ke - kb) / 64, lds, fin, [&](int p, unsigned char *st) {
+#pragma unroll
+        for (int j = 0; j < LPW; j++) lds_load16(src[j] + 64 * p, st + 1024 * (wave + NW2 * j));
+    });
+}
