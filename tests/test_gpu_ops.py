@@ -464,3 +464,78 @@ def test_causal_attention_wide_blocks(P, qa, gpu, sq, sk, q_off):
     ref = gpu.bmm(gpu.softmax(sc.masked_fill(mask, float("-inf")), -1), v).transpose(0, 1).reshape(sq, nh * hd)
     # the bar of the other attention tests: the bf16 pairs leave 2^-16 per product
     assert bool(((out.double() - ref).abs() <= 3e-5 + 1e-4 * ref.abs()).all())
+
+
+# the vector and scalar forms of the elementwise operators: whole and ragged
+# vectors, rows longer than a block's registers, pointers off 16 bytes
+@pytest.mark.parametrize("S,D", [(1, 4), (3, 100), (1, 1024), (5, 1028), (2, 2048), (2, 4096), (2, 4100), (4, 6)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_elementwise_forms(P, qa, gpu, S, D, off):
+    lib, g = qa.lib(), gpu.Generator(device="cuda").manual_seed(S * D)
+
+    def buf(n):                                   # n floats, `off` floats past a 16-byte boundary
+        t = gpu.empty(n + 4, device="cuda")[off:off + n]
+        return t.copy_(gpu.randn(n, generator=g, device="cuda"))
+    n, one = S * D, 2.0 ** -22
+    a, b = buf(n), buf(n)
+    want = a.double() + b.double()
+    qa.check(lib.qwen_hip_add_inplace(ptr(a), ptr(b), n, None))
+    assert bool(((a.double() - want).abs() <= one * want.abs() + 1e-30).all())
+    x, w, o = buf(n), buf(D), buf(n)
+    qa.check(lib.qwen_hip_rms_norm(ptr(o), ptr(x), ptr(w), S, D, 1e-6, None))
+    xd = x.double().view(S, D)
+    want = (xd * w.double() / gpu.sqrt((xd * xd).mean(1, keepdim=True) + 1e-6)).view(-1)
+    tol = (4 + D ** 0.5) * 2.0 ** -24             # the row's sum of squares, then three roundings
+    assert bool(((o.double() - want).abs() <= tol * want.abs() + 1e-30).all())
+    # SwiGLU, and in place, where the outputs overwrite the inputs of the rows before
+    gu, o = buf(2 * n), buf(n)
+    gd = gu.double().view(n, 2)
+    want = gd[:, 0] / (1 + gpu.exp(-gd[:, 0])) * gd[:, 1]
+    qa.check(lib.qwen_hip_swiglu_multiply(ptr(o), ptr(gu), S, D, None))
+    assert bool(((o.double() - want).abs() <= 8 * 2.0 ** -24 * want.abs() + 1e-30).all())
+    qa.check(lib.qwen_hip_swiglu_multiply(ptr(gu), ptr(gu), S, D, None))
+    assert bool(gpu.equal(gu[:n], o))
+
+
+@pytest.mark.parametrize("S,inter", [(1, 6144), (2, 6144), (3, 3072), (9, 2000), (401, 3072)])
+def test_swiglu_in_place_rows(P, qa, gpu, S, inter):
+    g = gpu.Generator(device="cuda").manual_seed(S)
+    gu = gpu.randn(S * 2 * inter, generator=g, device="cuda")
+    o = gpu.empty(S * inter, device="cuda")
+    qa.check(qa.lib().qwen_hip_swiglu_multiply(ptr(o), ptr(gu), S, inter, None))
+    qa.check(qa.lib().qwen_hip_swiglu_multiply(ptr(gu), ptr(gu), S, inter, None))
+    assert bool(gpu.equal(gu[:S * inter], o))
+    assert qa.lib().qwen_hip_swiglu_multiply(ptr(gu), ptr(gu), 1, 24 * 256 + 1, None) == -1
+
+
+@pytest.mark.parametrize("S,nh,off", [(1, 16, 0), (7, 3, 0), (5, 8, 1)])
+def test_head_norm_rope_forms(P, qa, gpu, S, nh, off):
+    lib, g = qa.lib(), gpu.Generator(device="cuda").manual_seed(S)
+    x = gpu.empty(S * nh * 128 + 4, device="cuda")[off:off + S * nh * 128]
+    x.copy_(gpu.randn(S * nh * 128, generator=g, device="cuda"))
+    w, c, s = (gpu.randn(k, 128, generator=g, device="cuda") for k in (1, S, S))
+    xd = x.double().view(S, nh, 128)
+    y = xd * w.double() / gpu.sqrt((xd * xd).mean(-1, keepdim=True) + 1e-6)
+    qa.check(lib.qwen_hip_rms_norm_per_head(ptr(x), ptr(w), S, nh, 128, 1e-6, None))
+    assert bool(((x.double().view_as(y) - y).abs() <= 16 * 2.0 ** -24 * y.abs() + 1e-30).all())
+    yd = x.double().view_as(y)
+    a, b, cd, sd = yd[..., :64], yd[..., 64:], c.double()[:, None, :64], s.double()[:, None, :64]
+    want = gpu.cat([a * cd - b * sd, b * cd + a * sd], -1)
+    size = gpu.cat([(a * cd).abs() + (b * sd).abs(), (b * cd).abs() + (a * sd).abs()], -1)
+    qa.check(lib.qwen_hip_apply_rope_neox(ptr(x), ptr(c), ptr(s), S, nh, 128, None))
+    assert bool(((x.double().view_as(y) - want).abs() <= 2 * 2.0 ** -24 * size + 1e-30).all())
+
+
+# one query over 1 .. 32 splits of its keys (the combine takes 16 at a time)
+@pytest.mark.parametrize("sk", [1, 32, 33, 512, 513, 1024, 1500])
+def test_one_query_splits(P, qa, gpu, sk):
+    g = gpu.Generator(device="cuda").manual_seed(sk)
+    Q, K, V = (gpu.randn(n, h * 128, generator=g, device="cuda") for n, h in ((1, 16), (sk, 8), (sk, 8)))
+    out = gpu.empty(1, 2048, device="cuda")
+    qa.check(qa.lib().qwen_hip_causal_attention(ptr(out), ptr(Q), ptr(K), ptr(V), 1, sk, 16, 8, 128,
+                                                1.0 / np.sqrt(128.0), sk - 1, None))
+    k = K.double().view(sk, 8, 128).repeat_interleave(2, 1).permute(1, 2, 0).contiguous()
+    v = V.double().view(sk, 8, 128).repeat_interleave(2, 1).transpose(0, 1).contiguous()
+    p = gpu.softmax(gpu.bmm(Q.double().view(16, 1, 128), k) / np.sqrt(128.0), -1)
+    ref = gpu.bmm(p, v).view(1, 2048)
+    assert bool(((out.double() - ref).abs() <= 1e-6 + 1e-5 * ref.abs()).all())     # fp32 products and sums
