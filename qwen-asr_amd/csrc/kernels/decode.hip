@@ -48,7 +48,7 @@ __device__ __forceinline__ void gemv_load(uint4 (&w)[ROWS][NC], const uint16_t *
 // only the argmax epilogue walks several row groups per wave (iters), so the
 // other instances hold no second weight buffer and no merge registers.
 template <int NC, int ROWS, int EPI, bool MERGE>
-__global__ __launch_bounds__(256) void gemv_kernel(qk_gemv_args a, int iters_arg) {
+__device__ __forceinline__ void gemv_block(const qk_gemv_args &a, const int iters_arg, const int block) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int K = a.K, R = a.rows;
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(qk_gemv_args a, int iters_arg
     // loads before the prologue so HBM latency overlaps the gather / norm.
     const int rows_per_block = 4 * ROWS * iters;
     uint4 w[ROWS][NC];
-    int rbase = blockIdx.x * rows_per_block + wave * ROWS;
+    int rbase = block * rows_per_block + wave * ROWS;
     if (rbase < R) gemv_load<NC, ROWS>(w, a.W, R, K, rbase, lane);
 
     // ---- prologue: the input row, optionally gathered and RMS-normed ----
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(qk_gemv_args a, int iters_arg
             for (int j = 0; j < 8; j++) xr[c][j] = 0.0f;
         }
     }
-    if (tok >= 0 && a.x_store && blockIdx.x == 0 && wave == 0) {
+    if (tok >= 0 && a.x_store && block == 0 && wave == 0) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const int col = c * 512 + lane * 8;
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(qk_gemv_args a, int iters_arg
                 for (int j = 0; j < 8; j++) xr[c][j] = (xr[c][j] * a.norm_w[col + j]) * rinv;
         }
     }
-    if (a.normed_store && blockIdx.x == 0 && wave == 0) {
+    if (a.normed_store && block == 0 && wave == 0) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const int col = c * 512 + lane * 8;
@@ -241,10 +241,37 @@ __global__ __launch_bounds__(256) void gemv_kernel(qk_gemv_args a, int iters_arg
             int bi = si[0];
             for (int i = 1; i < 4; i++)
                 if (argmax_better(sv[i], si[i], bv, bi)) { bv = sv[i]; bi = si[i]; }
-            a.cand_val[blockIdx.x] = bv;
-            a.cand_idx[blockIdx.x] = bi;
+            a.cand_val[block] = bv;
+            a.cand_idx[block] = bi;
         }
     }
+}
+
+template <int NC, int ROWS, int EPI, bool MERGE>
+__global__ __launch_bounds__(256) void gemv_kernel(qk_gemv_args a, int iters) {
+    gemv_block<NC, ROWS, EPI, MERGE>(a, iters, blockIdx.x);
+}
+
+// Three products of one plain input row: a grid of all their row groups, in order.
+// Each product alone is 2.3 to 3 us of kernel, less than a host program needs to
+// issue it, and leaves CUs without a block; a decoder layer's attention half called
+// operator by operator takes 81 us (hidden 1024; 89 with three launches) and 67 (hidden
+// 2048; 82).  Two rows a wave: 512 blocks for 4096 rows in all.
+template <int NC, int ROWS>
+__global__ __launch_bounds__(256) void gemv3_kernel(qk_gemv3_args t) {
+    int b = blockIdx.x, m = 0;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int n = (t.rows[i] + 4 * ROWS - 1) / (4 * ROWS);
+        if (m == i && b >= n) { b -= n; m++; }
+    }
+    qk_gemv_args a = {};
+    a.W = m == 0 ? t.W[0] : m == 1 ? t.W[1] : t.W[2];
+    a.y = m == 0 ? t.y[0] : m == 1 ? t.y[1] : t.y[2];
+    a.rows = m == 0 ? t.rows[0] : m == 1 ? t.rows[1] : t.rows[2];
+    a.K = t.K;
+    a.x = t.x;
+    gemv_block<NC, ROWS, QK_EPI_STORE, false>(a, 1, b);
 }
 
 // Long rows (STORE or ADD, plain x; gemv_ks_fits): the block's four waves split
@@ -398,6 +425,26 @@ extern "C" int qk_gemv_launch(const qk_gemv_args *a, hipStream_t s) {
     case 7:
     case 8: gemv_dispatch_rows<8>(a, rows_pw, iters, blocks, s); break;
     default: gemv_dispatch_rows<12>(a, rows_pw, iters, blocks, s); break;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
+}
+
+template <int NC>
+static void gemv3_dispatch(const qk_gemv3_args *t, hipStream_t s) {
+    constexpr int ROWS = 2;
+    int blocks = 0;
+    for (int i = 0; i < 3; i++) blocks += (t->rows[i] + 4 * ROWS - 1) / (4 * ROWS);
+    gemv3_kernel<NC, ROWS><<<blocks, 256, 0, s>>>(*t);
+}
+
+extern "C" int qk_gemv3_launch(const qk_gemv3_args *t, hipStream_t s) {
+    if (!t || !t->x || t->K <= 0 || (t->K & 7) || t->K > 4 * 512) return QWEN_HIP_EINVAL;
+    for (int i = 0; i < 3; i++)
+        if (!t->W[i] || !t->y[i] || t->rows[i] <= 0 || t->rows[i] > (1 << 28)) return QWEN_HIP_EINVAL;
+    switch ((t->K + 511) / 512) {
+    case 1: gemv3_dispatch<1>(t, s); break;
+    case 2: gemv3_dispatch<2>(t, s); break;
+    default: gemv3_dispatch<4>(t, s); break;
     }
     return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
 }

@@ -43,6 +43,14 @@ typedef struct {
 #define QK_MERGE_MAX_K 2048       /* ... over an input row of at most this length */
 
 int qk_gemv_launch(const qk_gemv_args *a, hipStream_t s);
+/* y[i] = W[i] x for three matrices of one input row, in one launch (K <= 2048) */
+typedef struct {
+    const uint16_t *W[3];     /* [rows[i]][K] bf16 */
+    float *y[3];
+    int rows[3], K;
+    const float *x;
+} qk_gemv3_args;
+int qk_gemv3_launch(const qk_gemv3_args *t, hipStream_t s);
 /* number of blocks qk_gemv_launch uses (= candidates for ARGMAX) */
 int qk_gemv_blocks(int rows, int K, int epi);
 

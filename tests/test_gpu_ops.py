@@ -539,3 +539,23 @@ def test_one_query_splits(P, qa, gpu, sk):
     p = gpu.softmax(gpu.bmm(Q.double().view(16, 1, 128), k) / np.sqrt(128.0), -1)
     ref = gpu.bmm(p, v).view(1, 2048)
     assert bool(((out.double() - ref).abs() <= 1e-6 + 1e-5 * ref.abs()).all())     # fp32 products and sums
+
+
+# the three products of one row in one launch (K <= 2048; 8 rows a block), and
+# the separate ones above: row counts around a block's, every K chunk count
+@pytest.mark.parametrize("hidden", [8, 520, 1024, 1032, 2048, 2056])
+@pytest.mark.parametrize("qd,kvd", [(1, 1), (8, 9), (23, 7)])
+def test_linear_qkv_edges(P, qa, gpu, hidden, qd, kvd):
+    Ws = [P.synth_bf16(n * hidden, 2, 9500 + i).reshape(n, hidden) for i, n in enumerate((qd, kvd, kvd))]
+    x = P.synth_uniform(hidden, 2, 9550 + hidden)
+    dW, dx = [dev(gpu, W.view(np.int16)) for W in Ws], dev(gpu, x)
+    # one value past each output stays as it is
+    out = [gpu.full((n + 1,), 7.0, dtype=gpu.float32, device="cuda") for n in (qd, kvd, kvd)]
+    qa.check(qa.lib().qwen_hip_linear_nobias_bf16_qkv(*[ptr(o) for o in out], ptr(dx), *[ptr(W) for W in dW],
+                                                      hidden, qd, kvd, None), "qkv")
+    gpu.cuda.synchronize()
+    for W, o in zip(Ws, out):
+        y = host(o)
+        exp = P.bf16_to_f32(W).astype(np.float64) @ x.astype(np.float64)
+        bound = 8 * hidden * 2.0 ** -24 * (np.abs(P.bf16_to_f32(W)) @ np.abs(x)) + 1e-12
+        assert np.all(np.abs(y[:-1] - exp) <= bound) and y[-1] == 7.0
