@@ -754,6 +754,17 @@ static int gemm_ring_launch(const uint16_t *a_hi, const uint16_t *a_lo, const ui
         gemm_ring_dispatch<BM_, BN_, NST_, 1>(a_hi, a_lo, W, M, N, K, p, epi, y, oh, ol, s);        \
         return 1;                                                                                \
     }
+    if (p->bn == QK_GEMM_NARROW_BN && epi == QK_GEMM_SWIGLU && K % QK_BK == 0 && p->kc >= K && M <= p->bm) {
+        const dim3 grid(N / QK_GEMM_NARROW_BN), block(2 * 64 * ring_waves(32, QK_GEMM_NARROW_BN));
+        static_assert(ring_waves(32, QK_GEMM_NARROW_BN) == ring_waves(64, QK_GEMM_NARROW_BN), "block");
+        if (p->bm == 32 && p->nst == 8)
+            gemm_hilo_ring<QK_GEMM_SWIGLU, 32, QK_GEMM_NARROW_BN, 8, 2><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
+        else if (p->bm == 64 && p->nst == 6)
+            gemm_hilo_ring<QK_GEMM_SWIGLU, 64, QK_GEMM_NARROW_BN, 6, 2><<<grid, block, 0, s>>>(a_hi, a_lo, W, M, N, K, p->kc, y, oh, ol);
+        else
+            return 0;
+        return 1;
+    }
     QK_RING(64, 128, QK_GEMM_RING_NST) QK_RING(32, 128, QK_GEMM_RING_NST) QK_RING(128, 128, 3)
 #undef QK_RING
     return 0;
@@ -786,6 +797,22 @@ extern "C" void qk_gemm_plan_epi(int M, int N, int K, int epi, qk_gemm_plan *p) 
         p->bn = 256;
         p->nsplit = 1;
         p->kc = (K + QK_BK - 1) / QK_BK * QK_BK;
+        return;
+    }
+    // SwiGLU of up to 64 rows: bound by the weight bytes in flight.  64-column
+    // tiles, one block per CU with a ring of 8 (6) stages and the whole k walk, so
+    // neither partials nor a reduce pass, where they give half the CUs a block.
+    // Prefill of 4 layers over 300 positions, against split 128-column tiles and a
+    // reduce: 12288 columns (192 tiles) 31 rows 320 -> 301 us, 64 rows 383 -> 354;
+    // 6144 (96 tiles) 64 rows 282 -> 272, 31 rows 231 -> 229, 2 rows 201 -> 205.
+    const int narrow = N / QK_GEMM_NARROW_BN;
+    if (epi == QK_GEMM_SWIGLU && M <= 64 && N % QK_GEMM_NARROW_BN == 0 && K % QK_BK == 0 &&
+        narrow >= (M <= 32 ? 128 : 96) && narrow <= QK_GEMM_TARGET) {
+        p->bm = M <= 32 ? 32 : 64;
+        p->bn = QK_GEMM_NARROW_BN;
+        p->nst = M <= 32 ? 8 : 6;
+        p->nsplit = 1;
+        p->kc = K;
         return;
     }
     // otherwise 32 x 128 (M <= 32) or 64 x 128 tiles on the LDS ring where the

@@ -321,7 +321,8 @@ enum { QK_GEMM_STORE = 0, QK_GEMM_ADD = 1, QK_GEMM_SWIGLU = 2, QK_GEMM_ROPE = 3 
 /* Tiling of one M x N x K product: block rows bm x columns bn (32 / 64 x
  * QK_GEMM_BN on the LDS ring of nst stages, 128 x QK_GEMM_BN on a 3-stage
  * ring for STORE and SwiGLU products above 512 rows, 32 / 64 / 128 x
- * QK_GEMM_BN register-staged (nst 0), or 128 / 256 x 256 for large M), and
+ * QK_GEMM_BN register-staged (nst 0), or 128 / 256 x 256 for large M; 32 / 64
+ * x QK_GEMM_NARROW_BN for SwiGLU products of up to 64 rows, one split), and
  * nsplit slices of kc (a multiple of 64) along K so a launch has enough
  * blocks.  Split rule on the ring: about QK_GEMM_RING_TARGET blocks, and two
  * splits at least for k walks of QK_GEMM_RING_KSPLIT or more; a STORE product
@@ -331,6 +332,7 @@ enum { QK_GEMM_STORE = 0, QK_GEMM_ADD = 1, QK_GEMM_SWIGLU = 2, QK_GEMM_ROPE = 3 
  * split where its output tiles alone number QK_GEMM_TARGET or more. */
 #define QK_GEMM_BN 128
 #define QK_GEMM_TARGET 256
+#define QK_GEMM_NARROW_BN 64         /* column tile of a SwiGLU product of up to 64 rows */
 #define QK_GEMM_MAX_SPLIT 16
 #define QK_GEMM_RING_NST 4           /* 64 KB of LDS at 64 x 128: two blocks per CU */
 #define QK_GEMM_RING_TARGET 224      /* blocks a ring launch aims for */

@@ -541,6 +541,18 @@ def test_one_query_splits(P, qa, gpu, sk):
     assert bool(((out.double() - ref).abs() <= 1e-6 + 1e-5 * ref.abs()).all())     # fp32 products and sums
 
 
+# the 64-column SwiGLU tiles of up to 64 rows: both row tiles, rows short of a
+# tile, the fewest and the most column tiles, k walks shorter than the ring and
+# not a multiple of its depth
+@pytest.mark.parametrize("M", [2, 31, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(8192, 64), (8192, 1024), (16384, 320), (12288, 2048)])
+def test_gemm_swiglu_narrow(P, qa, gpu, M, N, K):
+    p = GemmPlan()
+    qa.lib().qk_gemm_plan_epi(M, N, K, 2, C.byref(p))
+    assert (p.bm, p.bn, p.nsplit) == (32 if M <= 32 else 64, 64, 1)
+    check_gemm(P, qa, gpu, M, N, K, p, 2)
+
+
 # the three products of one row in one launch (K <= 2048; 8 rows a block), and
 # the separate ones above: row counts around a block's, every K chunk count
 @pytest.mark.parametrize("hidden", [8, 520, 1024, 1032, 2048, 2056])
