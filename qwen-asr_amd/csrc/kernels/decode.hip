@@ -255,8 +255,8 @@ __global__ __launch_bounds__(256) void gemv_kernel(qk_gemv_args a, int iters) {
 // Three products of one plain input row: a grid of all their row groups, in order.
 // Each product alone is 2.3 to 3 us of kernel, less than a host program needs to
 // issue it, and leaves CUs without a block; a decoder layer's attention half called
-// operator by operator takes 81 us (hidden 1024; 89 with three launches) and 67 (hidden
-// 2048; 82).  Two rows a wave: 512 blocks for 4096 rows in all.
+// operator by operator takes 75 us (hidden 1024; 82 with three launches) and 76 (hidden
+// 2048; 81).  Two rows a wave: 512 blocks for 4096 rows in all.
 template <int NC, int ROWS>
 __global__ __launch_bounds__(256) void gemv3_kernel(qk_gemv3_args t) {
     int b = blockIdx.x, m = 0;

@@ -596,15 +596,15 @@ enum { ENC_PART, ENC_F32, ENC_GELU };
 // epilogue is chosen at compile time: with tests between the 32 values of a lane
 // their chains ran one after the other, 9.3 us of a 390 x 3584 x 896 GELU
 // product's 20 against 1.9 of its 12 now.
-template <int BM, int NST, bool GATHER, int EPI, int KG>
-__global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_ring_args a) {
-    using RS = RingShape<BM, 128>;
+template <int BM, int BN, int NST, bool GATHER, int EPI, int KG>
+__global__ __launch_bounds__(KG *ring_waves(BM, BN) * 64) void enc_ring(qk_enc_ring_args a) {
+    using RS = RingShape<BM, BN>;
     constexpr int NW = RS::NW, WGN = RS::WGN, WTN = RS::WTN, TN = RS::TN, AB = RS::AB, LPW = RS::LPW;
     constexpr int NI = KG == 2 ? 1 : 2;                // 16-row tiles this wave finishes
     __shared__ __attribute__((aligned(1024))) unsigned char lds[KG * NST * RS::STAGE];   // two groups: RingShape2's stages
     const int lane = threadIdx.x & 63, bwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = bwave / NW, wave = bwave % NW;      // k group, wave of the group
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * 128;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
     const int kb = blockIdx.z * a.kc, ke = min(a.K, kb + a.kc), nk = (ke - kb) / QK_GBK;
     const int rr = lane >> 2, cl = (lane & 3) ^ ((rr >> 1) & 3);
     f32x4 acc[NI][TN];
@@ -638,7 +638,7 @@ __global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_
             w[j] = a.W + (size_t)(kb / QK_GBK) * a.N * QK_GBK + (size_t)min(n0 + 16 * (wave + NW * j) + rr, a.N - 1) * QK_GBK +
                    8 * cl;
         const size_t wstep = (size_t)a.N * QK_GBK;
-        ring_walk<BM, 128, NST, true>(nk, lds, acc, [&](int kt, unsigned char *st) {
+        ring_walk<BM, BN, NST, true>(nk, lds, acc, [&](int kt, unsigned char *st) {
             // a 32-wide k tile lies in one tap
             const int k = kb + kt * QK_GBK, tap = k / QK_ENC_CH, ic = k - tap * QK_ENC_CH;
             const int off = a.taps == 9 ? (tap / 3) * a.in_w + tap % 3 : tap * a.in_w;
@@ -651,7 +651,7 @@ __global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_
             for (int j = 0; j < LPW - 2; j++) lds_load16(w[j] + kt * wstep, st + 2 * AB + 1024 * (wave + NW * j));
         });
     } else if constexpr (KG == 2) {
-        using R2 = RingShape2<BM, 128>;
+        using R2 = RingShape2<BM, BN>;
         const int r8 = lane >> 3, c8 = (lane & 7) ^ r8;
         const uint16_t *src[R2::LPW2];
 #pragma unroll
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_
             src[j] = (g < BM / 4 ? a.A + (size_t)min(m0 + 8 * ga + r8, a.M - 1) * (2 * a.K) + (g < BM / 8 ? 0 : a.K)
                                  : a.W + (size_t)min(n0 + 8 * (g - BM / 4) + r8, a.N - 1) * a.K) + kb + 8 * c8;
         }
-        ring_walk2<BM, 128, NST>(nk / 2, lds, acc[0], [&](int p, unsigned char *st) {
+        ring_walk2<BM, BN, NST>(nk / 2, lds, acc[0], [&](int p, unsigned char *st) {
 #pragma unroll
             for (int j = 0; j < R2::LPW2; j++) lds_load16(src[j] + 64 * p, st + 1024 * (bwave + 2 * NW * j));
         });
@@ -674,7 +674,7 @@ __global__ __launch_bounds__(KG *ring_waves(BM, 128) * 64) void enc_ring(qk_enc_
                                  : a.W + (size_t)min(n0 + 16 * (g - BM / 8) + rr, a.N - 1) * a.K) + kb + 8 * cl;
             dst[j] = 1024 * g;         // A_hi, A_lo and W groups follow one another
         }
-        ring_walk<BM, 128, NST>(nk, lds, acc, [&](int kt, unsigned char *st) {
+        ring_walk<BM, BN, NST>(nk, lds, acc, [&](int kt, unsigned char *st) {
 #pragma unroll
             for (int j = 0; j < LPW; j++) lds_load16(src[j] + kt * QK_GBK, st + dst[j]);
         });
@@ -794,7 +794,7 @@ __global__ __launch_bounds__(256) void enc_ring_reduce_ln(qk_enc_ring_args a) {
 // in six splits 18.2 us, 245 in five 14.2), k walks of 4 k tiles at least.  A
 // product whose epilogue needs no reduce pass (`fused`) and walks up to
 // QK_ENC_RING_FUSED k tiles is not cut in two: that saves 3.5 us, the reduce takes
-// 4.5 (in five, 97 x 3072 x 1024: 7.6 + 4.5 us against 13.4 unsplit).
+// 4.5.
 extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, long ws_elems, int *bm, int *kc,
                                  int *split) {
     const long nt = (N + 127) / 128;
@@ -813,6 +813,17 @@ extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, lon
     *split = (kt + per - 1) / per;
 }
 
+// Products with their own epilogue over few rows: 32 x 64 tiles, unsplit, on at
+// most one block per CU, whose ring of 8 stages keeps the loads in flight that a
+// split's extra blocks did: no partials, no reduce pass.  Whole encoder against
+// split 64 x 128 tiles: 1.7B shape, 97 rows 1364 -> 1194 us, 47 rows 1254 -> 1134,
+// 156 rows 1588 -> 1466; 0.6B, 97 rows 1062 -> 899; with few blocks (8 rows, 42 of
+// them; 32-row tiles before) 728 -> 714.
+static bool enc_ring_narrow(int M, int N, int K) {
+    const long blocks = (long)((M + 31) / 32) * ((N + 63) / 64);
+    return K % 64 == 0 && K <= QK_ENC_RING_FUSED * QK_GBK && blocks >= QK_ENC_NARROW_MIN && blocks <= 256;
+}
+
 extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_elems, hipStream_t s) {
     if (!a || !a->A || !a->W || a->M <= 0 || a->N <= 0 || (a->N & 3) || a->K <= 0 || a->K % QK_GBK) return QWEN_HIP_EINVAL;
     const bool ln = a->ln_w != nullptr, gather = a->taps > 0;
@@ -824,6 +835,16 @@ extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_
         return QWEN_HIP_EINVAL;
     if (a->valid > 0 && (a->col_h <= 0 || a->col_w <= 0)) return QWEN_HIP_EINVAL;
     qk_enc_ring_args g = *a;
+    if (!ln && !gather && enc_ring_narrow(a->M, a->N, a->K)) {
+        const dim3 grid((a->N + 63) / 64, (a->M + 31) / 32);
+        g.kc = a->K;
+        g.split = 1;
+        g.ws = nullptr;
+        constexpr int threads = 2 * 64 * ring_waves(32, 64);
+        if (a->C) enc_ring<32, 64, 8, false, ENC_F32, 2><<<grid, threads, 0, s>>>(g);
+        else enc_ring<32, 64, 8, false, ENC_GELU, 2><<<grid, threads, 0, s>>>(g);
+        return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
+    }
     int bm;
     qk_enc_ring_plan(a->M, a->N, a->K, !ln, gather, ws ? ws_elems : 0, &bm, &g.kc, &g.split);
     g.ws = ln || g.split > 1 ? ws : nullptr;
@@ -833,7 +854,7 @@ extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_
     const int epi = g.ws ? ENC_PART : a->C ? ENC_F32 : ENC_GELU;
 #define QK_ENC_RING(BM_, NST_, G_, E_, KG_)                               \
     if (bm == BM_ && gather == G_ && epi == E_ && kgs == KG_)             \
-        enc_ring<BM_, NST_, G_, E_, KG_><<<grid, KG_ * 64 * ring_waves(BM_, 128), 0, s>>>(g);
+        enc_ring<BM_, 128, NST_, G_, E_, KG_><<<grid, KG_ * 64 * ring_waves(BM_, 128), 0, s>>>(g);
 #define QK_ENC_RING_BM(BM_, NST_, G_, KG_) \
     QK_ENC_RING(BM_, NST_, G_, ENC_PART, KG_) QK_ENC_RING(BM_, NST_, G_, ENC_GELU, KG_)
     QK_ENC_RING_BM(128, 3, true, 1) QK_ENC_RING_BM(64, 4, true, 1)

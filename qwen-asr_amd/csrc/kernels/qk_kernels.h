@@ -440,6 +440,7 @@ int qk_enc_attention_launch(const float *qkv, float *out, uint16_t *out16, int T
 #define QK_ENC_RING_TARGET 256    /* blocks a split launch aims for */
 #define QK_ENC_RING_FUSED 32      /* k tiles up to which a product without a reduce pass is not split */
 #define QK_ENC_RING_SPLIT 8       /* at most */
+#define QK_ENC_NARROW_MIN 32      /* blocks from which such a product over few rows takes 32 x 64 tiles */
 typedef struct {
     const uint16_t *A, *W, *zero;
     int M, N, K;

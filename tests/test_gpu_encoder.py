@@ -262,6 +262,14 @@ def test_ring_products(P, qa, gpu, M, N, K, what):
         assert float((unhalve(gpu, out, N) - ref).abs().max()) < 2e-4      # 2^-16 of values up to ~8
 
 
+# few rows with an own epilogue: 32 x 64 tiles on one block per CU, at the fewest
+# and the most blocks, ragged rows and columns, k walks shorter than the ring
+@pytest.mark.parametrize("M,N,K", [(1, 8192, 64), (33, 3080, 128), (97, 2688, 896), (128, 4096, 1024), (160, 3068, 640)])
+@pytest.mark.parametrize("what", ["f32", "gelu"])
+def test_ring_products_narrow(P, qa, gpu, M, N, K, what):
+    test_ring_products(P, qa, gpu, M, N, K, what)
+
+
 @pytest.mark.parametrize("chunks,h,w,valid", [(1, 8, 5, 3), (3, 32, 25, 1), (9, 32, 50, 25), (2, 4, 1, 1)])
 def test_ring_convolution(P, qa, gpu, chunks, h, w, valid):
     """The gathered 3x3 / stride 2 / padding 1 convolution with GELU, weights
