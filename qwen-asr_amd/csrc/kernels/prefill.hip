@@ -784,6 +784,25 @@ static void gemm_dispatch(const uint16_t *a_hi, const uint16_t *a_lo, const uint
 
 extern "C" void qk_gemm_plan_for(int M, int N, int K, qk_gemm_plan *p) { qk_gemm_plan_epi(M, N, K, QK_GEMM_STORE, p); }
 
+// SwiGLU of up to 64 rows: bound by the weight bytes in flight.  64-column
+// tiles, one block per CU with a ring of 8 (6) stages and the whole k walk, so
+// neither partials nor a reduce pass, where they give half the CUs a block.
+// Prefill of 4 layers over 300 positions, against split 128-column tiles and a
+// reduce: 12288 columns (192 tiles) 31 rows 320 -> 301 us, 64 rows 383 -> 354;
+// 6144 (96 tiles) 64 rows 282 -> 272, 31 rows 231 -> 229, 2 rows 201 -> 205.
+extern "C" int qk_gemm_plan_narrow(int M, int N, int K, qk_gemm_plan *p) {
+    const int narrow = N / QK_GEMM_NARROW_BN;
+    if (M <= 0 || M > 64 || N % QK_GEMM_NARROW_BN || K <= 0 || K % QK_BK || narrow < (M <= 32 ? 128 : 96) ||
+        narrow > QK_GEMM_TARGET)
+        return 0;
+    p->bm = M <= 32 ? 32 : 64;
+    p->bn = QK_GEMM_NARROW_BN;
+    p->nst = M <= 32 ? 8 : 6;
+    p->nsplit = 1;
+    p->kc = K;
+    return 1;
+}
+
 extern "C" void qk_gemm_plan_epi(int M, int N, int K, int epi, qk_gemm_plan *p) {
     p->nst = 0;
     // 256 x 256 or 128 x 256 tiles (one block per CU) where they alone fill
@@ -797,22 +816,6 @@ extern "C" void qk_gemm_plan_epi(int M, int N, int K, int epi, qk_gemm_plan *p) 
         p->bn = 256;
         p->nsplit = 1;
         p->kc = (K + QK_BK - 1) / QK_BK * QK_BK;
-        return;
-    }
-    // SwiGLU of up to 64 rows: bound by the weight bytes in flight.  64-column
-    // tiles, one block per CU with a ring of 8 (6) stages and the whole k walk, so
-    // neither partials nor a reduce pass, where they give half the CUs a block.
-    // Prefill of 4 layers over 300 positions, against split 128-column tiles and a
-    // reduce: 12288 columns (192 tiles) 31 rows 320 -> 301 us, 64 rows 383 -> 354;
-    // 6144 (96 tiles) 64 rows 282 -> 272, 31 rows 231 -> 229, 2 rows 201 -> 205.
-    const int narrow = N / QK_GEMM_NARROW_BN;
-    if (epi == QK_GEMM_SWIGLU && M <= 64 && N % QK_GEMM_NARROW_BN == 0 && K % QK_BK == 0 &&
-        narrow >= (M <= 32 ? 128 : 96) && narrow <= QK_GEMM_TARGET) {
-        p->bm = M <= 32 ? 32 : 64;
-        p->bn = QK_GEMM_NARROW_BN;
-        p->nst = M <= 32 ? 8 : 6;
-        p->nsplit = 1;
-        p->kc = K;
         return;
     }
     // otherwise 32 x 128 (M <= 32) or 64 x 128 tiles on the LDS ring where the

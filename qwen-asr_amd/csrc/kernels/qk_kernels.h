@@ -343,6 +343,8 @@ void qk_gemm_plan_for(int M, int N, int K, qk_gemm_plan *p);
  * to fill the chip (its split partials need a reduce pass), and so does a
  * ROPE one (the Q|K|V product of qk_gemm_rope_launch) */
 void qk_gemm_plan_epi(int M, int N, int K, int epi, qk_gemm_plan *p);
+/* the plan of a SwiGLU product of up to 64 rows where it takes 64-column tiles: 1, else 0 */
+int qk_gemm_plan_narrow(int M, int N, int K, qk_gemm_plan *p);
 /* Y[M][N] (=, +=) (A_hi + A_lo)[M][K] . W[N][K]^T on bf16 MFMA with fp32
  * accumulation; SWIGLU writes silu(Y[:,2j]) * Y[:,2j+1] as a bf16 hi/lo
  * split [M][N/2] into out_hi/out_lo.  With nsplit > 1 only STORE is allowed

@@ -548,7 +548,7 @@ def test_one_query_splits(P, qa, gpu, sk):
 @pytest.mark.parametrize("N,K", [(8192, 64), (8192, 1024), (16384, 320), (12288, 2048)])
 def test_gemm_swiglu_narrow(P, qa, gpu, M, N, K):
     p = GemmPlan()
-    qa.lib().qk_gemm_plan_epi(M, N, K, 2, C.byref(p))
+    assert qa.lib().qk_gemm_plan_narrow(M, N, K, C.byref(p)) == 1
     assert (p.bm, p.bn, p.nsplit) == (32 if M <= 32 else 64, 64, 1)
     check_gemm(P, qa, gpu, M, N, K, p, 2)
 
