@@ -1046,6 +1046,13 @@ __global__ __launch_bounds__(256) void enc_attention(const float *qkv, float *ou
             for (int c = 0; c < 4; c++)
                 vv[t][c] = *reinterpret_cast<const float4 *>(vbase + (long)min(k0 + 16 * t + 4 * lg + c, T - 1) * stride +
                                                              4 * lq);
+        if (k0 + EA_KW > we) {                         // rows past the window weigh 0: not 0 times what they hold
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (k0 + 16 * t + 4 * lg + c >= we) vv[t][c] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
         float p[2][4];                                 // key k0 + 16 t + 4 lg + r
         float mx = -INFINITY;
 #pragma unroll

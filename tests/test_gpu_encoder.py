@@ -324,3 +324,31 @@ def test_window_attention(P, qa, gpu, T, win):
     ref = ref.view(T, H * 64)
     assert float((out.double() - ref).abs().max()) < 1e-5                # fp32 products and sums
     assert bool(((unhalve(gpu, out16, H * 64) - out.double()).abs() <= 2.0 ** -16 * out.double().abs() + 1e-9).all())
+
+
+# a window's rows stay in it: the rows of the next window that a wave's 32 keys reach
+# over weigh nothing, whatever they hold
+@pytest.mark.parametrize("T,win", [(260, 104), (100, 16), (97, 33), (301, 150)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_window_attention_nonfinite_rows(P, qa, gpu, T, win, bad):
+    lib, H = qa.lib(), 2
+    lib.qk_enc_attention_launch.argtypes = [C.c_void_p] * 3 + [C.c_int] * 4 + [C.c_float, C.c_void_p]
+    g = gpu.Generator(device="cuda").manual_seed(T)
+    qkv = gpu.randn(T, 3, H, 64, generator=g, device="cuda")
+
+    def run(x):
+        out = gpu.empty(T, H * 64, device="cuda")
+        qa.check(lib.qk_enc_attention_launch(x.data_ptr(), out.data_ptr(), None, T, H, 64, win, 0.125, None), "attn")
+        gpu.cuda.synchronize()
+        return out
+    clean = run(qkv)
+    for w0 in range(0, T, win):
+        w1 = min(T, w0 + win)
+        x = qkv.clone()
+        x[w0:w1] = bad
+        out = run(x)
+        assert gpu.equal(out[:w0], clean[:w0]) and gpu.equal(out[w1:], clean[w1:]), w0
+        # an infinite value of the window's last key weighs more than 0 in each of its rows
+        x = qkv.clone()
+        x[w1 - 1, 2] = float("inf")
+        assert bool((run(x)[w0:w1] == float("inf")).all()), w0
