@@ -422,27 +422,22 @@ __global__ __launch_bounds__(256) void gemm_hilo(const uint16_t *__restrict__ ah
     }
 }
 
-// silu(g) u: swiglu1 with the hardware exponential, whose error (|g| ulp of e^-g,
-// weighted by e^-g / (1 + e^-g)) stays two orders below the halves' 2^-17
-__device__ __forceinline__ float gemm_swiglu(float g, float u) {
-    return (g * __builtin_amdgcn_rcpf(1.0f + __expf(-g))) * u;
-}
-
 // The epilogue of a tile held as acc[i][j][r]: row mr + 16 i + r, column nc + 16 j
 // (nc = ... + (lane & 15), whole 16-column tiles inside N).  ADD reads every old
 // value of a row tile before it stores one: written as y += v the compiler must
 // keep each load behind the store before it, a memory latency per value (8191 rows
-// by 1024 columns: K 2048 88 -> 72 us, K 3072 106 -> 101).  SWIGLU: the four lanes of a quad hold
-// the gates and ups of two outputs; lanes 0, 1 store the hi and the lo word of one
-// row's two outputs, lanes 2, 3 those of the next row
-// (401 x 6144 x 1024: 21.7 -> 20.0 us against 2-byte stores from every second lane
-// and scalar roundings).
+// by 1024 columns: K 2048 88 -> 72 us, K 3072 106 -> 101).  SWIGLU: the lanes of a
+// pair hold the gates and the ups of one output column; the even lane computes row
+// r's output, the odd one row r + 1's (computed in both lanes 401 x 6144 x 1024 took
+// 18.0 us, 17.0 so: the exponentials are what the epilogue spends).  Of a quad's two
+// columns lanes 0, 1 store their row's word of hi halves, lanes 2, 3 that of lo halves.
 template <int EPI, int TM, int TN>
 __device__ __forceinline__ void gemm_store(const f32x4 (&acc)[TM][TN], int mr, int nc, int M, int N, float *y,
                                            uint16_t *ohi, uint16_t *olo) {
     if constexpr (EPI == QK_GEMM_SWIGLU) {
         const int q = threadIdx.x & 3;
-        uint16_t *o = (q & 1) ? olo : ohi;
+        const bool odd = q & 1;
+        uint16_t *o = q < 2 ? ohi : olo;
         const int oc = (nc - q) / 2;                      // the quad's first output column
 #pragma unroll
         for (int i = 0; i < TM; i++)
@@ -450,17 +445,14 @@ __device__ __forceinline__ void gemm_store(const f32x4 (&acc)[TM][TN], int mr, i
             for (int j = 0; j < TN; j++)
 #pragma unroll
                 for (int r = 0; r < 4; r += 2) {
-                    float s[2], t[2];
-#pragma unroll
-                    for (int k = 0; k < 2; k++) {
-                        const float v = acc[i][j][r + k], p = dpp_read<0xB1>(v);
-                        s[k] = gemm_swiglu((q & 1) ? p : v, (q & 1) ? v : p);
-                        t[k] = dpp_read<0x4E>(s[k]);       // the other pair's output
-                    }
+                    const float v0 = acc[i][j][r], v1 = acc[i][j][r + 1];
+                    const float p = dpp_read<0xB1>(odd ? v0 : v1);       // the partner's gate or up
+                    const float s = swiglu1(odd ? p : v0, odd ? v1 : p);
+                    const float t = dpp_read<0x4E>(s);                   // the other pair's output
                     uint32_t h, l;
-                    bf16_split2(q < 2 ? s[0] : t[1], q < 2 ? t[0] : s[1], h, l);
-                    const int m = mr + 16 * i + r + (q >> 1);
-                    if (m < M) *reinterpret_cast<uint32_t *>(o + (size_t)m * (N / 2) + oc + 8 * j) = (q & 1) ? l : h;
+                    bf16_split2(q < 2 ? s : t, q < 2 ? t : s, h, l);
+                    const int m = mr + 16 * i + r + (q & 1);
+                    if (m < M) *reinterpret_cast<uint32_t *>(o + (size_t)m * (N / 2) + oc + 8 * j) = q < 2 ? h : l;
                 }
     } else {
 #pragma unroll

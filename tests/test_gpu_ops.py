@@ -571,3 +571,46 @@ def test_linear_qkv_edges(P, qa, gpu, hidden, qd, kvd):
         exp = P.bf16_to_f32(W).astype(np.float64) @ x.astype(np.float64)
         bound = 8 * hidden * 2.0 ** -24 * (np.abs(P.bf16_to_f32(W)) @ np.abs(x)) + 1e-12
         assert np.all(np.abs(y[:-1] - exp) <= bound) and y[-1] == 7.0
+
+
+# the SwiGLU epilogues over the gates of the whole range, with products that are exact
+# (one 1 per row of A), on every kernel that has one.  A value within 2^-21 of silu(g)
+# (exponential and reciprocal 1 ulp each, half an ulp of 1 + e^-g and of two products:
+# 3.5 * 2^-23) is stored as its halves, which do not decrease with it.
+@pytest.mark.parametrize("M,N,K,bm,nst,ns", [(32, 8192, 64, 32, 8, 1), (64, 8192, 64, 64, 6, 1), (300, 6144, 64, 64, 4, 1),
+                                             (401, 6144, 128, 64, 4, 1), (600, 8192, 64, 128, 3, 1),
+                                             (1000, 16384, 64, 256, 0, 1), (31, 6144, 320, 32, 4, 5),
+                                             (100, 1000, 64, 64, 0, 1)])
+def test_gemm_swiglu_gate_range(P, qa, gpu, M, N, K, bm, nst, ns):
+    lib, p = qa.lib(), GemmPlan()
+    if not lib.qk_gemm_plan_narrow(M, N, K, C.byref(p)):
+        lib.qk_gemm_plan_epi(M, N, K, 2, C.byref(p))
+    assert (p.bm, p.nst, p.nsplit) == (bm, nst, ns), (p.bm, p.nst, p.nsplit)
+    A = np.zeros((M, K), np.float32)
+    A[:, 0] = A[:, 1] = 1.0
+    W = np.zeros((N, K), np.float32)
+    W[0::2, 0] = np.linspace(-75.0, 30.0, N // 2)                 # gates
+    W[1::2, 1] = np.linspace(0.5, 1.5, N // 2)                    # ups
+    hi, Wb = P.f32_to_bf16(A), P.f32_to_bf16(W)
+    dh, dl = dev(gpu, hi.view(np.int16)), gpu.zeros((M, K), dtype=gpu.int16, device="cuda")
+    dW = dev(gpu, Wb.view(np.int16))
+    oh, ol = (gpu.zeros((M, N // 2), dtype=gpu.int16, device="cuda") for _ in range(2))
+    lib.qk_gemm_launch.argtypes = [C.c_void_p] * 3 + [C.c_int] * 3 + [C.c_void_p, C.c_int] + [C.c_void_p] * 4
+    lib.qk_gemm_reduce_launch.argtypes = [C.c_void_p] + [C.c_int] * 4 + [C.c_void_p] * 4
+    part = gpu.empty((p.nsplit, M, N), dtype=gpu.float32, device="cuda") if p.nsplit > 1 else None
+    qa.check(lib.qk_gemm_launch(ptr(dh), ptr(dl), ptr(dW), M, N, K, C.byref(p), 0 if p.nsplit > 1 else 2,
+                                ptr(part) if p.nsplit > 1 else None, ptr(oh), ptr(ol), None), "gemm")
+    if p.nsplit > 1:
+        qa.check(lib.qk_gemm_reduce_launch(ptr(part), p.nsplit, M, N, 2, None, ptr(oh), ptr(ol), None), "reduce")
+    gpu.cuda.synchronize()
+    w = P.bf16_to_f32(Wb).astype(np.float64)
+    g, u = w[0::2, 0], w[1::2, 1]
+    y = g / (1.0 + np.exp(-g)) * u
+
+    def halves(v):
+        v = v.astype(np.float32)
+        h = P.bf16_to_f32(P.f32_to_bf16(v))
+        return h.astype(np.float64) + P.bf16_to_f32(P.f32_to_bf16(v - h))
+    e = 2.0 ** -21 * np.abs(y)
+    got = P.bf16_to_f32(host(oh).view(np.uint16)).astype(np.float64) + P.bf16_to_f32(host(ol).view(np.uint16))
+    assert np.all(got >= halves(y - e)) and np.all(got <= halves(y + e)), float(np.max(np.abs(got - y) / np.abs(y).clip(1e-30)))
