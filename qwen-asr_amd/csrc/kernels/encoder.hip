@@ -40,14 +40,23 @@ __device__ __forceinline__ f32x4 enc_mfma(float a, float b, f32x4 c) {
 }
 
 // GELU, tanh form (qwen_gelu, qwen_asr_kernels.c:886-893): 0.5 v (1 + tanh u) =
-// v / (1 + e^(-2u)), with no cancellation for negative u.  The hardware exponential
-// and reciprocal: the error of e^(-2u) (|2u| ulp) is weighted by e / (1 + e)^2, at
-// most 0.4 ulp of v, as tanhf's.  (With tanhf or expf the serial chains of a GEMM
-// tile's 32 values per lane took as long as its k walk.)
+// v / (1 + e^(-2u)), with no cancellation for negative u.  No error of its own but
+// the hardware exponential's and the last rounding: the exponent -2u log2(e) is
+// hi + lo, the quotient is corrected by the remainder of v - (1 + e) q, whose 1 + e
+// counts with what its rounding lost.  Error against 64 bits (root mean square,
+// relative): at most 3.0e-8 for v > 0 and 1.2e-7 on [-2, 0]; the fp32 expression with
+// tanhf has 4.3e-8 and 2.2e-7, and cancels below.  Beyond 9 in size the expression is
+// v or 0, infinities and NaN as there.  268 M values 161 us, with tanhf 214.
 __device__ __forceinline__ float enc_gelu(float v) {
-    const float x3 = v * v * v;
-    const float inner = 0.7978845608028654f * (v + 0.044715f * x3);
-    return v * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * inner));
+    constexpr double c = -2.0 * 0.7978845608028654 * 1.4426950408889634;
+    constexpr float c_hi = (float)c, c_lo = (float)(c - (double)c_hi);
+    const float w = v * fmaf(0.044715f, v * v, 1.0f), hi = w * c_hi;
+    const float lo = fmaf(w, c_lo, fmaf(w, c_hi, -hi));
+    float e = __builtin_amdgcn_exp2f(hi);
+    e = fmaf(e, 0.693147181f * lo, e);
+    const float d = 1.0f + e, lost = e - (d - 1.0f), r = __builtin_amdgcn_rcpf(d), q = v * r;
+    const float y = fmaf(fmaf(-lost, q, fmaf(-d, q, v)), r, q);
+    return fabsf(v) > 9.0f ? v * __builtin_amdgcn_fmed3f(v, 0.0f, 1.0f) : y;
 }
 
 // ---------------------------------------------------------------------------
