@@ -222,11 +222,19 @@ static int up(float **dst, const float *src, size_t n) {
     return 0;
 }
 
-/* the gathering products' copy of a bf16 matrix [rows][ch * h] */
-static int tiled(qwen_hip_encoder *e, const enc_mat *m, uint16_t **t, int rows, int ch, int h) {
-    if (!m->b16) return 0;
-    if (!*t) QK_TRY(dmalloc((void **)t, (size_t)rows * ch * h * 2));
-    return qk_enc_tile_weights_launch(m->b16, *t, rows, ch, h, e->stream);
+/* a stem matrix [rows][ch * h] and, where it is bf16-valued, the gathering
+ * products' copy of it: the copy is there only where it is the matrix's own */
+static int up_stem(qwen_hip_encoder *e, enc_mat *m, uint16_t **t, const float *src, int rows, int ch, int h) {
+    const size_t n = (size_t)rows * ch * h;
+    if (!src) { qk_set_err("encoder weight pointer is NULL"); return QWEN_HIP_EINVAL; }
+    int rc = up_mat(m, n, 0, src, n, bf16_exact(src, n));
+    if (!rc && m->b16) {
+        if (!*t) rc = dmalloc((void **)t, n * 2);
+        if (!rc) rc = qk_enc_tile_weights_launch(m->b16, *t, rows, ch, h, e->stream);
+        if (!rc && hipStreamSynchronize(e->stream) != hipSuccess) rc = QWEN_HIP_EDEVICE;
+    }
+    if (rc || !m->b16) dfree((void **)t);
+    return rc;
 }
 
 int qwen_hip_encoder_load_layer(qwen_hip_encoder *e, int l, const qwen_hip_enc_layer_weights *w) {
@@ -271,7 +279,7 @@ int qwen_hip_encoder_load_stem(qwen_hip_encoder *e, const qwen_hip_enc_stem_weig
     for (int oc = 0; oc < ENC_CH; oc++) memcpy(c1 + oc * ENC_K1, w->conv1_w + oc * 9, 9 * sizeof(float));
     QK_TRY(up(&e->c1w, c1, ENC_CH * ENC_K1));
     QK_TRY(up(&e->c1b, w->conv1_b, ENC_CH));
-    const size_t k2 = (size_t)ENC_CH * ENC_K2, ko = d * ENC_CH * 16;
+    const size_t k2 = (size_t)ENC_CH * ENC_K2;
     /* conv2 / conv3 [480][480][3][3]: columns reordered tap-major (k = tap *
      * 480 + ic) to match the channel-last stem activations */
     if (!w->conv2_w || !w->conv3_w) { qk_set_err("encoder weight pointer is NULL"); return QWEN_HIP_EINVAL; }
@@ -279,23 +287,20 @@ int qwen_hip_encoder_load_stem(qwen_hip_encoder *e, const qwen_hip_enc_stem_weig
     if (!tm) { qk_set_err("out of host memory"); return QWEN_HIP_ENOMEM; }
     const float *cw[2] = {w->conv2_w, w->conv3_w};
     enc_mat *cm[2] = {&e->c2w, &e->c3w};
+    uint16_t **ct[2] = {&e->c2t, &e->c3t};
     int rc = 0;
     for (int i = 0; i < 2 && !rc; i++) {
         for (size_t oc = 0; oc < ENC_CH; oc++)
             for (size_t ic = 0; ic < ENC_CH; ic++)
                 for (size_t tap = 0; tap < 9; tap++)
                     tm[oc * ENC_K2 + tap * ENC_CH + ic] = cw[i][oc * ENC_K2 + ic * 9 + tap];
-        rc = up_mat(cm[i], k2, 0, tm, k2, bf16_exact(tm, k2));
+        rc = up_stem(e, cm[i], ct[i], tm, ENC_CH, ENC_K2, 1);
     }
     free(tm);
     QK_TRY(rc);
     QK_TRY(up(&e->c2b, w->conv2_b, ENC_CH));
     QK_TRY(up(&e->c3b, w->conv3_b, ENC_CH));
-    QK_TRY(up_mat(&e->cow, ko, 0, w->conv_out_w, ko, w->conv_out_w && bf16_exact(w->conv_out_w, ko)));
-    QK_TRY(tiled(e, &e->c2w, &e->c2t, ENC_CH, ENC_K2, 1));
-    QK_TRY(tiled(e, &e->c3w, &e->c3t, ENC_CH, ENC_K2, 1));
-    QK_TRY(tiled(e, &e->cow, &e->cowt, (int)d, ENC_CH, 16));
-    QK_HIP(hipStreamSynchronize(e->stream));
+    QK_TRY(up_stem(e, &e->cow, &e->cowt, w->conv_out_w, (int)d, ENC_CH, 16));
     QK_TRY(up(&e->lnpw, w->ln_post_w, d));
     QK_TRY(up(&e->lnpb, w->ln_post_b, d));
     QK_TRY(up_mat(&e->p1w, d * d, 0, w->proj1_w, d * d, w->proj1_w && bf16_exact(w->proj1_w, d * d)));
@@ -430,7 +435,7 @@ static int reserve_cols(qwen_hip_encoder *e, int chunks) {
 static int ring_ok(const qwen_hip_encoder *e) {
     const qwen_hip_enc_config *c = &e->cfg;
     if (c->d_model > 1024 || c->ffn_dim % 32 || c->output_dim % 4) return 0;
-    int ok = e->c2w.b16 && e->c3w.b16 && e->cow.b16 && e->p1w.b16 && e->p2w.b16;
+    int ok = e->c2t && e->c3t && e->cowt && e->p1w.b16 && e->p2w.b16;
     for (int l = 0; l < c->layers; l++)
         ok = ok && e->L[l].wqkv.b16 && e->L[l].wo.b16 && e->L[l].fc1w.b16 && e->L[l].fc2w.b16;
     return ok;

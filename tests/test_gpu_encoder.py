@@ -396,3 +396,23 @@ def test_gelu_precision(P, qa, gpu):
     assert e[0] == 0 and e[1] == 9 and e[2] == f32(9.5) and e[5] == f32(1e30) and e[7] == np.inf
     assert np.all(np.abs(e[[3, 4, 6]]) < 1e-27) and np.isnan(e[8]) and np.isnan(e[9])     # -inf * 0 is the reference's
     assert np.allclose(e[10:], f32([5e-31, -5e-31]), rtol=1e-6, atol=0)
+
+
+def test_encoder_stem_reload_that_fails(P, qa, gpu):
+    """A stem reload that fails at conv2's bias leaves the new conv1, conv2 and
+    conv3 matrices beside the old rest: both forms of a matrix, as loaded and as
+    the products read it, are the same one."""
+    cfg = qa.EncConfig(128, 2, 2, 64, 256, 96, 100, 200)
+    a, b = P.SynthEncoder(cfg, seed=5), P.SynthEncoder(cfg, seed=6)
+    mel = P.synth_mel(250, 5, 3)
+    e = load(qa, cfg, a)
+    arrs = [np.ascontiguousarray(x, np.float32) for x in b.stem]
+    w = qa.EncStemWeights(*[x.ctypes.data for x in arrs])
+    w.conv2_b = None
+    assert qa.lib().qwen_hip_encoder_load_stem(e.h, C.byref(w)) < 0
+    out = e.forward(mel)
+    a.stem[0:3], a.stem[4] = b.stem[0:3], b.stem[4]
+    m = load(qa, cfg, a)
+    assert np.array_equal(out, m.forward(mel))
+    e.close()
+    m.close()
