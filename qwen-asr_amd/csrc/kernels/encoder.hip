@@ -840,9 +840,10 @@ extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_
            : (!a->C == !a->out || a->pe || a->add || (a->gelu ? !a->out : !a->C) || (gather && a->C)))
         return QWEN_HIP_EINVAL;
     if (gather && (a->K != a->taps * QK_ENC_CH || (a->taps != 9 && a->taps != a->in_h) || a->taps > 32 || !a->zero ||
-                   a->in_h <= 0 || a->in_w <= 0 || (a->taps == 9 && (a->col_h <= 0 || a->col_w <= 0))))
+                   a->in_h <= 0 || a->in_w <= 0 || (!ln && a->N % 32) ||
+                   (a->taps == 9 && (a->col_h <= 0 || a->col_w <= 0 || (long)a->chunks * a->col_h * a->col_w < a->M))))
         return QWEN_HIP_EINVAL;
-    if (a->valid > 0 && (a->col_h <= 0 || a->col_w <= 0)) return QWEN_HIP_EINVAL;
+    if (a->valid > 0 && (!gather || ln || a->col_h <= 0 || a->col_w <= 0)) return QWEN_HIP_EINVAL;   // stem layers only
     qk_enc_ring_args g = *a;
     if (!ln && !gather && enc_ring_narrow(a->M, a->N, a->K)) {
         const dim3 grid((a->N + 63) / 64, (a->M + 31) / 32);

@@ -434,7 +434,7 @@ int qk_enc_attention_launch(const float *qkv, float *out, uint16_t *out16, int T
  * col_h x col_w, with `zero` (64 zeros) outside; taps == in_h is pixel
  * column m % in_w of chunk m / in_w, top to bottom.
  * Result, one of: C fp32 [M][N] (+ bias); out halves [M][2 N] of the GELU (bias
- * added before; valid > 0: row m's positions ow >= valid of the last chunk are 0); with
+ * added before; gathered rows, valid > 0: positions ow >= valid of the last chunk are 0); with
  * ln_w, x = C (+= when add) product + bias + pe[m % pe_rows] and out = halves of
  * LayerNorm(x) (N <= 1024).  ws: split-K partials (always used with ln_w, then at
  * least M N floats).  kc, split and ws of the struct are set by the launcher. */

@@ -176,3 +176,28 @@ def test_linear_op_workspace_advice_case(qa):
     lib.qk_linear_ws_bytes.restype = C.c_size_t
     assert lib.qk_linear_ws_bytes(1024, 1024, 4096) == 4 * 1024 * 1024      # x halves only
     assert lib.qk_linear_ws_bytes(1024, 1024, 4096) <= lib.qwen_hip_linear_noalloc_max_bytes()
+
+
+class RingArgs(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("A", "W", "zero")] + [(n, C.c_int) for n in (
+        "M", "N", "K", "taps", "in_h", "in_w", "col_h", "col_w", "chunks", "valid")] + [
+        ("bias", C.c_void_p), ("pe", C.c_void_p), ("pe_rows", C.c_int), ("gelu", C.c_int), ("add", C.c_int),
+        ("C", C.c_void_p), ("out", C.c_void_p), ("ln_w", C.c_void_p), ("ln_b", C.c_void_p), ("ln_eps", C.c_float),
+        ("ws", C.c_void_p), ("kc", C.c_int), ("split", C.c_int)]
+
+
+@pytest.mark.parametrize("change", [
+    dict(valid=3, col_h=4, col_w=5, chunks=1),       # padded positions exist only in the stem's GELU products
+    dict(valid=3, col_h=4, col_w=5, chunks=1, ln_w=1, ln_b=1, C=1, gelu=0),
+    dict(N=66), dict(K=72), dict(K=0), dict(M=0), dict(A=None), dict(W=None), dict(C=1), dict(gelu=0),
+    dict(ln_w=1, ln_b=1, C=1, N=1028), dict(taps=9), dict(taps=9, K=9 * 480, zero=1), dict(add=1),
+    dict(taps=9, K=9 * 480, zero=1, in_h=8, in_w=10, col_h=4, col_w=5, chunks=1, N=36),       # whole 32-channel groups
+    dict(taps=9, K=9 * 480, zero=1, in_h=8, in_w=10, col_h=4, col_w=5, chunks=1, M=21)])      # rows past the pixels
+def test_ring_product_refusals(qa, change):
+    """qk_enc_ring_launch refuses what its kernels do not do, before anything
+    is launched (the pointers are never followed)."""
+    lib = qa.lib()
+    lib.qk_enc_ring_launch.argtypes = [C.c_void_p, C.c_void_p, C.c_long, C.c_void_p]
+    a = dict(A=1, W=1, M=20, N=64, K=64, gelu=1, out=1)
+    a.update(change)
+    assert lib.qk_enc_ring_launch(C.byref(RingArgs(**a)), C.c_void_p(1), 1 << 20, None) == -1
