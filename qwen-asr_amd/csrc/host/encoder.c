@@ -602,17 +602,31 @@ int qwen_hip_encoder_forward(qwen_hip_encoder *e, const float *mel, int mel_fram
     return T;
 }
 
+/* whether a mel of this memory type and device is read where it is: device
+ * memory of the encoder's own device.  A kernel cannot be relied on to reach
+ * another device's memory or the host's; a copy can, so that is copied first. */
+int qk_enc_mel_in_place(int type, int mem_device, int device) {
+    return type == hipMemoryTypeDevice && mem_device == device;
+}
+
+static int mel_in_place(const qwen_hip_encoder *e, const float *mel) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, mel) != hipSuccess) {
+        (void)hipGetLastError();   /* memory the runtime does not know; the launches check this error */
+        return 0;
+    }
+    return qk_enc_mel_in_place(at.type, at.device, e->device);
+}
+
 int qwen_hip_encoder_forward_device(qwen_hip_encoder *e, const float *d_mel, int mel_frames, const float **d_out) {
     int rc = ready(e, mel_frames);
     if (rc) return rc;
     if (!d_mel || !d_out) { qk_set_err("encoder: NULL mel or output"); return QWEN_HIP_EINVAL; }
     int T = 0;
-    if (ring_ok(e)) {
-        QK_TRY(run_ring(e, d_mel, mel_frames, &T));
-    } else {
+    const int ring = ring_ok(e), in_place = ring && mel_in_place(e, d_mel);
+    if (!in_place)
         QK_HIP(hipMemcpyAsync(e->mel, d_mel, (size_t)ENC_MEL * mel_frames * 4, hipMemcpyDeviceToDevice, e->stream));
-        QK_TRY(run_general(e, mel_frames, &T));
-    }
+    QK_TRY(ring ? run_ring(e, in_place ? d_mel : e->mel, mel_frames, &T) : run_general(e, mel_frames, &T));
     QK_HIP(hipStreamSynchronize(e->stream));
     *d_out = e->out;
     return T;

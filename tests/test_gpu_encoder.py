@@ -416,3 +416,17 @@ def test_encoder_stem_reload_that_fails(P, qa, gpu):
     assert np.array_equal(out, m.forward(mel))
     e.close()
     m.close()
+
+
+def test_encoder_mel_in_host_memory(P, qa, gpu):
+    """a mel in pinned host memory: copied, with the same result"""
+    cfg = qa.EncConfig(128, 2, 2, 64, 256, 96, 100, 200)
+    e = qa.Encoder(cfg, 0)
+    e.load_synthetic(5, 0.02)
+    mel = P.synth_mel(250, 5, 3)
+    want = e.forward(mel)
+    h = gpu.empty(128, 250, pin_memory=True)
+    h.copy_(gpu.from_numpy(mel))
+    T, p = e.forward_device(h.data_ptr(), 250)
+    assert np.array_equal(d2h(p, (T, cfg.output_dim)), want)
+    e.close()

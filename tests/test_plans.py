@@ -201,3 +201,11 @@ def test_ring_product_refusals(qa, change):
     a = dict(A=1, W=1, M=20, N=64, K=64, gelu=1, out=1)
     a.update(change)
     assert lib.qk_enc_ring_launch(C.byref(RingArgs(**a)), C.c_void_p(1), 1 << 20, None) == -1
+
+
+def test_mel_read_in_place(qa):
+    """forward_device reads the mel where it is only in device memory of the
+    encoder's own device; host (1), managed (3), unregistered (0) memory and
+    another device's are copied."""
+    f = qa.lib().qk_enc_mel_in_place
+    assert [(t, m, d) for t in range(4) for m in (0, 1) for d in (0, 1) if f(t, m, d)] == [(2, 0, 0), (2, 1, 1)]
