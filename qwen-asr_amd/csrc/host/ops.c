@@ -127,13 +127,18 @@ int qwen_hip_linear_nobias_bf16(float *y, const float *x, const uint16_t *W, int
 }
 
 /* Rows of up to 2048 columns, which a wave holds whole; longer ones keep their
- * three launches of the k-split GEMV, and other widths are refused there. */
-static int qkv_one_launch(int in_dim) { return in_dim > 0 && in_dim % 8 == 0 && in_dim <= 2048; }
+ * three launches of the k-split GEMV, and other widths are refused there.  A
+ * launch counts its threads in 32 bits, 32 of them to a row here and 16 or fewer
+ * there, so more rows go there too. */
+static int qkv_one_launch(int in_dim, int q_dim, int kv_dim) {
+    return in_dim > 0 && in_dim % 8 == 0 && in_dim <= 2048 && q_dim > 0 && kv_dim > 0 &&
+           (long)q_dim + 2L * kv_dim <= 1L << 26;
+}
 
 int qwen_hip_linear_nobias_bf16_qkv(float *q, float *k, float *v, const float *x, const uint16_t *Wq,
                                     const uint16_t *Wk, const uint16_t *Wv, int in_dim, int q_dim, int kv_dim,
                                     hipStream_t s) {
-    if (q && k && v && x && Wq && Wk && Wv && q_dim > 0 && kv_dim > 0 && qkv_one_launch(in_dim)) {
+    if (q && k && v && x && Wq && Wk && Wv && qkv_one_launch(in_dim, q_dim, kv_dim)) {
         qk_gemv3_args t = {.W = {Wq, Wk, Wv}, .y = {q, k, v}, .rows = {q_dim, kv_dim, kv_dim}, .K = in_dim, .x = x};
         return qk_gemv3_launch(&t, s);
     }

@@ -439,8 +439,12 @@ static void gemv3_dispatch(const qk_gemv3_args *t, hipStream_t s) {
 
 extern "C" int qk_gemv3_launch(const qk_gemv3_args *t, hipStream_t s) {
     if (!t || !t->x || t->K <= 0 || (t->K & 7) || t->K > 4 * 512) return QWEN_HIP_EINVAL;
-    for (int i = 0; i < 3; i++)
-        if (!t->W[i] || !t->y[i] || t->rows[i] <= 0 || t->rows[i] > (1 << 28)) return QWEN_HIP_EINVAL;
+    long rows = 0;
+    for (int i = 0; i < 3; i++) {
+        if (!t->W[i] || !t->y[i] || t->rows[i] <= 0) return QWEN_HIP_EINVAL;
+        rows += t->rows[i];
+    }
+    if (rows > 1L << 26) return QWEN_HIP_EINVAL;          // 32 threads to a row, 2^32 to a launch
     switch ((t->K + 511) / 512) {
     case 1: gemv3_dispatch<1>(t, s); break;
     case 2: gemv3_dispatch<2>(t, s); break;

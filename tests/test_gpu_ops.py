@@ -614,3 +614,18 @@ def test_gemm_swiglu_gate_range(P, qa, gpu, M, N, K, bm, nst, ns):
     e = 2.0 ** -21 * np.abs(y)
     got = P.bf16_to_f32(host(oh).view(np.uint16)).astype(np.float64) + P.bf16_to_f32(host(ol).view(np.uint16))
     assert np.all(got >= halves(y - e)) and np.all(got <= halves(y + e)), float(np.max(np.abs(got - y) / np.abs(y).clip(1e-30)))
+
+
+# more rows than one launch of 256 threads to 8 rows can hold: the separate products
+def test_linear_qkv_many_rows(P, qa, gpu):
+    K, qd, kvd = 8, (1 << 27) + 16, 8
+    W = gpu.full((qd, K), 0.25, dtype=gpu.bfloat16, device="cuda")
+    W[-1], W[1 << 26] = 0.5, 2.0
+    x = gpu.arange(1, K + 1, dtype=gpu.float32, device="cuda")
+    q, k, v = (gpu.empty(n, device="cuda") for n in (qd, kvd, kvd))
+    qa.check(qa.lib().qwen_hip_linear_nobias_bf16_qkv(ptr(q), ptr(k), ptr(v), ptr(x), ptr(W), ptr(W), ptr(W), K, qd,
+                                                      kvd, None), "qkv")
+    gpu.cuda.synchronize()
+    want = gpu.full((qd,), 9.0, device="cuda")                    # 36 / 4
+    want[-1], want[1 << 26] = 18.0, 72.0
+    assert gpu.equal(q, want) and gpu.equal(k, want[:kvd]) and gpu.equal(v, want[:kvd])
