@@ -924,6 +924,10 @@ static bool al16(const void *a, const void *b = nullptr, const void *c = nullptr
     return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0;
 }
 
+// rows up to which a row's 16 or 32 threads are launched at once: a launch counts its
+// threads in 32 bits
+#define VEC_ROWS (1L << 26)
+
 static unsigned grid_for(long items) {
     const long blocks = (items + 255) / 256;
     return (unsigned)(blocks < 65536 ? blocks : 65536);
@@ -1031,7 +1035,7 @@ __global__ __launch_bounds__(256) void rms_norm_head_vec(float4 *x, const float4
 extern "C" int qk_rms_norm_per_head_launch(float *x, const float *w, int S, int nh, int hd, float eps, hipStream_t s) {
     if (S <= 0 || nh <= 0 || hd <= 0) return QWEN_HIP_EINVAL;
     const long rows = (long)S * nh;
-    if (hd == 128 && al16(x, w) && rows <= 0x7fffffffL)
+    if (hd == 128 && al16(x, w) && rows <= VEC_ROWS)
         rms_norm_head_vec<<<(unsigned)((rows + 7) / 8), 256, 0, s>>>(reinterpret_cast<float4 *>(x),
                                                                      reinterpret_cast<const float4 *>(w), rows, eps);
     else
@@ -1068,7 +1072,7 @@ __global__ __launch_bounds__(256) void rope_vec(float4 *x, const float4 *cv, con
 extern "C" int qk_rope_launch(float *x, const float *cos_v, const float *sin_v, int S, int nh, int hd, hipStream_t s) {
     if (S <= 0 || nh <= 0 || hd <= 0 || (hd & 1)) return QWEN_HIP_EINVAL;
     const long rows = (long)S * nh;
-    if (hd == 128 && al16(x, cos_v, sin_v) && rows <= 0x7fffffffL)
+    if (hd == 128 && al16(x, cos_v, sin_v) && rows <= VEC_ROWS)
         rope_vec<<<(unsigned)((rows + 15) / 16), 256, 0, s>>>(reinterpret_cast<float4 *>(x),
                                                               reinterpret_cast<const float4 *>(cos_v),
                                                               reinterpret_cast<const float4 *>(sin_v), nh, rows);

@@ -629,3 +629,26 @@ def test_linear_qkv_many_rows(P, qa, gpu):
     want = gpu.full((qd,), 9.0, device="cuda")                    # 36 / 4
     want[-1], want[1 << 26] = 18.0, 72.0
     assert gpu.equal(q, want) and gpu.equal(k, want[:kvd]) and gpu.equal(v, want[:kvd])
+
+
+# more rows than a launch of the vector forms holds threads for (2^32 in all, 32 to a
+# row of the norm and 16 of the rotation): the scalar forms
+@pytest.mark.parametrize("what,S", [("norm", (1 << 15) + 1), ("rope", (1 << 16) + 1)])
+def test_head_ops_many_rows(P, qa, gpu, what, S):
+    lib, nh = qa.lib(), 4096
+    if gpu.cuda.mem_get_info()[0] < S * nh * 512 + (8 << 30):
+        pytest.skip("needs the memory of S * nh rows")
+    x = gpu.ones(S * nh, 128, device="cuda")
+    if what == "norm":
+        w = gpu.full((128,), 2.0, device="cuda")
+        qa.check(lib.qwen_hip_rms_norm_per_head(ptr(x), ptr(w), S, nh, 128, 1e-6, None))
+        want = 2.0
+    else:
+        c, s = gpu.full((S, 128), 2.0, device="cuda"), gpu.full((S, 128), -1.0, device="cuda")
+        qa.check(lib.qwen_hip_apply_rope_neox(ptr(x), ptr(c), ptr(s), S, nh, 128, None))
+        want = 3.0                                    # 1 * 2 - 1 * -1, and 1 in the other half
+    gpu.cuda.synchronize()
+    wrong = int(((x[:, 0] - want).abs() > 1e-4).sum()) + int(((x[:, 127] - (2.0 if what == "norm" else 1.0)).abs() > 1e-4).sum())
+    del x
+    gpu.cuda.empty_cache()
+    assert wrong == 0
