@@ -52,7 +52,7 @@ struct qwen_hip_encoder {
     int stem_loaded;
     enc_layer L[QWEN_HIP_ENC_MAX_LAYERS];
     /* activations, sized for cap_chunks chunks */
-    int cap_chunks, cap_cols;
+    int cap_chunks, cap_general;
     float *mel, *cols, *c1, *c2, *c3, *rows, *x, *xn, *qkv, *att, *mid, *out;
     float *gws;   /* split-K partials of the GEMMs (gws_elems floats) */
     long gws_elems;
@@ -102,7 +102,7 @@ static void act_free(qwen_hip_encoder *e) {
                   (void **)&e->rows, (void **)&e->x, (void **)&e->xn, (void **)&e->qkv, (void **)&e->att,
                   (void **)&e->mid, (void **)&e->out, (void **)&e->gws};
     for (size_t i = 0; i < sizeof(b) / sizeof(b[0]); i++) dfree(b[i]);
-    e->cap_chunks = e->cap_cols = 0;
+    e->cap_chunks = e->cap_general = 0;
 }
 
 void qwen_hip_encoder_destroy(qwen_hip_encoder *e) {
@@ -400,7 +400,6 @@ static int reserve(qwen_hip_encoder *e, int chunks, int tokens) {
     if (!rc) rc = dmalloc((void **)&e->c1, (size_t)ENC_CH * n1 * 4);
     if (!rc) rc = dmalloc((void **)&e->c2, (size_t)ENC_CH * n2 * 4);
     if (!rc) rc = dmalloc((void **)&e->c3, (size_t)ENC_CH * n3 * 4);
-    if (!rc) rc = dmalloc((void **)&e->rows, T * ENC_CH * 16 * 4);
     if (!rc) rc = dmalloc((void **)&e->x, T * d * 4);
     if (!rc) rc = dmalloc((void **)&e->xn, T * d * 4);
     if (!rc) rc = dmalloc((void **)&e->qkv, T * 3 * d * 4);
@@ -414,18 +413,20 @@ static int reserve(qwen_hip_encoder *e, int chunks, int tokens) {
     return 0;
 }
 
-/* the im2col patches of the general path */
-static int reserve_cols(qwen_hip_encoder *e, int chunks) {
-    if (chunks <= e->cap_cols) return 0;
+/* the im2col patches and token rows of the general path */
+static int reserve_general(qwen_hip_encoder *e, int chunks) {
+    if (chunks <= e->cap_general) return 0;
     QK_HIP(hipStreamSynchronize(e->stream));
     dfree((void **)&e->cols);
-    e->cap_cols = 0;
+    dfree((void **)&e->rows);
+    e->cap_general = 0;
     const size_t w1 = conv_out(e->cfg.chunk_size), w2 = conv_out(w1), w3 = conv_out(w2);
     const size_t n[3] = {chunks * 64 * w1 * ENC_K1, chunks * 32 * w2 * ENC_K2, chunks * 16 * w3 * ENC_K2};
     size_t cols = n[0];
     for (int i = 1; i < 3; i++) cols = n[i] > cols ? n[i] : cols;
     QK_TRY(dmalloc((void **)&e->cols, cols * 4));
-    e->cap_cols = chunks;
+    QK_TRY(dmalloc((void **)&e->rows, chunks * w3 * ENC_CH * 16 * 4));
+    e->cap_general = chunks;
     return 0;
 }
 
@@ -490,7 +491,7 @@ static int run_general(qwen_hip_encoder *e, int mel_frames, int *tokens_out) {
     const int last = mel_frames - (chunks - 1) * cw;
     const int w1 = conv_out(cw), w2 = conv_out(w1), w3 = conv_out(w2);
     const int T = qwen_hip_encoder_tokens(c, mel_frames);
-    QK_TRY(reserve_cols(e, chunks));
+    QK_TRY(reserve_general(e, chunks));
     /* conv stem (qwen_asr_encoder.c:237-279); the mel is [128][mel_frames] */
     QK_TRY(stem_layer(e, e->mel, 1, chunks, ENC_MEL, cw, ENC_K1, mel_frames, e->c1w, NULL, e->c1b, e->c1,
                       conv_out(last)));

@@ -430,3 +430,23 @@ def test_encoder_mel_in_host_memory(P, qa, gpu):
     T, p = e.forward_device(h.data_ptr(), 250)
     assert np.array_equal(d2h(p, (T, cfg.output_dim)), want)
     e.close()
+
+
+def test_encoder_activation_memory(P, qa, gpu):
+    """A bf16-valued encoder allocates what its products use: the stem's pixels,
+    the rows' activations and the split workspace, and no patch or row matrix of
+    the general path (80 MB of token rows here)."""
+    cfg = qa.EncConfig(128, 2, 2, 64, 256, 96, 100, 200)
+    frames, chunks = 20000, 200
+    e = qa.Encoder(cfg, 0)
+    e.load_synthetic(1, 0.02)
+    mel = P.synth_mel(frames, 1, 0)
+    before = gpu.cuda.mem_get_info()[0]
+    e.forward(mel)
+    used = before - gpu.cuda.mem_get_info()[0]
+    pixels = 480 * chunks * (64 * 50 + 32 * 25 + 16 * 13) * 4
+    T = chunks * 13
+    rows = T * 4 * (3 * 128 + 4 * 128 + 256 + 96)
+    ws = 2048 * 64 * 64 * 4
+    assert used <= 128 * frames * 4 + pixels + rows + ws + (40 << 20), used     # 12 buffers, rounded up each
+    e.close()
