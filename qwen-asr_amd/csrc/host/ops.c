@@ -127,12 +127,14 @@ int qwen_hip_linear_nobias_bf16(float *y, const float *x, const uint16_t *W, int
 }
 
 /* Rows of up to 2048 columns, which a wave holds whole; longer ones keep their
- * three launches of the k-split GEMV, and other widths are refused there.  A
- * launch counts its threads in 32 bits, 32 of them to a row here and 16 or fewer
- * there, so more rows go there too. */
+ * three launches of the k-split GEMV, and other widths are refused there.  Up to
+ * 2^17 rows in all one launch is the faster (8192 rows of 1024 columns 4.8 us
+ * against 9.3, 65536 of 128 columns 5.9 against 9.4, of 2048 37 against 41), above
+ * them a row of the narrow ones is cheaper with four to a wave (2^18 of 512: 45.7
+ * against 41.1), and past 2^27 the launch could not count its threads. */
 static int qkv_one_launch(int in_dim, int q_dim, int kv_dim) {
     return in_dim > 0 && in_dim % 8 == 0 && in_dim <= 2048 && q_dim > 0 && kv_dim > 0 &&
-           (long)q_dim + 2L * kv_dim <= 1L << 26;
+           (long)q_dim + 2L * kv_dim <= 1L << 17;
 }
 
 int qwen_hip_linear_nobias_bf16_qkv(float *q, float *k, float *v, const float *x, const uint16_t *Wq,

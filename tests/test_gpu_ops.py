@@ -652,3 +652,18 @@ def test_head_ops_many_rows(P, qa, gpu, what, S):
     del x
     gpu.cuda.empty_cache()
     assert wrong == 0
+
+
+# around the 2^17 rows up to which the three products are one launch
+@pytest.mark.parametrize("qd", [(1 << 17) - 8, (1 << 17) - 7])
+def test_linear_qkv_launch_limit(P, qa, gpu, qd):
+    K, kvd = 64, 4
+    g = gpu.Generator(device="cuda").manual_seed(qd)
+    W, x = [gpu.randn(n, K, generator=g, device="cuda").bfloat16() for n in (qd, kvd, kvd)], gpu.randn(K, generator=g, device="cuda")
+    y = [gpu.full((n,), 7.0, device="cuda") for n in (qd, kvd, kvd)]
+    qa.check(qa.lib().qwen_hip_linear_nobias_bf16_qkv(*[ptr(t) for t in y], ptr(x), *[ptr(t) for t in W], K, qd, kvd,
+                                                      None), "qkv")
+    gpu.cuda.synchronize()
+    for w, o in zip(W, y):
+        exp, size = w.double() @ x.double(), w.double().abs() @ x.double().abs()
+        assert bool(((o.double() - exp).abs() <= 8 * K * 2.0 ** -24 * size).all())
