@@ -667,3 +667,17 @@ def test_linear_qkv_launch_limit(P, qa, gpu, qd):
     for w, o in zip(W, y):
         exp, size = w.double() @ x.double(), w.double().abs() @ x.double().abs()
         assert bool(((o.double() - exp).abs() <= 8 * K * 2.0 ** -24 * size).all())
+
+
+# more values than 65536 blocks take in one walk, and a ragged end
+def test_elementwise_large(P, qa, gpu):
+    lib, n = qa.lib(), (1 << 26) + 1026
+    a, b = gpu.arange(n, dtype=gpu.float32, device="cuda"), gpu.full((n,), 2.0, device="cuda")
+    qa.check(lib.qwen_hip_add_inplace(ptr(a), ptr(b), n, None))
+    gpu.cuda.synchronize()
+    assert gpu.equal(a, gpu.arange(n, dtype=gpu.float32, device="cuda") + 2.0)
+    gu = gpu.stack([gpu.zeros(n, device="cuda"), b], 1)
+    gu[-1, 0] = gu[1 << 26, 0] = 100.0                          # silu(100) = 100
+    qa.check(lib.qwen_hip_swiglu_multiply(ptr(a), ptr(gu), n // 2, 2, None))
+    gpu.cuda.synchronize()
+    assert float(a[-1]) == 200.0 and float(a[1 << 26]) == 200.0 and int(a.count_nonzero()) == 2
