@@ -599,9 +599,12 @@ static void gemm_wide_dispatch(const uint16_t *a_hi, const uint16_t *a_lo, const
 // per CU.  The 16-row load groups of a stage (A_hi, A_lo, W) are dealt
 // round-robin to the waves: LPW 1 KB load instructions per wave and stage.
 // ---------------------------------------------------------------------------
-// KG 2: launches of about one block per CU (ring_walk2)
+// KG 2: launches of about one block per CU (ring_walk2).  The four-wave blocks name
+// the two that share a CU: without, one accumulator of the 64 x 128 and 32 x 128 tiles
+// was copied to and from its registers in every k step, behind all MFMAs before it
+// (401 x 12288 x 2048, op level: 72.6 us, 69.7 with)
 template <int EPI, int BM, int BN, int NST, int KG>
-__global__ __launch_bounds__(KG *ring_waves(BM, BN) * 64) void gemm_hilo_ring(const uint16_t *__restrict__ ahi,
+__global__ __launch_bounds__(KG *ring_waves(BM, BN) * 64, KG == 1 && ring_waves(BM, BN) == 4 ? 2 : 1) void gemm_hilo_ring(const uint16_t *__restrict__ ahi,
                                                                                const uint16_t *__restrict__ alo,
                                                                                const uint16_t *__restrict__ W, int M,
                                                                                int N, int K, int kc, float *y,
