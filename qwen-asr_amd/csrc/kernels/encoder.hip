@@ -797,31 +797,6 @@ __global__ __launch_bounds__(256) void enc_ring_reduce_ln(qk_enc_ring_args a) {
                                      dw * inv * w.w + b.w));
 }
 
-// Tile height and split of an M x N x K product.  64-row tiles (32 up to 32
-// rows; 128 where those alone give every CU a block).  K is split while the launch
-// stays within QK_ENC_RING_TARGET blocks, one per CU (fc2 at 390 rows: 294 blocks
-// in six splits 18.2 us, 245 in five 14.2), k walks of 4 k tiles at least.  A
-// product whose epilogue needs no reduce pass (`fused`) and walks up to
-// QK_ENC_RING_FUSED k tiles is not cut in two: that saves 3.5 us, the reduce takes
-// 4.5.
-extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, long ws_elems, int *bm, int *kc,
-                                 int *split) {
-    const long nt = (N + 127) / 128;
-    *bm = M <= 32 && !gather ? 32 : (long)((M + 127) / 128) * nt >= 256 ? 128 : 64;
-    const long tiles = (M + *bm - 1) / *bm * nt;
-    const int kt = K / QK_GBK;
-    long ns = QK_ENC_RING_TARGET / tiles;
-    if (fused && ns <= 2 && kt <= QK_ENC_RING_FUSED) ns = 1;
-    if (ns > QK_ENC_RING_SPLIT) ns = QK_ENC_RING_SPLIT;
-    if (ns > kt / 4) ns = kt / 4;
-    while (ns > 1 && ns * M * N > ws_elems) ns--;
-    if (ns < 1) ns = 1;
-    int per = (int)((kt + ns - 1) / ns);
-    if (K % 64 == 0) per += per & 1;      // whole 64-deep stages
-    *kc = per * QK_GBK;
-    *split = (kt + per - 1) / per;
-}
-
 // Products with their own epilogue over few rows: 32 x 64 tiles, unsplit, on at
 // most one block per CU, whose ring of 8 stages keeps the loads in flight that a
 // split's extra blocks did: no partials, no reduce pass.  Whole encoder against
@@ -831,6 +806,36 @@ extern "C" void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, lon
 static bool enc_ring_narrow(int M, int N, int K) {
     const long blocks = (long)((M + 31) / 32) * ((N + 63) / 64);
     return K % 64 == 0 && K <= QK_ENC_RING_FUSED * QK_GBK && blocks >= QK_ENC_NARROW_MIN && blocks <= 256;
+}
+
+// Tile, split and k groups of an M x N x K product.  64-row tiles (32 up to 32
+// rows; 128 where those alone give every CU a block).  K is split while the launch
+// stays within QK_ENC_RING_TARGET blocks, one per CU (fc2 at 390 rows: 294 blocks
+// in six splits 18.2 us, 245 in five 14.2), k walks of 4 k tiles at least.  A
+// product whose epilogue needs no reduce pass (`fused`) and walks up to
+// QK_ENC_RING_FUSED k tiles is not cut in two: that saves 3.5 us, the reduce takes
+// 4.5.  Launches of at most one block per CU take 64-deep stages and two k groups.
+extern "C" void qk_enc_ring_plan_for(int M, int N, int K, int fused, int gather, long ws_elems, qk_enc_ring_plan *p) {
+    if (fused && !gather && enc_ring_narrow(M, N, K)) {
+        *p = {.bm = 32, .bn = 64, .groups = 2, .kc = K, .split = 1};
+        return;
+    }
+    const long nt = (N + 127) / 128;
+    p->bm = M <= 32 && !gather ? 32 : (long)((M + 127) / 128) * nt >= 256 ? 128 : 64;
+    p->bn = 128;
+    const long tiles = (M + p->bm - 1) / p->bm * nt;
+    const int kt = K / QK_GBK;
+    long ns = QK_ENC_RING_TARGET / tiles;
+    if (fused && ns <= 2 && kt <= QK_ENC_RING_FUSED) ns = 1;
+    if (ns > QK_ENC_RING_SPLIT) ns = QK_ENC_RING_SPLIT;
+    if (ns > kt / 4) ns = kt / 4;
+    while (ns > 1 && ns * M * N > ws_elems) ns--;
+    if (ns < 1) ns = 1;
+    int per = (int)((kt + ns - 1) / ns);
+    if (K % 64 == 0) per += per & 1;      // whole 64-deep stages
+    p->kc = per * QK_GBK;
+    p->split = (kt + per - 1) / per;
+    p->groups = p->bm < 128 && !gather && K % 64 == 0 && p->kc % 64 == 0 && tiles * p->split <= 256 ? 2 : 1;
 }
 
 extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_elems, hipStream_t s) {
@@ -844,26 +849,22 @@ extern "C" int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_
                    (a->taps == 9 && (a->col_h <= 0 || a->col_w <= 0 || (long)a->chunks * a->col_h * a->col_w < a->M))))
         return QWEN_HIP_EINVAL;
     if (a->valid > 0 && (!gather || ln || a->col_h <= 0 || a->col_w <= 0)) return QWEN_HIP_EINVAL;   // stem layers only
+    qk_enc_ring_plan p;
+    qk_enc_ring_plan_for(a->M, a->N, a->K, !ln, gather, ws ? ws_elems : 0, &p);
     qk_enc_ring_args g = *a;
-    if (!ln && !gather && enc_ring_narrow(a->M, a->N, a->K)) {
-        const dim3 grid((a->N + 63) / 64, (a->M + 31) / 32);
-        g.kc = a->K;
-        g.split = 1;
-        g.ws = nullptr;
+    g.kc = p.kc;
+    g.split = p.split;
+    g.ws = ln || p.split > 1 ? ws : nullptr;
+    const dim3 grid((a->N + p.bn - 1) / p.bn, (a->M + p.bm - 1) / p.bm, p.split);
+    if (p.bn == 64) {
         constexpr int threads = 2 * 64 * ring_waves(32, 64);
         if (a->C) enc_ring<32, 64, 8, false, ENC_F32, 2><<<grid, threads, 0, s>>>(g);
         else enc_ring<32, 64, 8, false, ENC_GELU, 2><<<grid, threads, 0, s>>>(g);
         return hipGetLastError() == hipSuccess ? 0 : QWEN_HIP_EDEVICE;
     }
-    int bm;
-    qk_enc_ring_plan(a->M, a->N, a->K, !ln, gather, ws ? ws_elems : 0, &bm, &g.kc, &g.split);
-    g.ws = ln || g.split > 1 ? ws : nullptr;
-    const dim3 grid((a->N + 127) / 128, (a->M + bm - 1) / bm, g.split);
-    // launches of at most one block per CU: 64-deep stages, two k groups per block
-    const int kgs = bm < 128 && !gather && a->K % 64 == 0 && g.kc % 64 == 0 && (long)grid.x * grid.y * grid.z <= 256 ? 2 : 1;
     const int epi = g.ws ? ENC_PART : a->C ? ENC_F32 : ENC_GELU;
 #define QK_ENC_RING(BM_, NST_, G_, E_, KG_)                               \
-    if (bm == BM_ && gather == G_ && epi == E_ && kgs == KG_)             \
+    if (p.bm == BM_ && gather == G_ && epi == E_ && p.groups == KG_)      \
         enc_ring<BM_, 128, NST_, G_, E_, KG_><<<grid, KG_ * 64 * ring_waves(BM_, 128), 0, s>>>(g);
 #define QK_ENC_RING_BM(BM_, NST_, G_, KG_) \
     QK_ENC_RING(BM_, NST_, G_, ENC_PART, KG_) QK_ENC_RING(BM_, NST_, G_, ENC_GELU, KG_)

@@ -457,8 +457,12 @@ typedef struct {
     int kc, split;
 } qk_enc_ring_args;
 int qk_enc_ring_launch(const qk_enc_ring_args *a, float *ws, long ws_elems, hipStream_t s);
-/* tile rows, k per split and splits of such a product (fused: no reduce pass needed) */
-void qk_enc_ring_plan(int M, int N, int K, int fused, int gather, long ws_elems, int *bm, int *kc, int *split);
+/* tile rows and columns, k groups, k per split and splits of such a product (fused:
+ * no reduce pass needed; gather: taps > 0) */
+typedef struct {
+    int bm, bn, groups, kc, split;
+} qk_enc_ring_plan;
+void qk_enc_ring_plan_for(int M, int N, int K, int fused, int gather, long ws_elems, qk_enc_ring_plan *p);
 /* conv1 from the mel [h_in][mel_frames] (chunks of w_in frames) and weights
  * w[480][kpad] (9 taps) as pixels [chunk][h_out][w_out], + bias, GELU,
  * the last chunk's positions ow >= valid 0 */

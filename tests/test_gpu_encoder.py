@@ -215,15 +215,40 @@ def gelu64(gpu, v):
     return 0.5 * v * (1 + gpu.tanh(0.7978845608028654 * (v + 0.044715 * v ** 3)))
 
 
-# 32-, 64- and 128-row tiles; one and two k groups; split and unsplit; ragged
-# rows, columns and k walks (K 96: no whole 64-deep stages)
-@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (32, 96, 64), (33, 192, 96), (97, 1024, 1024), (390, 896, 3584),
-                                   (65, 4096, 896), (1600, 3072, 128), (4100, 1024, 64)])
+class RingPlan(C.Structure):
+    _fields_ = [(n, C.c_int) for n in ("bm", "bn", "groups", "kc", "split")]
+
+
+def ring_choice(lib, M, N, K, fused, ws, gather=0):
+    """(tile rows, tile columns, k groups, splits) of the launch"""
+    p = RingPlan()
+    lib.qk_enc_ring_plan_for(M, N, K, int(fused), gather, C.c_long(ws), C.byref(p))
+    return p.bm, p.bn, p.groups, p.split
+
+
+# every kernel of the products: the tile, k groups and splits that a product with an
+# own epilogue (fp32, GELU) and one that is split for the LayerNorm pass launch; ragged
+# rows and columns, k walks shorter and longer than the ring, no whole 64-deep stages
+@pytest.mark.parametrize("M,N,K,own,part", [
+    (1, 128, 128, (32, 128, 2, 1), (32, 128, 2, 1)), (32, 96, 64, (32, 128, 2, 1), (32, 128, 2, 1)),
+    (20, 1000, 1120, (32, 128, 1, 7), (32, 128, 1, 7)), (31, 960, 96, (32, 128, 1, 1), (32, 128, 1, 1)),
+    (33, 192, 96, (64, 128, 1, 1), (64, 128, 1, 1)), (97, 1024, 1024, (32, 64, 2, 1), (64, 128, 2, 8)),
+    (390, 896, 3584, (64, 128, 2, 5), (64, 128, 2, 5)), (390, 2688, 896, (64, 128, 2, 1), None),
+    (390, 3584, 896, (64, 128, 2, 1), None), (300, 1000, 1120, (64, 128, 1, 6), (64, 128, 1, 6)),
+    (1030, 2048, 96, (64, 128, 1, 1), None), (65, 4096, 896, (32, 64, 2, 1), None), (1600, 3072, 128, (128, 128, 1, 1), None),
+    (4100, 1024, 64, (128, 128, 1, 1), (128, 128, 1, 1))])
 @pytest.mark.parametrize("what", ["f32", "gelu", "ln"])
-def test_ring_products(P, qa, gpu, M, N, K, what):
+def test_ring_products(P, qa, gpu, M, N, K, own, part, what):
     """qk_enc_ring_launch on rows of halves against a float64 product of the
     same halves: fp32 accumulation leaves 4 K 2^-24 sum |x w|, halves of the
     result 2^-16 relative."""
+    if part or what != "ln":
+        got = ring_choice(qa.lib(), M, N, K, what != "ln", max(8 * 64 * 64 * 1024, M * N))
+        assert got == (part if what == "ln" else own), got
+    ring_product(qa, gpu, M, N, K, what)
+
+
+def ring_product(qa, gpu, M, N, K, what):
     lib = qa.lib()
     lib.qk_enc_ring_launch.argtypes = [C.c_void_p, C.c_void_p, C.c_long, C.c_void_p]
     g = gpu.Generator(device="cuda").manual_seed(M + N)
@@ -263,15 +288,20 @@ def test_ring_products(P, qa, gpu, M, N, K, what):
 
 
 # few rows with an own epilogue: 32 x 64 tiles on one block per CU, at the fewest
-# and the most blocks, ragged rows and columns, k walks shorter than the ring
-@pytest.mark.parametrize("M,N,K", [(1, 8192, 64), (33, 3080, 128), (97, 2688, 896), (128, 4096, 1024), (160, 3068, 640)])
+# blocks (32) and the most (256), ragged rows and columns, k walks shorter than the ring
+@pytest.mark.parametrize("M,N,K", [(1, 2048, 128), (64, 1024, 64), (1, 8192, 64), (33, 3080, 128), (97, 2688, 896),
+                                   (128, 4096, 1024), (160, 3068, 640)])
 @pytest.mark.parametrize("what", ["f32", "gelu"])
 def test_ring_products_narrow(P, qa, gpu, M, N, K, what):
-    test_ring_products(P, qa, gpu, M, N, K, what)
+    assert ring_choice(qa.lib(), M, N, K, 1, 1 << 30) == (32, 64, 2, 1)
+    ring_product(qa, gpu, M, N, K, what)
 
 
-@pytest.mark.parametrize("chunks,h,w,valid", [(1, 8, 5, 3), (3, 32, 25, 1), (9, 32, 50, 25), (2, 4, 1, 1)])
-def test_ring_convolution(P, qa, gpu, chunks, h, w, valid):
+# 64-row tiles, split and unsplit; 128-row tiles (the second layer of 11 chunks and
+# more), with a ragged last one
+@pytest.mark.parametrize("chunks,h,w,valid,bm,split", [(1, 8, 5, 3, 64, 8), (3, 32, 25, 1, 64, 6), (9, 32, 50, 25, 64, 1),
+                                                       (2, 4, 1, 1, 64, 8), (10, 64, 50, 7, 64, 1), (11, 64, 50, 12, 128, 1)])
+def test_ring_convolution(P, qa, gpu, chunks, h, w, valid, bm, split):
     """The gathered 3x3 / stride 2 / padding 1 convolution with GELU, weights
     through qk_enc_tile_weights_launch, and the last chunk's padding zeroed,
     against float64 on the same halves."""
@@ -286,6 +316,8 @@ def test_ring_convolution(P, qa, gpu, chunks, h, w, valid):
     A, xv = halves(gpu, x, pixel=True)
     ho, wo = (h + 1) // 2, (w + 1) // 2
     M = chunks * ho * wo
+    got = ring_choice(lib, M, CH, 9 * CH, 1, 8 * M * CH, 1)
+    assert got == (bm, 128, 1, split), got
     bias = gpu.randn(CH, generator=g, device="cuda")
     out = gpu.full((M, 2 * CH), 7.0, dtype=gpu.bfloat16, device="cuda")
     ws = gpu.empty(8 * M * CH, device="cuda")
@@ -302,6 +334,41 @@ def test_ring_convolution(P, qa, gpu, chunks, h, w, valid):
     ref = ref.view(M, CH)
     got = unhalve(gpu, out, CH, pixel=True)
     assert bool(((got - ref).abs() <= 1.2 * bound + 2.0 ** -16 * ref.abs() + 2.0 ** -22 * y.abs()).all())
+
+
+# a token's pixels, top to bottom, against the positions' table and the first LayerNorm:
+# 64-row tiles in splits and 128-row tiles, ragged last ones
+@pytest.mark.parametrize("T,w,N,bm,split", [(1, 1, 128, 64, 8), (39, 13, 896, 64, 8), (390, 13, 896, 64, 5),
+                                            (4750, 13, 896, 128, 1), (4161, 13, 1024, 128, 1)])
+def test_ring_token_rows(P, qa, gpu, T, w, N, bm, split):
+    lib, CH, H = qa.lib(), 480, 16
+    lib.qk_enc_ring_launch.argtypes = [C.c_void_p, C.c_void_p, C.c_long, C.c_void_p]
+    lib.qk_enc_tile_weights_launch.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p]
+    g = gpu.Generator(device="cuda").manual_seed(T)
+    chunks, K = -(-T // w), CH * H
+    x = gpu.randn(chunks * H * w, CH, generator=g, device="cuda")
+    W = (gpu.randn(N, K, generator=g, device="cuda") * 0.02).bfloat16()            # column channel * 16 + row
+    Wt, zero = gpu.empty_like(W), gpu.zeros(64, dtype=gpu.bfloat16, device="cuda")
+    qa.check(lib.qk_enc_tile_weights_launch(W.data_ptr(), Wt.data_ptr(), N, CH, H, None), "tile")
+    A, xv = halves(gpu, x, pixel=True)
+    pe, lw, lb = (gpu.randn(n, N, generator=g, device="cuda") for n in (w, 1, 1))
+    f, out = gpu.empty(T, N, device="cuda"), gpu.empty(T, 2 * N, dtype=gpu.bfloat16, device="cuda")
+    ws = gpu.empty(max(2048 * 64 * 64, T * N), device="cuda")
+    got = ring_choice(lib, T, N, K, 0, ws.numel(), 1)
+    assert got == (bm, 128, 1, split), got
+    a = RingArgs(A=A.data_ptr(), W=Wt.data_ptr(), zero=zero.data_ptr(), M=T, N=N, K=K, taps=H, in_h=H, in_w=w,
+                 pe=pe.data_ptr(), pe_rows=w, C=f.data_ptr(), out=out.data_ptr(), ln_w=lw.data_ptr(), ln_b=lb.data_ptr(),
+                 ln_eps=1e-5)
+    qa.check(lib.qk_enc_ring_launch(C.byref(a), ws.data_ptr(), ws.numel(), None), "ring")
+    gpu.cuda.synchronize()
+    cols = xv.view(chunks, H, w, CH).permute(0, 2, 3, 1).reshape(chunks * w, K)[:T].contiguous()
+    rows = pe.double()[gpu.arange(T, device="cuda") % w]
+    y = cols @ W.double().t().contiguous() + rows
+    bound = 4 * K * 2.0 ** -24 * (cols.abs() @ W.double().abs().t().contiguous()) + 2.0 ** -22 * rows.abs() + 1e-6
+    assert bool(((f.double() - y).abs() <= bound).all())
+    fd = f.double()
+    ref = (fd - fd.mean(1, keepdim=True)) / gpu.sqrt(fd.var(1, unbiased=False, keepdim=True) + 1e-5) * lw + lb
+    assert bool(((unhalve(gpu, out, N) - ref).abs() <= 2.0 ** -16 * ref.abs() + 2e-5).all())   # fp32 sums of the row
 
 
 # windows of one and several rounds of the four waves' 128 keys; ragged last
