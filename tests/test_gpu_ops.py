@@ -187,8 +187,9 @@ class RopeArgs(C.Structure):
 
 # the Q|K|V GEMM with rope_append's work as its epilogue: bit for bit the
 # GEMM (STORE) followed by rope_append, on a full and a partial last row tile,
-# at a nonzero start position, for the 0.6B and 1.7B widths
-@pytest.mark.parametrize("M,K,start", [(401, 1024, 37), (130, 2048, 0), (64, 1024, 900)])
+# at a nonzero start position, for the 0.6B and 1.7B widths; up to 512 rows by two k
+# groups, above by one
+@pytest.mark.parametrize("M,K,start", [(401, 1024, 37), (130, 2048, 0), (64, 1024, 900), (513, 1024, 41), (577, 2048, 0)])
 def test_gemm_rope_epilogue(P, qa, gpu, M, K, start):
     lib = qa.lib()
     H, KVH, hd, cap = 16, 8, 128, 1024
@@ -542,8 +543,8 @@ def test_one_query_splits(P, qa, gpu, sk):
 
 
 # the 64-column SwiGLU tiles of up to 64 rows: both row tiles, rows short of a
-# tile, the fewest and the most column tiles, k walks shorter than the ring and
-# not a multiple of its depth
+# tile, 128 column tiles (the fewest up to 32 rows) and the most, k walks shorter
+# than the ring and not a multiple of its depth
 @pytest.mark.parametrize("M", [2, 31, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(8192, 64), (8192, 1024), (16384, 320), (12288, 2048)])
 def test_gemm_swiglu_narrow(P, qa, gpu, M, N, K):
@@ -681,3 +682,24 @@ def test_elementwise_large(P, qa, gpu):
     qa.check(lib.qwen_hip_swiglu_multiply(ptr(a), ptr(gu), n // 2, 2, None))
     gpu.cuda.synchronize()
     assert float(a[-1]) == 200.0 and float(a[1 << 26]) == 200.0 and int(a.count_nonzero()) == 2
+
+
+# the prefill's SwiGLU products on 64 x 128 tiles, unsplit, by two k groups (up to 256
+# blocks: 257 to 320 rows of the 0.6B gate|up) and by one (336), k walks of many rings
+@pytest.mark.parametrize("M", [257, 300, 320, 321])
+def test_gemm_swiglu_planned(P, qa, gpu, M):
+    N, K, p = 6144, 1024, GemmPlan()
+    assert not qa.lib().qk_gemm_plan_narrow(M, N, K, C.byref(p))
+    qa.lib().qk_gemm_plan_epi(M, N, K, 2, C.byref(p))
+    assert (p.bm, p.bn, p.nst, p.nsplit) == (64, 128, 4, 1)
+    assert (-(-M // 64) * (N // 128) <= 256) == (M <= 320)
+    check_gemm(P, qa, gpu, M, N, K, p, 2)
+
+
+# the 0.6B gate|up (96 column tiles) on the 64-column tiles of 33 to 64 rows
+@pytest.mark.parametrize("M", [33, 64])
+def test_gemm_swiglu_narrow_fewest(P, qa, gpu, M):
+    p = GemmPlan()
+    assert qa.lib().qk_gemm_plan_narrow(M, 6144, 1024, C.byref(p)) == 1
+    assert (p.bm, p.bn, p.nst, p.nsplit) == (64, 64, 6, 1)
+    check_gemm(P, qa, gpu, M, 6144, 1024, p, 2)
