@@ -433,7 +433,7 @@ static int reserve_general(qwen_hip_encoder *e, int chunks) {
 /* Every matrix bf16-valued and of widths the ring products take (d <= 1024,
  * k walks of whole 32-deep tiles, rows of whole float4s): the path of
  * run_ring; otherwise the general one. */
-static int ring_ok(const qwen_hip_encoder *e) {
+int qk_enc_ring_ok(const qwen_hip_encoder *e) {
     const qwen_hip_enc_config *c = &e->cfg;
     if (c->d_model > 1024 || c->ffn_dim % 32 || c->output_dim % 4) return 0;
     int ok = e->c2t && e->c3t && e->cowt && e->p1w.b16 && e->p2w.b16;
@@ -597,7 +597,7 @@ int qwen_hip_encoder_forward(qwen_hip_encoder *e, const float *mel, int mel_fram
     if (!mel || !out) { qk_set_err("encoder: NULL mel or output"); return QWEN_HIP_EINVAL; }
     QK_HIP(hipMemcpyAsync(e->mel, mel, (size_t)ENC_MEL * mel_frames * 4, hipMemcpyHostToDevice, e->stream));
     int T = 0;
-    QK_TRY(ring_ok(e) ? run_ring(e, e->mel, mel_frames, &T) : run_general(e, mel_frames, &T));
+    QK_TRY(qk_enc_ring_ok(e) ? run_ring(e, e->mel, mel_frames, &T) : run_general(e, mel_frames, &T));
     QK_HIP(hipMemcpyAsync(out, e->out, (size_t)T * e->cfg.output_dim * 4, hipMemcpyDeviceToHost, e->stream));
     QK_HIP(hipStreamSynchronize(e->stream));
     return T;
@@ -624,7 +624,7 @@ int qwen_hip_encoder_forward_device(qwen_hip_encoder *e, const float *d_mel, int
     if (rc) return rc;
     if (!d_mel || !d_out) { qk_set_err("encoder: NULL mel or output"); return QWEN_HIP_EINVAL; }
     int T = 0;
-    const int ring = ring_ok(e), in_place = ring && mel_in_place(e, d_mel);
+    const int ring = qk_enc_ring_ok(e), in_place = ring && mel_in_place(e, d_mel);
     if (!in_place)
         QK_HIP(hipMemcpyAsync(e->mel, d_mel, (size_t)ENC_MEL * mel_frames * 4, hipMemcpyDeviceToDevice, e->stream));
     QK_TRY(ring ? run_ring(e, in_place ? d_mel : e->mel, mel_frames, &T) : run_general(e, mel_frames, &T));

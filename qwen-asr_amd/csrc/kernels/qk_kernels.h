@@ -472,6 +472,12 @@ int qk_enc_conv1_halves_launch(const float *mel, int kpad, const float *w, const
  * + c, [k / 32][row][k % 32] (h 1: the columns keep their order) */
 int qk_enc_tile_weights_launch(const uint16_t *in, uint16_t *out, int rows, int ch, int h, hipStream_t s);
 
+/* whether the encoder's loaded weights and widths take the ring products (encoder.c) */
+struct qwen_hip_encoder;
+int qk_enc_ring_ok(const struct qwen_hip_encoder *e);
+/* whether forward_device reads a mel of this memory type and device where it is */
+int qk_enc_mel_in_place(int type, int mem_device, int device);
+
 /* ---- elementwise (op-level ABI) --------------------------------------- */
 int qk_add_launch(float *a, const float *b, long n, hipStream_t s);
 int qk_rms_norm_launch(float *out, const float *x, const float *w, int S, int D,

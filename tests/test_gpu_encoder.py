@@ -47,6 +47,7 @@ def test_encoder_matches_reference(P, qa, gpu, name):
     g = fixture(name)
     cfg, m, mel = build(qa, P, g)
     e = load(qa, cfg, m)
+    assert qa.lib().qk_enc_ring_ok(C.c_void_p(e.h))
     out = e.forward(mel)
     ref = g["out"]
     assert out.shape == ref.shape
@@ -516,4 +517,89 @@ def test_encoder_activation_memory(P, qa, gpu):
     rows = T * 4 * (3 * 128 + 4 * 128 + 256 + 96)
     ws = 2048 * 64 * 64 * 4
     assert used <= 128 * frames * 4 + pixels + rows + ws + (40 << 20), used     # 12 buffers, rounded up each
+    e.close()
+
+
+def encoder64(gpu, m, mel):
+    """qwen_encoder_forward (qwen_asr_encoder.c:171-372) in float64 on a SynthEncoder's arrays"""
+    t = lambda a: gpu.from_numpy(np.ascontiguousarray(a, np.float32)).cuda().double()
+    c, cw = m.cfg, m.cfg.chunk_size
+    stem, F = [t(a) for a in m.stem], gpu.nn.functional
+    x, n = t(mel), -(-mel.shape[1] // cw)
+
+    def ln(v, w, b):
+        d = v - v.mean(-1, keepdim=True)
+        return d / gpu.sqrt((d * d).mean(-1, keepdim=True) + 1e-5) * w + b
+    rows = []
+    for i in range(n):                                       # every chunk is an image of its own
+        y = x[None, None, :, i * cw:(i + 1) * cw]
+        for k in range(0, 6, 2):
+            co, ci, (h, w) = 480, y.shape[1], y.shape[2:]
+            ho, wo = (h + 1) // 2, (w + 1) // 2
+            im = F.pad(y, (1, 2, 1, 2))[0]
+            cols = gpu.stack([im[:, a:a + 2 * ho - 1:2, b:b + 2 * wo - 1:2] for a in range(3) for b in range(3)], 1)
+            y = gelu64(gpu, stem[k].view(co, ci * 9) @ cols.reshape(ci * 9, ho * wo) + stem[k + 1][:, None])
+            y = y.view(1, co, ho, wo)
+        y = y[0].permute(2, 0, 1).reshape(y.shape[3], -1) @ stem[6].t()
+        half = c.d_model // 2
+        inv = gpu.exp(-gpu.arange(half, device="cuda").double() * np.log(10000.0) / (half - 1))
+        a = gpu.arange(y.shape[0], device="cuda").double()[:, None] * inv
+        rows.append(y + gpu.cat([gpu.sin(a), gpu.cos(a)], 1))
+    x = gpu.cat(rows)
+    tpc = cw
+    for _ in range(3):
+        tpc = (tpc + 1) // 2
+    win, H = tpc * (c.n_window_infer // cw), c.heads
+    for arrs in m.layers:
+        w = [t(a) for a in arrs]
+        v = ln(x, w[8], w[9])
+        q, k, u = (v @ w[2 * i].t() + w[2 * i + 1] for i in range(3))
+        att = gpu.empty_like(q)
+        for t0 in range(0, x.shape[0], win):
+            s = slice(t0, t0 + win)
+            qq, kk, uu = (z[s].view(-1, H, 64).transpose(0, 1) for z in (q, k, u))
+            att[s] = (gpu.softmax(qq @ kk.transpose(1, 2) / 8.0, -1) @ uu).transpose(0, 1).reshape(-1, c.d_model)
+        x = x + att @ w[6].t() + w[7]
+        x = x + gelu64(gpu, ln(x, w[14], w[15]) @ w[10].t() + w[11]) @ w[12].t() + w[13]
+    return gelu64(gpu, ln(x, stem[7], stem[8]) @ stem[9].t() + stem[10]) @ stem[11].t() + stem[12]
+
+
+def test_encoder64_is_the_reference(P, qa, gpu):
+    """the float64 encoder of this file against the compiled reference's output"""
+    g = fixture("enc_tiny")
+    cfg, m, mel = build(qa, P, g)
+    err = np.abs(encoder64(gpu, m, mel).cpu().numpy() - g["out"])
+    assert np.all(err <= ATOL + RTOL * np.abs(g["out"])), float(err.max())
+
+
+# The general path: off-grid weights (fp32 products), bf16-valued ones of widths the ring
+# products do not take (d above 1024; outputs that are no whole float4s), off-grid ones
+# among bf16-valued ones (stem, a layer's fc2, the output projection), an ffn of no whole
+# 32-wide tiles; a few rows (split products, LayerNorm in the reduce) and 12 chunks
+# (128 x 128 tiles of the second convolution)
+@pytest.mark.parametrize("frames", [41, 350, 1230])
+@pytest.mark.parametrize("d,ffn,out,off", [(128, 256, 96, "all"), (1088, 256, 96, ""), (128, 256, 98, ""),
+                                           (128, 256, 96, "mixed"), (128, 132, 96, "all"), (192, 1056, 1030, "")])
+def test_encoder_general_path(P, qa, gpu, d, ffn, out, off, frames):
+    cfg = qa.EncConfig(d, 2, d // 64, 64, ffn, out, 100, 200)
+    m = P.SynthEncoder(cfg, seed=11)
+    rng = np.random.default_rng(11)
+
+    def nudge(arrs, ids):
+        for i in ids:
+            arrs[i] = (arrs[i] * (1.0 + 1e-3 * rng.standard_normal(arrs[i].shape))).astype(np.float32)
+    if off == "all":
+        for l in m.layers:
+            nudge(l, (0, 2, 4, 6, 10, 12))
+        nudge(m.stem, (2, 4, 6, 9, 11))
+    elif off == "mixed":
+        nudge(m.stem, (4, 11))
+        nudge(m.layers[1], (12,))
+    mel = P.synth_mel(frames, 11, 2)
+    e = load(qa, cfg, m)
+    assert not qa.lib().qk_enc_ring_ok(C.c_void_p(e.h))
+    got, ref = e.forward(mel), encoder64(gpu, m, mel).cpu().numpy()
+    err = np.abs(got - ref)
+    assert got.shape == ref.shape and np.all(err <= ATOL + RTOL * np.abs(ref)), float(err.max())
+    assert np.array_equal(e.forward(mel[:, :40]), load(qa, cfg, m).forward(mel[:, :40]))     # after a longer call
     e.close()
