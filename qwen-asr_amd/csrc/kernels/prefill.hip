@@ -779,16 +779,20 @@ static void gemm_dispatch(const uint16_t *a_hi, const uint16_t *a_lo, const uint
 
 extern "C" void qk_gemm_plan_for(int M, int N, int K, qk_gemm_plan *p) { qk_gemm_plan_epi(M, N, K, QK_GEMM_STORE, p); }
 
-// SwiGLU of up to 64 rows: bound by the weight bytes in flight.  64-column
-// tiles, one block per CU with a ring of 8 (6) stages and the whole k walk, so
-// neither partials nor a reduce pass, where they give half the CUs a block.
-// Prefill of 4 layers over 300 positions, against split 128-column tiles and a
-// reduce: 12288 columns (192 tiles) 31 rows 320 -> 301 us, 64 rows 383 -> 354;
-// 6144 (96 tiles) 64 rows 282 -> 272, 31 rows 231 -> 229, 2 rows 201 -> 205.
+// SwiGLU of up to 64 rows: bound by the weight bytes in flight.  64-column tiles, one
+// block per CU with a ring of 8 (6) stages and the whole k walk, so neither partials
+// nor a reduce pass.  A block walks all of K alone, so it needs a short walk or a full
+// chip: K up to 1024 (two rings) from 64 column tiles, up to 2048 from 192.  Against
+// split 128-column tiles and a reduce, weights not in the caches, 2 / 32 / 64 rows:
+// K 1024, 64 tiles 7.3 / 8.7 / 11.7 -> 6.5 / 7.7 / 10.0 us, 96 (the 0.6B gate|up) 7.3 /
+// 8.2 / 10.4 -> 6.5 / 7.9 / 10.1, 256 10.2 / 11.8 / 14.8 -> 8.1 / 9.0 / 11.2; K 2048, 192
+// (1.7B) 17.3 / 20.4 / 23.7 -> 12.5 / 14.5 / 18.2, 256 15.6 / 17.1 / 20.6 -> 16.3 / 16.8 /
+// 19.8, but 128 tiles 10.4 / 11.5 / 13.9 -> 10.4 / 13.2 / 17.3 and 160 11.6 / 12.9 / 15.6
+// -> 11.2 / 13.9 / 18.0.  28 layers of 0.6B, 32 rows: 1285 -> 1257 us.
 extern "C" int qk_gemm_plan_narrow(int M, int N, int K, qk_gemm_plan *p) {
     const int narrow = N / QK_GEMM_NARROW_BN;
-    if (M <= 0 || M > 64 || N % QK_GEMM_NARROW_BN || K <= 0 || K % QK_BK || narrow < (M <= 32 ? 128 : 96) ||
-        narrow > QK_GEMM_TARGET)
+    if (M <= 0 || M > 64 || N % QK_GEMM_NARROW_BN || K <= 0 || K % QK_BK || K > 2048 ||
+        narrow < (K <= 1024 ? 64 : 192) || narrow > QK_GEMM_TARGET)
         return 0;
     p->bm = M <= 32 ? 32 : 64;
     p->bn = QK_GEMM_NARROW_BN;

@@ -543,8 +543,8 @@ def test_one_query_splits(P, qa, gpu, sk):
 
 
 # the 64-column SwiGLU tiles of up to 64 rows: both row tiles, rows short of a
-# tile, 128 column tiles (the fewest up to 32 rows) and the most, k walks shorter
-# than the ring and not a multiple of its depth
+# tile, many column tiles and the most, k walks shorter than the ring and not a
+# multiple of its depth
 @pytest.mark.parametrize("M", [2, 31, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(8192, 64), (8192, 1024), (16384, 320), (12288, 2048)])
 def test_gemm_swiglu_narrow(P, qa, gpu, M, N, K):
@@ -580,7 +580,7 @@ def test_linear_qkv_edges(P, qa, gpu, hidden, qd, kvd):
 # 3.5 * 2^-23) is stored as its halves, which do not decrease with it.
 @pytest.mark.parametrize("M,N,K,bm,nst,ns", [(32, 8192, 64, 32, 8, 1), (64, 8192, 64, 64, 6, 1), (300, 6144, 64, 64, 4, 1),
                                              (401, 6144, 128, 64, 4, 1), (600, 8192, 64, 128, 3, 1),
-                                             (1000, 16384, 64, 256, 0, 1), (31, 6144, 320, 32, 4, 5),
+                                             (1000, 16384, 64, 256, 0, 1), (31, 3968, 320, 32, 4, 5),
                                              (100, 1000, 64, 64, 0, 1)])
 def test_gemm_swiglu_gate_range(P, qa, gpu, M, N, K, bm, nst, ns):
     lib, p = qa.lib(), GemmPlan()
@@ -696,10 +696,13 @@ def test_gemm_swiglu_planned(P, qa, gpu, M):
     check_gemm(P, qa, gpu, M, N, K, p, 2)
 
 
-# the 0.6B gate|up (96 column tiles) on the 64-column tiles of 33 to 64 rows
-@pytest.mark.parametrize("M", [33, 64])
-def test_gemm_swiglu_narrow_fewest(P, qa, gpu, M):
-    p = GemmPlan()
-    assert qa.lib().qk_gemm_plan_narrow(M, 6144, 1024, C.byref(p)) == 1
-    assert (p.bm, p.bn, p.nst, p.nsplit) == (64, 64, 6, 1)
-    check_gemm(P, qa, gpu, M, 6144, 1024, p, 2)
+# the fewest 64-column tiles, the 0.6B gate|up (96), and the one tile less that splits
+@pytest.mark.parametrize("M", [2, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(4096, 1024), (6144, 1024), (12288, 2048), (4096 - 128, 1024), (12288 - 128, 2048)])
+def test_gemm_swiglu_narrow_fewest(P, qa, gpu, M, N, K):
+    p, narrow = GemmPlan(), N in (4096, 6144, 12288)
+    assert qa.lib().qk_gemm_plan_narrow(M, N, K, C.byref(p)) == narrow
+    if not narrow:
+        qa.lib().qk_gemm_plan_epi(M, N, K, 2, C.byref(p))
+    assert (p.bm, p.bn, p.nsplit > 1) == (32 if M <= 32 else 64, 64 if narrow else 128, not narrow)
+    check_gemm(P, qa, gpu, M, N, K, p, 2)

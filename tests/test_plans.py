@@ -212,13 +212,16 @@ def test_mel_read_in_place(qa):
 
 
 def test_gemm_plan_narrow_limits(qa):
-    """64-column SwiGLU tiles: up to 32 rows from 128 column tiles, up to 64
-    from 96, to 256; whole 64-deep stages and whole tiles."""
+    """64-column SwiGLU tiles of up to 64 rows: 64 to 256 column tiles for K up
+    to 1024, 192 to 256 for K up to 2048; whole 64-deep stages and whole tiles."""
     p, f = GemmPlan(), qa.lib().qk_gemm_plan_narrow
-    for M, lo in ((1, 128), (32, 128), (33, 96), (64, 96)):
-        for tiles in (lo, 192, 256):
-            assert f(M, 64 * tiles, 1024, C.byref(p)) == 1
-            assert (p.bm, p.bn, p.nst, p.nsplit, p.kc) == (32 if M <= 32 else 64, 64, 8 if M <= 32 else 6, 1, 1024)
-        for N, K in ((64 * lo - 64, 1024), (64 * 257, 1024), (64 * 200 + 32, 1024), (64 * 200, 1000), (64 * 200, 0)):
-            assert f(M, N, K, C.byref(p)) == 0, (M, N, K)
+    for M in (1, 32, 33, 64):
+        for K, lo in ((64, 64), (1024, 64), (1088, 192), (2048, 192)):
+            for tiles in (lo, 224, 256):
+                assert f(M, 64 * tiles, K, C.byref(p)) == 1
+                assert (p.bm, p.bn, p.nst, p.nsplit, p.kc) == (32 if M <= 32 else 64, 64, 8 if M <= 32 else 6, 1, K)
+            for N in (64 * lo - 64, 64 * 257, 64 * 200 + 32):
+                assert f(M, N, K, C.byref(p)) == 0, (M, N, K)
+        for K in (0, 1000, 2112):
+            assert f(M, 64 * 200, K, C.byref(p)) == 0, (M, K)
     assert f(65, 64 * 200, 1024, C.byref(p)) == 0 and f(0, 64 * 200, 1024, C.byref(p)) == 0
