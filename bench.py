@@ -1,9 +1,8 @@
 #!/usr/bin/env python3
 """Benchmark of the Qwen3 decoder token loop on one MI355X.
 
-Metric (BASELINE.json): decode tok/s at batch 1 + achieved fraction of the
-HBM roofline; prefill tok/s reported alongside.  Workload (default, configs[0]
-= C1): Qwen3-ASR-0.6B decoder, random-init bf16 weights N(0, 0.02) with
+Metric: decode tok/s at batch 1 + achieved fraction of the
+HBM roofline; prefill tok/s reported alongside.  Workload (default, C1): Qwen3-ASR-0.6B decoder, random-init bf16 weights N(0, 0.02) with
 all-ones norms (seed 0), 390 synthetic audio rows N(0,1) + 12 random prompt
 ids; prefill 401 rows, forward the last row, then greedy decode.  A "step" is
 one greedy decode forward (one token); K timed steps start at the C1
@@ -419,9 +418,9 @@ def run_encoder(qa, args, wl):
         "config": {"workload": wl["desc"], "tokens": T, "weights": "synthetic N(0,0.02), seed 0"},
         "roofline": {"bound": "mfma", "achieved": round(tfs, 2), "peak": BF16_MFMA_PEAK_TFS, "unit": "TFLOP/s",
                      "frac": round(tfs / BF16_MFMA_PEAK_TFS, 4), "traffic": None,
-                     "kernel": "encoder forward (all launches; enc_gemm_hl dominant)",
+                     "kernel": "encoder forward (all launches; enc_ring products dominant)",
                      "note": "achieved counts the reference's fp32 flops; the GEMMs issue two bf16 MFMAs per "
-                             "product (fp32 activation split hi + lo, bf16 weights exact), conv1 runs on fp32 MFMA",
+                             "product (fp32 activation split hi + lo, bf16 weights exact), conv1 runs on fp32 VALU",
                      "flops_per_launch": fl, "launch_us": round(gpu_ms / K * 1e3, 2)},
         "wall_ms_per_step": round(wall / K * 1e3, 4), "cpu_baseline": cpu}), flush=True)
 

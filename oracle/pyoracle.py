@@ -431,7 +431,7 @@ class RefStream:
 
 
 # ---------------------------------------------------------------------------
-# workload inputs (BASELINE.json configs)
+# workload inputs
 # ---------------------------------------------------------------------------
 def prompt_rows(model: SynthModel, n_audio, n_ids, seed=0, audio_chunk=0, token_set=0, embed=None):
     """ids[:n_ids//2] || n_audio audio rows N(0,1) || ids[n_ids//2:], the

@@ -572,8 +572,9 @@ extern "C" int qk_enc_stem_rows_launch(const float *c3, float *rows, int chunks,
 // reads whole 128-byte lines (with half lines the load path bounded these
 // products: conv2 of 743 frames 102 -> 75 us, conv_out of 3000 41 -> 29; on
 // enc_gemm_hl they took 172 and ~45).
-// Weights of other than bf16 values, or widths that are no multiple of 128,
-// run on enc_gemm_hl / enc_gemm above.
+// Encoders with a matrix of other than bf16 values, d above 1024, an ffn that is no
+// multiple of 32 or outputs that are no whole float4s run on enc_gemm_hl / enc_gemm
+// above (qk_enc_ring_ok); ragged columns otherwise are the ring's.
 //
 // What bounds it: at 100 to 400 rows these products are a few microseconds
 // each, mostly ramp, the k walk's load path and drain; a k tile staged through
@@ -1013,7 +1014,7 @@ extern "C" int qk_enc_layernorm_launch(const float *x, const float *w, const flo
 // consecutive dims.  Online softmax per wave; the waves' (m, l, o) meet in LDS.
 // Bound by latency (104 keys a window: one round of 16 independent 16-byte
 // loads per lane, then 64 MFMAs): a window walked by one wave in blocks of 64
-// keys with 4-byte V loads took 12.6 us at 390 tokens x 14 heads, this 7.5.
+// keys with 4-byte V loads took 12.6 us at 390 tokens x 14 heads, this 6.6 (97 x 16: 4.6).
 // The result goes out as fp32 or, for the bf16 products, as halves.
 // ---------------------------------------------------------------------------
 #define EA_Q 16

@@ -23,7 +23,7 @@ def ptr(t):
     return t.data_ptr()
 
 
-# BASELINE configs[1]: the GEMV sweep (rows x cols), plus the true 1.7B 2048x2048
+# the GEMV sweep (rows x cols), plus the true 1.7B 2048x2048
 SWEEP = [(2048, 1024), (1024, 2048), (6144, 1024), (1024, 3072), (151936, 1024), (4096, 2048),
          (2048, 4096), (12288, 2048), (2048, 6144), (151936, 2048), (2048, 2048)]
 
