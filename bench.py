@@ -1,10 +1,11 @@
 #!/usr/bin/env python3
 """Benchmark of the Qwen3 decoder token loop on one MI355X.
 
-Metric: decode tok/s at batch 1 + achieved fraction of the
-HBM roofline; prefill tok/s reported alongside.  Workload (default, C1): Qwen3-ASR-0.6B decoder, random-init bf16 weights N(0, 0.02) with
-all-ones norms (seed 0), 390 synthetic audio rows N(0,1) + 12 random prompt
-ids; prefill 401 rows, forward the last row, then greedy decode.  A "step" is
+Metric: decode tok/s at batch 1 + achieved fraction of the HBM roofline;
+prefill tok/s reported alongside.  Workload (default, C1): Qwen3-ASR-0.6B
+decoder, random-init bf16 weights N(0, 0.02) with all-ones norms (seed 0),
+390 synthetic audio rows N(0,1) + 12 random prompt ids; prefill 401 rows,
+forward the last row, then greedy decode.  A "step" is
 one greedy decode forward (one token); K timed steps start at the C1
 positions (402 ..), fed back on the device (qwen_hip_decoder_generate).
 

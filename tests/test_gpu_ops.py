@@ -706,3 +706,30 @@ def test_gemm_swiglu_narrow_fewest(P, qa, gpu, M, N, K):
         qa.lib().qk_gemm_plan_epi(M, N, K, 2, C.byref(p))
     assert (p.bm, p.bn, p.nsplit > 1) == (32 if M <= 32 else 64, 64 if narrow else 128, not narrow)
     check_gemm(P, qa, gpu, M, N, K, p, 2)
+
+
+# the longest key range whose offsets the wide blocks hold in 32 bits (2^31 bytes of a
+# 256-head cache, 128 rows short), and one key more, which the 64-query blocks take
+@pytest.mark.parametrize("sk", [16255, 16256])
+def test_causal_attention_offset_limit(P, qa, gpu, sk):
+    sq, nkv, hd = 65, 256, 128
+    off = sk - sq
+    if gpu.cuda.mem_get_info()[0] < 16 << 30:
+        pytest.skip("needs 5 GB of keys and values")
+    chunk, nsplit = C.c_int(), C.c_int()
+    qa.lib().qk_attn_prefill_plan(sq, sk, off, 2 * nkv, nkv, C.byref(chunk), C.byref(nsplit))
+    assert nsplit.value == 1
+    g = gpu.Generator(device="cuda").manual_seed(sk)
+    Q, K, V = (gpu.randn(n, h * hd, generator=g, device="cuda") for n, h in ((sq, 2 * nkv), (sk, nkv), (sk, nkv)))
+    out = gpu.full((sq, 2 * nkv * hd), float("nan"), device="cuda")
+    qa.check(qa.lib().qwen_hip_causal_attention(ptr(out), ptr(Q), ptr(K), ptr(V), sq, sk, 2 * nkv, nkv, hd,
+                                                1.0 / np.sqrt(128.0), off, None), "attention")
+    gpu.cuda.synchronize()
+    mask = gpu.arange(sk, device="cuda")[None, :] > off + gpu.arange(sq, device="cuda")[:, None]
+    for h in (0, 255, 511):
+        k, v = (t[:, h // 2 * hd:(h // 2 + 1) * hd].double() for t in (K, V))
+        sc = (Q[:, h * hd:(h + 1) * hd].double() @ k.t().contiguous() / np.sqrt(128.0)).masked_fill(mask, float("-inf"))
+        ref = gpu.softmax(sc, -1) @ v
+        # the bar of the other attention tests
+        assert bool(((out[:, h * hd:(h + 1) * hd].double() - ref).abs() <= 3e-5 + 1e-4 * ref.abs()).all()), h
+    assert not bool(out.isnan().any())
