@@ -603,3 +603,18 @@ def test_encoder_general_path(P, qa, gpu, d, ffn, out, off, frames):
     assert got.shape == ref.shape and np.all(err <= ATOL + RTOL * np.abs(ref)), float(err.max())
     assert np.array_equal(e.forward(mel[:, :40]), load(qa, cfg, m).forward(mel[:, :40]))     # after a longer call
     e.close()
+
+
+# the ring path at its narrowest and widest, products narrower than a tile, k walks of
+# odd 32-deep tiles, one-frame and one-chunk inputs
+@pytest.mark.parametrize("frames", [1, 100, 431])
+@pytest.mark.parametrize("d,ffn,out", [(64, 32, 4), (192, 96, 100), (320, 1056, 36), (1024, 64, 2048)])
+def test_encoder_ring_path_widths(P, qa, gpu, d, ffn, out, frames):
+    cfg = qa.EncConfig(d, 2, d // 64, 64, ffn, out, 100, 200)
+    m, mel = P.SynthEncoder(cfg, seed=13), P.synth_mel(frames, 13, 1)
+    e = load(qa, cfg, m)
+    assert qa.lib().qk_enc_ring_ok(C.c_void_p(e.h))
+    got, ref = e.forward(mel), encoder64(gpu, m, mel).cpu().numpy()
+    err = np.abs(got - ref)
+    assert got.shape == ref.shape and np.all(err <= ATOL + RTOL * np.abs(ref)), float(err.max())
+    e.close()
